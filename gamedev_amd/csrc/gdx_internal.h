@@ -238,6 +238,8 @@ struct morton_index
     dbuf<int> idx;             // sorted record -> source index
     dbuf<float4> rec;          // sorted records {x, y, z, code}; code sign bit marks inactive
     dbuf<gdx_node> nodes;
+    dbuf<gdx_box> boxes;       // per node: the box and children the search reads
+    dbuf<gdx_box> chunks;      // per eight sorted records: the box of the active ones
     int node_count = 0;
     int leaf_count = 0;
 };

@@ -55,6 +55,16 @@ struct gdx_node
     int begin, count, first_child, child_count;
 };
 
+// axis-aligned box as the neighbour search reads it, 32 bytes. Of a node: first = its first child and
+// info = its child count, or first = its first record and info = minus its record count (a leaf)
+struct gdx_box
+{
+    float lx, ly, lz;
+    int first;
+    float hx, hy, hz;
+    int info;
+};
+
 // per raw controller bin (spatial group x size bin) sums of one bath-start rating pass
 struct gdx_raw_rate
 {

@@ -28,6 +28,7 @@ void hip_check(hipError_t e, const char *what)
 namespace {
 
 constexpr int WAVE = 64;
+constexpr int CHUNK = 8;                 // sorted records per chunk box
 
 __device__ __forceinline__ unsigned long long lanemask_lt(int lane) { return (1ull << lane) - 1ull; }
 
@@ -274,17 +275,47 @@ __global__ __launch_bounds__(256) void k_morton_keys(const float4 *pts, int n, f
     vals[i] = int(i);
 }
 
-// sorted record m carries its code 3*i + image; the activity of physical particle i marks it
+// sorted record m carries its code 3*i + image; the activity of physical particle i marks it. Every
+// CHUNK consecutive records also get the tight box of their active ones (empty, lo > hi, without any):
+// the search skips the chunks of a leaf that no query of the wavefront can use.
 __global__ __launch_bounds__(256) void k_records(const int *sidx, const float4 *pts, const unsigned char *active,
-                                                const int *codes, int n, float4 *rec)
+                                                const int *codes, int n, float4 *rec, gdx_box *chunk)
 {
-    long long m = (long long)blockIdx.x*blockDim.x + threadIdx.x;
-    if (m >= n) return;
-    int p = sidx[m];
-    float4 q = pts[p];
-    int code = codes ? codes[p] : 3*p;
-    if (active && !active[code / 3]) code |= int(0x80000000u);
-    rec[m] = make_float4(q.x, q.y, q.z, __int_as_float(code));
+    const long long m = (long long)blockIdx.x*blockDim.x + threadIdx.x;
+    float lo[3], hi[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) { lo[a] = __builtin_inff(); hi[a] = -__builtin_inff(); }
+    if (m < n)
+    {
+        int p = sidx[m];
+        float4 q = pts[p];
+        int code = codes ? codes[p] : 3*p;
+        if (active && !active[code / 3])
+        {
+            // no coordinates: no distance to it passes a test
+            rec[m] = make_float4(__builtin_nanf(""), __builtin_nanf(""), __builtin_nanf(""),
+                                 __int_as_float(code | int(0x80000000u)));
+        }
+        else
+        {
+            rec[m] = make_float4(q.x, q.y, q.z, __int_as_float(code));
+            lo[0] = hi[0] = q.x;
+            lo[1] = hi[1] = q.y;
+            lo[2] = hi[2] = q.z;
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+    {
+#pragma unroll
+        for (int o = 1; o < CHUNK; o <<= 1)
+        {
+            lo[a] = fminf(lo[a], __shfl_xor(lo[a], o, WAVE));
+            hi[a] = fmaxf(hi[a], __shfl_xor(hi[a], o, WAVE));
+        }
+    }
+    if (m < n && threadIdx.x % CHUNK == 0)
+        chunk[m / CHUNK] = gdx_box{lo[0], lo[1], lo[2], 0, hi[0], hi[1], hi[2], 0};
 }
 
 // ============================================================================================
@@ -422,26 +453,73 @@ __global__ __launch_bounds__(256) void k_node_expand(gdx_node *nodes, const uint
 
 // ============================================================================================
 // exact top-K: one lane per query, 64 Morton-consecutive queries per wavefront share one
-// traversal; leaf records are loaded as 64-record tiles and broadcast lane by lane
+// traversal of the hierarchy's boxes
 // ============================================================================================
 constexpr int TOPK_BLOCK = 256;
-constexpr int TOPK_STACK = 256;
+// a popped node of level l pushes at most its eight children: 20 levels hold at most 20*7 + 1 entries
+constexpr int TOPK_STACK = 160;
 
 __device__ __forceinline__ bool nb_less(float da, int ia, float db, int ib)   // morton_types.cuh:68-72
 { return da < db || (da == db && ia < ib); }
 
-// padded point-to-cell lower distance (morton_index.cuh:296-314)
-__device__ __forceinline__ float node_d2(float qx, float qy, float qz, const gdx_node &nd, int dim, int max_level)
+// box of a hierarchy node as the search reads it: its cube padded against the rounding of the keys
+// (morton_index.cuh:296-314), open in z for a two-dimensional index, and where its children or its records
+// are. Formed once per build: the pad alone is some fifteen instructions, and a node is tested by several
+// wavefronts.
+__global__ __launch_bounds__(256) void k_node_boxes(const gdx_node *nodes, int count, int dim, int max_level,
+                                                   gdx_box *box)
 {
-    float ux = nd.lx + nd.width, uy = nd.ly + nd.width, uz = nd.lz + nd.width;
-    float scale = fmaxf(1.0f, fmaxf(fmaxf(fabsf(nd.lx), fabsf(ux)),
+    const int i = blockIdx.x*blockDim.x + threadIdx.x;
+    if (i >= count) return;
+    const gdx_node nd = nodes[i];
+    const float ux = nd.lx + nd.width, uy = nd.ly + nd.width, uz = nd.lz + nd.width;
+    const float scale = fmaxf(1.0f, fmaxf(fmaxf(fabsf(nd.lx), fabsf(ux)),
         fmaxf(fmaxf(fabsf(nd.ly), fabsf(uy)), fmaxf(fabsf(nd.lz), fabsf(uz)))));
-    float pad = 2.0f*static_cast<float>(max_level + 2)*FLT_EPSILON*scale;
-    float dx = fmaxf(fmaxf(nd.lx - qx - pad, 0.0f), qx - ux - pad);
-    float dy = fmaxf(fmaxf(nd.ly - qy - pad, 0.0f), qy - uy - pad);
-    float dz = (dim == 2) ? 0.0f : fmaxf(fmaxf(nd.lz - qz - pad, 0.0f), qz - uz - pad);
-    return dx*dx + dy*dy + dz*dz;
+    const float pad = 2.0f*static_cast<float>(max_level + 2)*FLT_EPSILON*scale;
+    const int nch = nd.child_count & 15;
+    gdx_box b{nd.lx - pad, nd.ly - pad, nd.lz - pad, nch ? nd.first_child : nd.begin,
+              ux + pad, uy + pad, uz + pad, nch ? nch : -nd.count};
+    if (dim == 2) { b.lz = -__builtin_inff(); b.hz = __builtin_inff(); }
+    box[i] = b;
 }
+
+// two boxes, or four records, by one scalar load at a uniform address (field by field the compiler moves
+// each to its use and waits there again)
+typedef float f32x16 __attribute__((ext_vector_type(16), aligned(16)));
+// boxes read together; the box arrays hold as many more than they have boxes
+constexpr int BOX_GROUP = 4;
+
+// squared distance of a point to a box, rounded differently from the records' distances: reach() widens
+// the limit it is compared with, so that no record within the limit lies in a rejected box
+__device__ __forceinline__ float box_d2(float qx, float qy, float qz, float lx, float ly, float lz, float hx, float hy,
+                                        float hz)
+{
+    const float dx = fmaxf(fmaxf(lx - qx, qx - hx), 0.0f);
+    const float dy = fmaxf(fmaxf(ly - qy, qy - hy), 0.0f);
+    const float dz = fmaxf(fmaxf(lz - qz, qz - hz), 0.0f);
+    return fmaf(dz, dz, fmaf(dy, dy, dx*dx));
+}
+
+// the first `count` of the boxes [p, p + BOX_GROUP) that some lane's point reaches within its limit, as a mask
+__device__ __forceinline__ unsigned boxes_reached(const gdx_box *p, int count, float qx, float qy, float qz, float lim)
+{
+    const f32x16 *g = reinterpret_cast<const f32x16 *>(p);
+    const f32x16 v[BOX_GROUP / 2] = {g[0], g[1]};
+    unsigned mask = 0u;
+#pragma unroll
+    for (int u = 0; u < BOX_GROUP; ++u)
+    {
+        const f32x16 &w = v[u / 2];
+        const int o = 8*(u % 2);
+        const float d2 = box_d2(qx, qy, qz, w[o], w[o + 1], w[o + 2], w[o + 4], w[o + 5], w[o + 6]);
+        if (__ballot(d2 <= lim)) mask |= 1u << u;
+    }
+    return __builtin_amdgcn_readfirstlane(mask & ((2u << min(count - 1, BOX_GROUP - 1)) - 1u));
+}
+
+// |rounding| of both sums is below 3 ulp of the larger, or 2^-148 where they are subnormal; a negative
+// limit (a lane without a query) stays negative
+__device__ __forceinline__ float reach(float lim) { return lim < 0.0f ? lim : fmaf(lim, 1.000001f, 1.0e-37f); }
 
 // insert (nd, nc) into the ascending list; precondition: it precedes the current last entry
 template <int K>
@@ -501,78 +579,80 @@ __device__ __forceinline__ float readlane_f(float v, int l)
 { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
 
 // Traversal shared by both selection schemes: the wavefront pops nodes from one LDS stack, children
-// nearest-first from the wavefront's centre, and pushes only the nodes some lane needs; every needed leaf
-// goes to leaf(begin, end, need) with need the lane's own test. cut() is the lane's current pruning
-// distance (the smaller of its cap and its K-th candidate so far).
+// nearest-first from the wavefront's centre, and pushes only the nodes some lane needs; every popped leaf
+// goes to leaf(begin, end). cut() is the lane's current pruning distance (the smaller of its cap and its
+// K-th candidate so far, negative for a lane without a query). A stack entry holds the node's children or
+// records itself, so that a pop reads no node: testing a popped node again would spare one pop in twenty.
+// The children's boxes come through scalar loads, and once more as one box per lane for their distances
+// from the centre.
 template <class Cut, class Leaf>
-__device__ __forceinline__ void traverse(const gdx_node *nodes, int dim, int max_level, float qx, float qy, float qz,
-                                         bool qactive, float cx, float cy, float cz, int *stack,
-                                         unsigned int *overflow, Cut cut_of, Leaf leaf)
+__device__ __forceinline__ void traverse(const gdx_box *__restrict__ boxes, float qx, float qy, float qz, bool qactive,
+                                         float cx, float cy, float cz, int2 *stack, unsigned int *overflow, Cut cut_of,
+                                         Leaf leaf)
 {
     const int lane = threadIdx.x % WAVE;
     if (__ballot(qactive) == 0ull) return;
-    int sp = 1;
-    if (lane == 0) stack[0] = 0;
-    __builtin_amdgcn_wave_barrier();
-    while (sp > 0)
+    int sp = 0;
+    int first = boxes[0].first, info = boxes[0].info;
+    while (true)
     {
+        if (info < 0)
+        {
+            leaf(first, first - info);
+        }
+        else
+        {
+            // children some lane needs, each child's distance from the wavefront's centre kept by the lane of
+            // its index; the needed children go on the stack farthest first (nearest on top, equal distances
+            // in child order), each lane writing its own child at its rank
+            const int nch = info;
+            const gdx_box mine = boxes[first + min(lane, nch - 1)];
+            const float lim = reach(cut_of());
+            unsigned needed = boxes_reached(boxes + first, nch, qx, qy, qz, lim);
+            if (nch > BOX_GROUP)
+                needed |= boxes_reached(boxes + first + BOX_GROUP, nch - BOX_GROUP, qx, qy, qz, lim) << BOX_GROUP;
+            int nv = __popc(needed);
+            if (sp + nv > TOPK_STACK)
+            {
+                if (lane == 0) atomicOr(overflow, 1u);
+                nv = 0;
+            }
+            const float kd = box_d2(cx, cy, cz, mine.lx, mine.ly, mine.lz, mine.hx, mine.hy, mine.hz);
+            int rank = 0;
+            for (unsigned rest = needed; rest; rest &= rest - 1u)
+            {
+                const int m = __builtin_ctz(rest);
+                const float km = readlane_f(kd, m);
+                rank += km < kd || (km == kd && m < lane);
+            }
+            if (nv > 0 && lane < nch && ((needed >> lane) & 1u))
+                stack[sp + nv - 1 - rank] = make_int2(mine.first, mine.info);
+            sp += nv;
+            __builtin_amdgcn_wave_barrier();
+        }
+        sp = __builtin_amdgcn_readfirstlane(sp);
+        if (sp == 0) break;
         --sp;
-        int id = __builtin_amdgcn_readfirstlane(stack[sp]);
-        gdx_node nd = nodes[id];
-        float cut = cut_of();
-        bool need = qactive && node_d2(qx, qy, qz, nd, dim, max_level) <= cut;
-        if (__ballot(need) == 0ull) continue;
-        if (nd.child_count == 0)
-        {
-            leaf(nd.begin, nd.begin + nd.count, need);
-            continue;
-        }
-        // children some lane needs, each child's distance from the wavefront's centre kept by the lane of
-        // its index; the needed children go on the stack farthest first (nearest on top, equal distances
-        // in child order), each lane writing its own child at its rank
-        const int nch = nd.child_count & 15;
-        unsigned needed = 0u;
-        float kd = __builtin_inff();
-        for (int ch = 0; ch < nch; ++ch)
-        {
-            gdx_node cn = nodes[nd.first_child + ch];
-            bool cneed = qactive && node_d2(qx, qy, qz, cn, dim, max_level) <= cut;
-            if (__ballot(cneed) == 0ull) continue;
-            needed |= 1u << ch;
-            const float k = node_d2(cx, cy, cz, cn, dim, max_level);
-            if (lane == ch) kd = k;
-        }
-        int nv = __popc(needed);
-        if (sp + nv > TOPK_STACK)
-        {
-            if (lane == 0) atomicOr(overflow, 1u);
-            nv = 0;
-        }
-        // ranks by whole-wavefront shuffles (every lane active), then each needed child's lane writes it
-        int rank = 0;
-        for (int m = 0; m < nch; ++m)
-        {
-            const float km = __shfl(kd, m, WAVE);
-            rank += ((needed >> m) & 1u) && (km < kd || (km == kd && m < lane));
-        }
-        if (nv > 0 && lane < nch && ((needed >> lane) & 1u)) stack[sp + nv - 1 - rank] = nd.first_child + lane;
-        sp += nv;
+        const int2 e = stack[sp];
+        first = __builtin_amdgcn_readfirstlane(e.x);
+        info = __builtin_amdgcn_readfirstlane(e.y);
         __builtin_amdgcn_wave_barrier();
     }
 }
 
 // insertion scheme: every eligible record goes through the lane's sorted K-entry register list
 template <int K, bool DEDUP = false>
-__device__ void topk_wave(const float4 *rec, const gdx_node *nodes, int dim, int max_level, float qx, float qy,
-                          float qz, float q2, bool qactive, float cx, float cy, float cz, float (&d)[K], int (&c)[K],
-                          int *stack, unsigned int *overflow)
+__device__ void topk_wave(const float4 *rec, const gdx_box *__restrict__ boxes, float qx, float qy, float qz, float q2,
+                          bool qactive, float cx, float cy, float cz, float (&d)[K], int (&c)[K], int2 *stack,
+                          unsigned int *overflow)
 {
     const int lane = threadIdx.x % WAVE;
+    const float cap = qactive ? q2 : -1.0f;
 #pragma unroll
     for (int k = 0; k < K; ++k) { d[k] = __builtin_inff(); c[k] = INT_MAX; }
-    traverse(nodes, dim, max_level, qx, qy, qz, qactive, cx, cy, cz, stack, overflow,
-             [&] { return fminf(q2, d[K - 1]); },
-             [&](int begin, int end, bool need) {
+    traverse(boxes, qx, qy, qz, qactive, cx, cy, cz, stack, overflow,
+             [&] { return fminf(cap, d[K - 1]); },
+             [&](int begin, int end) {
                  for (int t0 = begin; t0 < end; t0 += WAVE)
                  {
                      int idx = t0 + lane;
@@ -584,7 +664,7 @@ __device__ void topk_wave(const float4 *rec, const gdx_node *nodes, int dim, int
                          int code = __builtin_amdgcn_readlane(__float_as_int(v.w), j);
                          float dx = qx - px, dy = qy - py, dz = qz - pz;
                          float d2 = dx*dx + dy*dy + dz*dz;
-                         bool e = need && code >= 0 && d2 <= q2 && nb_less(d2, code, d[K - 1], c[K - 1]);
+                         bool e = code >= 0 && d2 <= cap && nb_less(d2, code, d[K - 1], c[K - 1]);
                          if (e)
                          {
                              if constexpr (DEDUP) topk_insert_dedup<K>(d, c, d2, code);
@@ -596,16 +676,21 @@ __device__ void topk_wave(const float4 *rec, const gdx_node *nodes, int dim, int
 }
 
 // ---- tiled scheme: candidates collected per lane in LDS, merged B at a time (gdx_topk.h) ----
-// the lane's `cnt` buffered keys buf[r * WAVE] merged into L
+// the lane's `cnt` buffered keys buf[r * WAVE] merged into L. A slot past the count becomes a key above
+// TOPK_EMPTY by its upper word alone: no list entry is larger, so it never enters one.
+constexpr uint32_t TOPK_NO_KEY = 0x7fe00000u;
+constexpr unsigned TILE_ROW = WAVE*sizeof(uint64_t);      // bytes of one key per lane
+
 template <int K, int B>
-__device__ __forceinline__ void topk_flush(uint64_t (&L)[K], const uint64_t *buf, int cnt)
+__device__ __forceinline__ void topk_flush(uint64_t (&L)[K], const char *col, int cnt)
 {
     uint64_t S[B];
 #pragma unroll
     for (int r = 0; r < B; ++r)
     {
-        const uint64_t v = buf[r*WAVE];
-        S[r] = r < cnt ? v : TOPK_EMPTY;
+        const uint64_t v = *reinterpret_cast<const uint64_t *>(col + r*TILE_ROW);
+        const uint32_t hi = r < cnt ? uint32_t(v >> 32) : TOPK_NO_KEY;
+        S[r] = (uint64_t(hi) << 32) | uint32_t(v);
     }
     bitonic_sort<B>(S);
     topk_merge_sorted<K, B>(L, S);
@@ -618,54 +703,78 @@ __device__ __forceinline__ void topk_flush(uint64_t (&L)[K], const uint64_t *buf
 // not depend on the order of merging, so the result is the insertion scheme's, bit for bit.
 // records per overflow check of the tiled scheme: a merge runs before a group when some lane could not
 // take all of it
-constexpr int TILE_GROUP = 4;
+constexpr int TILE_GROUP = 4;             // one f32x16
 
 template <int K, int B>
-__device__ void topk_wave_tiled(const float4 *__restrict__ rec, const gdx_node *__restrict__ nodes, int dim, int max_level, float qx, float qy,
-                                float qz, float q2, bool qactive, float cx, float cy, float cz, float (&d)[K],
-                                int (&c)[K], int *stack, uint64_t *buf, unsigned int *overflow)
+__device__ void topk_wave_tiled(const float4 *__restrict__ rec, const gdx_box *__restrict__ boxes,
+                                const gdx_box *__restrict__ chunks, float qx, float qy, float qz, float q2,
+                                bool qactive, float cx, float cy, float cz, float (&d)[K], int (&c)[K], int2 *stack,
+                                uint64_t *buf, unsigned int *overflow)
 {
     const int lane = threadIdx.x % WAVE;
+    const float cap = qactive ? q2 : -1.0f;
     uint64_t L[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) L[k] = TOPK_EMPTY;
-    uint64_t *col = buf + lane;
-    int cnt = 0;
-    traverse(nodes, dim, max_level, qx, qy, qz, qactive, cx, cy, cz, stack, overflow,
-             [&] { return fminf(q2, __uint_as_float(uint32_t(L[K - 1] >> 32))); },
-             [&](int begin, int end, bool need) {
-                 // records at uniform addresses (scalar loads, four at a time); the filter is the lane's
-                 // cap and the distance of its K-th key as of its last merge (lanes that do not need the
-                 // leaf take nothing: d^2 >= 0 > -1); ties at that distance pass and the merge decides them
-                 const float cap = need ? q2 : -1.0f;
-                 float lim = fminf(cap, __uint_as_float(uint32_t(L[K - 1] >> 32)));
-                 for (int t = begin; t < end; t += TILE_GROUP)
+    char *tile = reinterpret_cast<char *>(buf);
+    const unsigned col = lane*unsigned(sizeof(uint64_t));
+    unsigned put = col;                       // byte offset of the lane's next free slot
+    // the lane's cap and the distance of its K-th key as of its last merge; ties at that distance pass and
+    // the merge decides them
+    float lim = fminf(cap, __uint_as_float(uint32_t(L[K - 1] >> 32)));
+    float far = reach(lim);
+    auto merge = [&] {
+        topk_flush<K, B>(L, tile + col, int((put - col)/TILE_ROW));
+        put = col;
+        lim = fminf(cap, __uint_as_float(uint32_t(L[K - 1] >> 32)));
+        far = reach(lim);
+    };
+    // inactive records hold no coordinates (k_records): their distance is NaN and passes nothing
+    auto test = [&](float x, float y, float z, float code) {
+        const float dx = qx - x, dy = qy - y, dz = qz - z;
+        const float d2 = dx*dx + dy*dy + dz*dz;
+        if (d2 <= lim)
+        {
+            *reinterpret_cast<uint64_t *>(tile + put) = (uint64_t(__float_as_uint(d2)) << 32)
+                | __float_as_uint(code);
+            put += TILE_ROW;
+        }
+    };
+    traverse(boxes, qx, qy, qz, qactive, cx, cy, cz, stack, overflow, [&] { return lim; },
+             [&](int begin, int end) {
+                 const int last = (end - 1) / CHUNK;
+                 for (int c0 = begin / CHUNK; c0 <= last; c0 += BOX_GROUP)
                  {
-                     if (__ballot(cnt > B - TILE_GROUP))
+                     unsigned needed = boxes_reached(chunks + c0, last - c0 + 1, qx, qy, qz, far);
+                     for (; needed; needed &= needed - 1u)
                      {
-                         topk_flush<K, B>(L, col, cnt);
-                         cnt = 0;
-                         lim = fminf(cap, __uint_as_float(uint32_t(L[K - 1] >> 32)));
-                     }
-                     // the group's loads first (indices clamped into the leaf), then its tests
-                     float4 v[TILE_GROUP];
-#pragma unroll
-                     for (int u = 0; u < TILE_GROUP; ++u) v[u] = rec[min(t + u, end - 1)];
-#pragma unroll
-                     for (int u = 0; u < TILE_GROUP; ++u)
-                     {
-                         const int code = __float_as_int(v[u].w);
-                         const float dx = qx - v[u].x, dy = qy - v[u].y, dz = qz - v[u].z;
-                         const float d2 = dx*dx + dy*dy + dz*dz;
-                         if (t + u < end && code >= 0 && d2 <= lim)
+                         // the chunk's records inside the leaf, at uniform addresses (scalar loads), four
+                         // together where the leaf holds them
+                         const int at = (c0 + __builtin_ctz(needed))*CHUNK;
+                         const int t1 = min(end, at + CHUNK);
+                         for (int t = max(begin, at); t < t1; t += TILE_GROUP)
                          {
-                             col[cnt*WAVE] = (uint64_t(__float_as_uint(d2)) << 32) | uint32_t(code);
-                             ++cnt;
+                             if (__ballot(put > col + (B - TILE_GROUP)*TILE_ROW)) merge();
+                             if (t + TILE_GROUP <= t1)
+                             {
+                                 const f32x16 v = *reinterpret_cast<const f32x16 *>(rec + t);
+#pragma unroll
+                                 for (int u = 0; u < TILE_GROUP; ++u)
+                                     test(v[4*u], v[4*u + 1], v[4*u + 2], v[4*u + 3]);
+                             }
+                             else
+                             {
+                                 for (int r = t; r < t1; ++r)
+                                 {
+                                     const float4 v = rec[r];
+                                     test(v.x, v.y, v.z, v.w);
+                                 }
+                             }
                          }
                      }
                  }
              });
-    if (__ballot(cnt > 0)) topk_flush<K, B>(L, col, cnt);
+    if (__ballot(put > col)) merge();
 #pragma unroll
     for (int k = 0; k < K; ++k)
     {
@@ -700,8 +809,9 @@ __device__ __forceinline__ void wave_centre(float qx, float qy, float qz, bool q
 // stack and tile, so the shape changes only how the wavefronts are packed onto the CUs)
 template <bool DEDUP, int TILE, int WPB>
 __global__ __launch_bounds__(WPB*WAVE) void k_col_topk(const float4 *__restrict__ rec,
-                                                        const gdx_node *__restrict__ nodes, int n, int dim,
-                                                        int max_level, const int *__restrict__ sidx,
+                                                        const gdx_box *__restrict__ boxes,
+                                                        const gdx_box *__restrict__ chunks, int n,
+                                                        const int *__restrict__ sidx,
                                                         const float4 *__restrict__ pts,
                                                         const int *__restrict__ pidx_slot,
                                                         const unsigned char *__restrict__ group,
@@ -713,7 +823,7 @@ __global__ __launch_bounds__(WPB*WAVE) void k_col_topk(const float4 *__restrict_
 {
     static_assert(!(DEDUP && TILE), "image dedup runs on the insertion scheme");
     static_assert(TILE == 0 || TILE >= TILE_GROUP, "a merge tile holds at least one record group");
-    __shared__ int stacks[WPB][TOPK_STACK];
+    __shared__ int2 stacks[WPB][TOPK_STACK];
     __shared__ uint64_t tiles[WPB][TILE > 0 ? TILE : 1][WAVE];
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     long long m = ((long long)xcd_block()*WPB + wave)*WAVE + lane;
@@ -729,11 +839,10 @@ __global__ __launch_bounds__(WPB*WAVE) void k_col_topk(const float4 *__restrict_
     float d[N_K];
     int c[N_K];
     if constexpr (TILE > 0)
-        topk_wave_tiled<N_K, TILE>(rec, nodes, dim, max_level, me.x, me.y, me.z, q2, qactive, cx, cy, cz, d, c,
-                                   stacks[wave], &tiles[wave][0][0], overflow);
+        topk_wave_tiled<N_K, TILE>(rec, boxes, chunks, me.x, me.y, me.z, q2, qactive, cx, cy, cz, d, c, stacks[wave],
+                                   &tiles[wave][0][0], overflow);
     else
-        topk_wave<N_K, DEDUP>(rec, nodes, dim, max_level, me.x, me.y, me.z, q2, qactive, cx, cy, cz, d, c,
-                              stacks[wave], overflow);
+        topk_wave<N_K, DEDUP>(rec, boxes, me.x, me.y, me.z, q2, qactive, cx, cy, cz, d, c, stacks[wave], overflow);
     unsigned long long mask = 0ull;
     int g = qactive ? int(group[p]) : -1;
     if (qactive)
@@ -789,11 +898,10 @@ __global__ __launch_bounds__(WPB*WAVE) void k_col_topk(const float4 *__restrict_
 
 // runtime-K exact top-K for arbitrary query points (test access to the search contract)
 template <int K>
-__global__ __launch_bounds__(TOPK_BLOCK) void k_knn(const float4 *rec, const gdx_node *nodes, int dim, int max_level,
-                                                   const float4 *queries, int nq, int *codes, float *dist,
+__global__ __launch_bounds__(TOPK_BLOCK) void k_knn(const float4 *rec, const gdx_box *boxes, const float4 *queries, int nq, int *codes, float *dist,
                                                    unsigned int *overflow)
 {
-    __shared__ int stacks[TOPK_BLOCK / WAVE][TOPK_STACK];
+    __shared__ int2 stacks[TOPK_BLOCK / WAVE][TOPK_STACK];
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     long long m = ((long long)blockIdx.x*(TOPK_BLOCK / WAVE) + wave)*WAVE + lane;
     bool valid = m < nq;
@@ -803,7 +911,7 @@ __global__ __launch_bounds__(TOPK_BLOCK) void k_knn(const float4 *rec, const gdx
     wave_centre(qp.x, qp.y, qp.z, valid, cx, cy, cz);
     float d[K];
     int c[K];
-    topk_wave<K>(rec, nodes, dim, max_level, qp.x, qp.y, qp.z, q2, valid, cx, cy, cz, d, c, stacks[wave], overflow);
+    topk_wave<K>(rec, boxes, qp.x, qp.y, qp.z, q2, valid, cx, cy, cz, d, c, stacks[wave], overflow);
     if (!valid) return;
 #pragma unroll
     for (int k = 0; k < K; ++k)
@@ -980,10 +1088,12 @@ void morton_build(morton_index &ix, const float4 *points, const unsigned char *a
     ix.keys.alloc(size_t(n));
     ix.idx.alloc(size_t(n));
     ix.rec.alloc(size_t(n));
+    ix.chunks.alloc(size_t(blocks_for(n, CHUNK) + BOX_GROUP));
     k_morton_keys<<<blocks_for(n, 256), 256, 0, st>>>(points, n, ox, oy, oz, width, max_level, dim, ix.keys.p, ix.idx.p);
     hip_check(hipGetLastError(), "launch morton keys");
     radix_sort_pairs(ix.keys.p, ix.idx.p, n, 0, 3*max_level, s, st);
-    k_records<<<blocks_for(n, 256), 256, 0, st>>>(ix.idx.p, points, active, codes, n, ix.rec.p);
+    k_records<<<blocks_for(n, 256), 256, 0, st>>>(ix.idx.p, points, active, codes, n, ix.rec.p,
+                                                     ix.chunks.p);
     hip_check(hipGetLastError(), "launch morton records");
 
     size_t cap = std::max<size_t>(1024, size_t(n) / size_t(std::max(1, leaf_target))*4 + 64);
@@ -1013,6 +1123,9 @@ void morton_build(morton_index &ix, const float4 *points, const unsigned char *a
         count = int(next);
     }
     ix.node_count = node_count;
+    ix.boxes.alloc(ix.nodes.n + BOX_GROUP);
+    k_node_boxes<<<blocks_for(node_count, 256), 256, 0, st>>>(ix.nodes.p, node_count, dim, max_level, ix.boxes.p);
+    hip_check(hipGetLastError(), "launch node boxes");
     hip_check(hipStreamSynchronize(st), "complete Morton hierarchy");
 }
 
@@ -1023,13 +1136,13 @@ void knn_query(const morton_index &ix, const float4 *queries, int nq, int k, int
     int nb = blocks_for(nq, TOPK_BLOCK);
     switch (k)
     {
-    case 1: k_knn<1><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.nodes.p, ix.dim, ix.max_level, queries, nq, codes, d2, overflow); break;
-    case 2: k_knn<2><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.nodes.p, ix.dim, ix.max_level, queries, nq, codes, d2, overflow); break;
-    case 4: k_knn<4><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.nodes.p, ix.dim, ix.max_level, queries, nq, codes, d2, overflow); break;
-    case 8: k_knn<8><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.nodes.p, ix.dim, ix.max_level, queries, nq, codes, d2, overflow); break;
-    case 16: k_knn<16><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.nodes.p, ix.dim, ix.max_level, queries, nq, codes, d2, overflow); break;
-    case 32: k_knn<32><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.nodes.p, ix.dim, ix.max_level, queries, nq, codes, d2, overflow); break;
-    case 64: k_knn<64><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.nodes.p, ix.dim, ix.max_level, queries, nq, codes, d2, overflow); break;
+    case 1: k_knn<1><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.boxes.p, queries, nq, codes, d2, overflow); break;
+    case 2: k_knn<2><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.boxes.p, queries, nq, codes, d2, overflow); break;
+    case 4: k_knn<4><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.boxes.p, queries, nq, codes, d2, overflow); break;
+    case 8: k_knn<8><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.boxes.p, queries, nq, codes, d2, overflow); break;
+    case 16: k_knn<16><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.boxes.p, queries, nq, codes, d2, overflow); break;
+    case 32: k_knn<32><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.boxes.p, queries, nq, codes, d2, overflow); break;
+    case 64: k_knn<64><<<nb, TOPK_BLOCK, 0, st>>>(ix.rec.p, ix.boxes.p, queries, nq, codes, d2, overflow); break;
     default: throw status_error(15, "knn query K must be 1, 2, 4, 8, 16, 32 or 64");
     }
     hip_check(hipGetLastError(), "launch knn");
@@ -1175,7 +1288,7 @@ void geometry_epoch(context &c)
         if (X_WEDGE) c.nbr_image.alloc(na*N_K);
 #define GDX_TOPK_SHAPED(DEDUP, TILE, WPB)                                                                    \
     k_col_topk<DEDUP, TILE, WPB><<<xcd_grid(blocks_for(waves, WPB)), WPB*WAVE, 0, st>>>(                     \
-        c.index.rec.p, c.index.nodes.p, nr, DIM, MORTON_MAX_LEVEL, c.index.idx.p, c.pts.p, c.pidx_slot.p,     \
+        c.index.rec.p, c.index.boxes.p, c.index.chunks.p, nr, c.index.idx.p, c.pts.p, c.pidx_slot.p,         \
         c.group.p, c.user, c.nbr.p, c.measure.p, c.graph.p, c.overflow.p, c.nbr_image.p)
 #define GDX_TOPK_LAUNCH(DEDUP, TILE)                                                                         \
     do                                                                                                        \

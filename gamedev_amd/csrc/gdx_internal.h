@@ -278,6 +278,7 @@ struct context
     dbuf<int> wedge_code;
     dbuf<unsigned int> ghost_count, ghost_off;
     dbuf<unsigned char> nbr_image;  // n_active x N_K image of each neighbour (slot order)
+    dbuf<unsigned long long> again; // per top-K wavefront: the queries left to the pass with image removal
     int n_records = 0;              // indexed records: n, plus ghosts in a wedge
     float q_max = 0.0f;             // largest search cap of the epoch (wedge seam test)
     bool unique_ids = true;         // images of one particle can never share a search ball

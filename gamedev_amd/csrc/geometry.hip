@@ -819,7 +819,8 @@ __global__ __launch_bounds__(WPB*WAVE) void k_col_topk(const float4 *__restrict_
                                                         double *__restrict__ measure,
                                                         unsigned long long *__restrict__ graph,
                                                         unsigned int *__restrict__ overflow,
-                                                        unsigned char *__restrict__ nbr_image)
+                                                        unsigned char *__restrict__ nbr_image,
+                                                        unsigned long long *__restrict__ again, float image_d2)
 {
     static_assert(!(DEDUP && TILE), "image dedup runs on the insertion scheme");
     static_assert(TILE == 0 || TILE >= TILE_GROUP, "a merge tile holds at least one record group");
@@ -831,6 +832,12 @@ __global__ __launch_bounds__(WPB*WAVE) void k_col_topk(const float4 *__restrict_
     float4 me = valid ? rec[m] : make_float4(0.f, 0.f, 0.f, __int_as_float(-1));
     int code = __float_as_int(me.w);
     bool qactive = valid && code >= 0 && (!X_WEDGE || code % 3 == 0);
+    if constexpr (DEDUP)
+    {
+        // after a tiled pass: only the queries it left
+        if (again) qactive = qactive && ((again[m / WAVE] >> lane) & 1ull);
+        if (__ballot(qactive) == 0ull) return;
+    }
     int p = valid ? sidx[m] : 0;
     float q = qactive ? pts[p].w : 0.0f;
     float q2 = q*q;
@@ -844,9 +851,8 @@ __global__ __launch_bounds__(WPB*WAVE) void k_col_topk(const float4 *__restrict_
     else
         topk_wave<N_K, DEDUP>(rec, boxes, me.x, me.y, me.z, q2, qactive, cx, cy, cz, d, c, stacks[wave], overflow);
     unsigned long long mask = 0ull;
-    int g = qactive ? int(group[p]) : -1;
-    if (qactive)
-    {
+    const int g = qactive ? int(group[p]) : -1;
+    auto write = [&]() {
         int s = pidx_slot[p];
         float max_d2 = 0.0f;
         int row[N_K];
@@ -881,7 +887,29 @@ __global__ __launch_bounds__(WPB*WAVE) void k_col_topk(const float4 *__restrict_
         }
         double radius = sqrt(static_cast<double>(max_d2));
         measure[s] = ball_measure(ld(u.y, p), ld(u.z, p), radius);
+    };
+    if constexpr (X_WEDGE && !DEDUP)
+    {
+        // Two images of one particle both in a list lie within twice the list's radius of each other. A list
+        // whose diameter is below the least distance of two images of any particle therefore holds every
+        // particle once and is what the search with removal would give; the caps that make the removal
+        // necessary are mostly far larger than the lists. The other queries (a list that is not full reaches
+        // to the cap) are left to a second pass with removal, as a mask per wavefront. Wedge of 1e6
+        // representatives, K = 32: 18.2 ms with removal for every query, 1.4 ms so.
+        if (again)
+        {
+            const float far2 = c[N_K - 1] != INT_MAX ? d[N_K - 1] : q2;
+            const bool left = qactive && !(4.001f*far2 < image_d2);
+            const unsigned long long mine = __ballot(left);
+            if (lane == 0 && valid) again[m / WAVE] = mine;
+            qactive = qactive && !left;
+        }
     }
+    else
+    {
+        (void)image_d2;
+    }
+    if (qactive) write();
     // one atomic per distinct owner group of this wavefront (col_dep_graph.cu:14-60)
     unsigned long long todo = __ballot(qactive);
     while (todo)
@@ -1148,6 +1176,15 @@ void knn_query(const morton_index &ix, const float4 *queries, int nq, int k, int
     hip_check(hipGetLastError(), "launch knn");
 }
 
+// the least distance any two images of one particle can have: rotated by the wedge's width from each
+// other, or, the two ghosts, by twice that
+static float image_distance()
+{
+    const double width = static_cast<double>(X_MAX) - static_cast<double>(X_MIN);
+    const double turn = std::fmin(std::fabs(std::sin(0.5*width)), std::fabs(std::sin(width)));
+    return static_cast<float>(2.0*Y_MIN*std::fmin(std::sin(Z_MIN), std::sin(Z_MAX))*turn);
+}
+
 // the largest search cap and the unique-identifier test of swarm_runtime.cu:331-340, 413-415
 static void wedge_cap(context &c)
 {
@@ -1286,10 +1323,11 @@ void geometry_epoch(context &c)
     {
         int waves = blocks_for(nr, WAVE);
         if (X_WEDGE) c.nbr_image.alloc(na*N_K);
+        const float image_d2 = X_WEDGE ? image_distance()*image_distance() : 0.0f;
 #define GDX_TOPK_SHAPED(DEDUP, TILE, WPB)                                                                    \
     k_col_topk<DEDUP, TILE, WPB><<<xcd_grid(blocks_for(waves, WPB)), WPB*WAVE, 0, st>>>(                     \
         c.index.rec.p, c.index.boxes.p, c.index.chunks.p, nr, c.index.idx.p, c.pts.p, c.pidx_slot.p,         \
-        c.group.p, c.user, c.nbr.p, c.measure.p, c.graph.p, c.overflow.p, c.nbr_image.p)
+        c.group.p, c.user, c.nbr.p, c.measure.p, c.graph.p, c.overflow.p, c.nbr_image.p, again, image_d2)
 #define GDX_TOPK_LAUNCH(DEDUP, TILE)                                                                         \
     do                                                                                                        \
     {                                                                                                         \
@@ -1297,16 +1335,21 @@ void geometry_epoch(context &c)
         else if (c.topk_waves == 2) GDX_TOPK_SHAPED(DEDUP, TILE, 2);                                          \
         else GDX_TOPK_SHAPED(DEDUP, TILE, 4);                                                                 \
     } while (0)
-        if (!c.unique_ids && X_WEDGE)
-            GDX_TOPK_LAUNCH(bool(X_WEDGE), 0);
-        else if (c.topk_tile == 8)
-            GDX_TOPK_LAUNCH(false, 8);
-        else if (c.topk_tile == 16)
-            GDX_TOPK_LAUNCH(false, 16);
-        else if (c.topk_tile == 32)
-            GDX_TOPK_LAUNCH(false, 32);
-        else
-            GDX_TOPK_LAUNCH(false, 0);
+        unsigned long long *again = nullptr;
+        const bool removal = X_WEDGE && !c.unique_ids;
+        if (removal && c.topk_tile)
+        {
+            c.again.alloc(size_t(waves));
+            again = c.again.p;
+        }
+        if (!removal || c.topk_tile)
+        {
+            if (c.topk_tile == 8) GDX_TOPK_LAUNCH(false, 8);
+            else if (c.topk_tile == 16) GDX_TOPK_LAUNCH(false, 16);
+            else if (c.topk_tile == 32) GDX_TOPK_LAUNCH(false, 32);
+            else GDX_TOPK_LAUNCH(false, 0);
+        }
+        if (removal) GDX_TOPK_LAUNCH(bool(X_WEDGE), 0);
 #undef GDX_TOPK_LAUNCH
 #undef GDX_TOPK_SHAPED
         hip_check(hipGetLastError(), "launch top-K");

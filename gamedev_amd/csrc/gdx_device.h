@@ -67,6 +67,74 @@ __device__ __forceinline__ double col_uniform(uint32_t pidx, uint64_t seed, uint
 }
 
 // ---------------------------------------------------------------------------------------------
+// correctly rounded quotients, reciprocals and roots for the pair terms
+// ---------------------------------------------------------------------------------------------
+// The pair terms are bound by vector issue, and some two fifths of it is division and square root, which
+// the compiler expands for the whole range of a double: two scalings, two Newton steps and a fixup a
+// quotient (11 instructions, the seed at a quarter of the rate), a scaling both ways a root. The forms
+// below leave the scalings out and take one cubic step, e + e^2, from the seed of v_rcp_f64 (relative error
+// below 2^-23, so the cubic's is below 2^-69), then the exact remainder (Markstein, IA-64 and Elementary
+// Functions, 2000, ch. 8; roots after ch. 9). The reciprocal then has at most a rounding's error, the
+// remainder a - b q is exact, and the last step rounds a / b once: the same bits as a / b wherever neither
+// operand nor quotient nor remainder leaves the normal range, |b| within 2^+-1021 and |a| above 2^-960.
+// Compared with a / b, 1 / b and sqrt(x) on the device for 4e9 random operands of exponents up to +-480,
+// all-ones and all-zero mantissas among them: no bit differs. On the host they are the operators.
+#ifdef __HIP_DEVICE_COMPILE__
+__device__ __forceinline__ double near_recip(double b)
+{
+    const double y = __builtin_amdgcn_rcp(b);
+    const double e = fma(-b, y, 1.0);
+    return fma(y, fma(e, e, e), y);
+}
+#endif
+// RN(a/b) for finite a and finite nonzero b
+GDX_FN double quot(double a, double b)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    const double y = near_recip(b);
+    const double q = a*y;
+    return fma(fma(-b, q, a), y, q);
+#else
+    return a / b;
+#endif
+}
+// RN(a/b), zero, infinite and NaN operands as the division has them
+GDX_FN double quot_any(double a, double b)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_div_fixup(quot(a, b), b, a);
+#else
+    return a / b;
+#endif
+}
+// RN(1/b), zero, infinite and NaN operands as the division has them
+GDX_FN double recip(double b)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    const double y = near_recip(b);
+    return __builtin_amdgcn_div_fixup(fma(fma(-b, y, 1.0), y, y), b, 1.0);
+#else
+    return 1.0 / b;
+#endif
+}
+// RN(sqrt(x)): Goldschmidt's coupled iteration from v_rsq_f64, then the exact residual twice; NaN below zero
+GDX_FN double root(double x)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x*y, h = 0.5*y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    g = fma(fma(-g, g, x), h, g);
+    return __builtin_amdgcn_class(x, 0x260) ? x : g;      // +-0 and +inf
+#else
+    return sqrt(x);
+#endif
+}
+
+// ---------------------------------------------------------------------------------------------
 // disk and grain profiles (inc/swarm/param_phys.cuh:16-210, param_grid.cuh:23-27)
 // ---------------------------------------------------------------------------------------------
 GDX_FN double grain_mass(double size) { return PI*RHO_0*size*size*size / 6.0; }
@@ -211,12 +279,12 @@ GDX_FN double vrel_t_merged(double ris, double vg_sq, double stokes_i, double st
     {
         if (sl < 0.2*ris)
         {
-            v = vg_sq*(sl - ss)*(sl - ss) / ris;
+            v = quot_any(vg_sq*(sl - ss)*(sl - ss), ris);
         }
         else
         {
-            v = vg_sq*(sl - ss) / (sl + ss);
-            v *= (sl / (1.0 + ris / sl) - ss / (1.0 + ris / ss));
+            v = quot_any(vg_sq*(sl - ss), sl + ss);
+            v *= (quot_any(sl, 1.0 + quot_any(ris, sl)) - quot_any(ss, 1.0 + quot_any(ris, ss)));
         }
     }
     else if (small || sl < 1.0)
@@ -230,33 +298,33 @@ GDX_FN double vrel_t_merged(double ris, double vg_sq, double stokes_i, double st
             y +=  0.32938936*sl*sl;
             y += -0.29847604*sl*sl*sl;
         }
-        double d1 = (r3 ? sl - ss : ss) / (r3 ? sl + ss : sl);
+        double d1 = quot(r3 ? sl - ss : ss, r3 ? sl + ss : sl);
         double eps = d1;
-        double d2 = (r3 ? sl : 2.0) / (r3 ? 1.0 + y_a : 1.0 + eps);
-        double d3 = (r3 ? ss*ss : eps*eps*eps) / (r3 ? ss + y_a*sl : y + eps);
+        double d2 = quot(r3 ? sl : 2.0, r3 ? 1.0 + y_a : 1.0 + eps);
+        double d3 = quot(r3 ? ss*ss : eps*eps*eps, r3 ? ss + y_a*sl : y + eps);
         if (r3)
         {
             double coeff = d1;
             coeff *= (d2 - d3);
             coeff += 2.0*(y_a*sl - ris) + d2;
-            coeff -= sl*sl / (sl + ris);
+            coeff -= quot(sl*sl, sl + ris);
             coeff += d3;
-            coeff -= ss*ss / (ss + ris);
+            coeff -= quot(ss*ss, ss + ris);
             v = vg_sq*coeff;
         }
         else
         {
             double inv = 1.0 / (1.0 + y_a);
-            if (!(sl < 0.2)) inv = 1.0 / (1.0 + y);
+            if (!(sl < 0.2)) inv = recip(1.0 + y);
             v = vg_sq*sl;
             v *= (2.0*y - (1.0 + eps) + d2*(inv + d3));
         }
     }
     else
     {
-        v = vg_sq*(1.0 / (1.0 + sl) + 1.0 / (1.0 + ss));
+        v = vg_sq*(recip(1.0 + sl) + recip(1.0 + ss));
     }
-    return v < 0.0 ? __builtin_nan("") : sqrt(v);
+    return root(v);                        // NaN for a negative square (an invalid state)
 }
 
 // query-local drift + settling + turbulence (+ Brownian) speed (_collision.cuh:275-325, _col_rates.cuh:127-141)
@@ -346,7 +414,7 @@ constexpr double SQRT_HALF = 7.07106781186547524401e-01;
 // log((1 + f) 2^k) + c for 1 + f in [sqrt(1/2), sqrt(2)) and a small correction c
 GDX_FN double log_kernel(double f, int k, double c)
 {
-    double s = f / (2.0 + f);
+    double s = quot(f, 2.0 + f);
     double z = s*s;
     double R = z*fma(z, fma(z, fma(z, fma(z, fma(z, fma(z, LG7, LG6), LG5), LG4), LG3), LG2), LG1);
     double hfsq = 0.5*f*f;
@@ -398,7 +466,7 @@ GDX_FN double ulog(double x)
 // outcomes (inc/swarm/_col_event.cuh:15-109)
 // ---------------------------------------------------------------------------------------------
 GDX_FN double sticking_packet(double q)
-{ return q > 0.0 && q <= 1.0e-06 ? fmax(1.0, floor(1.0e-04 / q)) : 1.0; }
+{ return q > 0.0 && q <= 1.0e-06 ? fmax(1.0, floor(quot_any(1.0e-04, q))) : 1.0; }
 GDX_FN double mass_ratio(double size_i, double size_j)
 { double r = size_j / size_i; return r*r*r; }
 
@@ -527,11 +595,11 @@ GDX_FN double stokes_partner(const owner_terms &t, double size)
 GDX_FN void owner_resize(owner_terms &t, double size_i)
 {
     t.size_i = size_i;
-    t.inv_size = 1.0 / size_i;
+    t.inv_size = recip(size_i);
     if constexpr (COAG_KERNEL == 3)
     {
         t.si = stokes_partner(t, size_i);
-        t.fi = 1.0 / (1.0 + t.si*t.si);
+        t.fi = recip(1.0 + t.si*t.si);
         t.ai = t.si*t.fi;
         t.mi = fmin(t.si, 0.5);
     }
@@ -541,7 +609,7 @@ GDX_FN owner_terms make_owner(const gdx_env &e, double size_i, double m, double 
 {
     owner_terms t{};
     t.m = m;
-    t.inv_m = 1.0 / m;
+    t.inv_m = recip(m);
     if constexpr (COAG_KERNEL == 3)
     {
         t.vn = e.vn;
@@ -549,9 +617,9 @@ GDX_FN owner_terms make_owner(const gdx_env &e, double size_i, double m, double 
         t.ris = e.re_inv_sqrt;
         t.vg_sq = e.vg_sq;
         t.radial = e.radial;
-        t.inv_radial = 1.0 / e.radial;
+        t.inv_radial = recip(e.radial);
         t.strat = e.strat;
-        t.inv_strat = 1.0 / e.strat;
+        t.inv_strat = recip(e.strat);
         t.cs = e.cs;
         t.hg = hg_i;
     }
@@ -575,7 +643,7 @@ GDX_FN double sample_outcome_owner(const owner_terms &t, double sj, bool high_sp
 GDX_FN double vrel_pair_terms(const owner_terms &t, double size_j)
 {
     double sj = stokes_partner(t, size_j);
-    double fj = 1.0 / (1.0 + sj*sj);
+    double fj = recip(1.0 + sj*sj);
     double dvr = 2.0*t.vn*(t.ai - sj*fj);
     double dvphi = t.vn*(t.fi - fj);
     double dvz = t.zo*(t.mi - fmin(sj, 0.5));
@@ -586,7 +654,7 @@ GDX_FN double vrel_pair_terms(const owner_terms &t, double size_j)
     double mj = grain_mass(size_j);
     vb = fmin(sqrt(8.0*t.cs*t.cs*M_MOL*(mi + mj) / (PI*mi*mj)), t.cs);
 #endif
-    return sqrt(dvr*dvr + dvphi*dvphi + dvz*dvz + vt*vt + vb*vb);
+    return root(dvr*dvr + dvphi*dvphi + dvz*dvz + vt*vt + vb*vb);
 }
 
 // partner-only factors of one slot, held for the whole of an owner's event chain: the owner's position
@@ -608,7 +676,7 @@ GDX_FN partner_terms make_partner_terms(const owner_terms &t, double size_j)
     if constexpr (COAG_KERNEL == 3)
     {
         p.sj = stokes_partner(t, size_j);
-        p.fj = 1.0 / (1.0 + p.sj*p.sj);
+        p.fj = recip(1.0 + p.sj*p.sj);
         p.aj = p.sj*p.fj;
         p.mj = fmin(p.sj, 0.5);
     }
@@ -634,7 +702,7 @@ GDX_FN double vrel_pair_held(const owner_terms &t, const partner_terms &p, doubl
 #else
     (void)size_j;
 #endif
-    return sqrt(dvr*dvr + dvphi*dvphi + dvz*dvz + vt*vt + vb*vb);
+    return root(dvr*dvr + dvphi*dvphi + dvz*dvz + vt*vt + vb*vb);
 }
 
 // catastrophic-fragmentation moments (_col_event.cuh:62-73): they depend on the owner size alone
@@ -706,17 +774,18 @@ GDX_FN double outcome_moments_terms(const owner_terms &t, const CM &cm, double s
         mean = div_rn(lp, 3.0, INV_THREE);
         second = mean*mean;
         maximum = mean;
-        return Gp == 1.0 ? 1.0 : 1.0 / Gp;
+        return Gp == 1.0 ? 1.0 : recip(Gp);
     }
     if (q <= 0.1)
     {
-        double remnant = Gp == 1.0 ? (1.0 - q) : (1.0 - q) / Gp;
+        double remnant = Gp == 1.0 ? (1.0 - q) : quot_any(1.0 - q, Gp);
         double debris = q;
         double factor = remnant + debris;
         double jr = div_rn(-lp, 3.0, INV_THREE);
         double jd = div_rn(-ulog(q), 3.0, INV_THREE);
-        mean = (remnant*jr + debris*jd) / factor;
-        second = (remnant*jr*jr + debris*jd*jd) / factor;
+        const double inv_factor = recip(factor);
+        mean = div_rn(remnant*jr + debris*jd, factor, inv_factor);
+        second = div_rn(remnant*jr*jr + debris*jd*jd, factor, inv_factor);
         maximum = fmax(jr, jd);
         return factor;
     }
@@ -775,7 +844,7 @@ GDX_FN pair_term eval_pair_terms(const owner_terms &t, const CM &cm, const partn
     {
         vrel = HELD ? vrel_pair_held(t, pt, size_j) : vrel_pair_terms(t, size_j);
         rate = numr_j*vrel*PI*(size_i + size_j)*(size_i + size_j) / 4.0;
-        if constexpr (N_Z == 1) rate /= sqrt(2.0*PI*(t.hg*t.hg + q.hg_j*q.hg_j));
+        if constexpr (N_Z == 1) rate = quot_any(rate, root(2.0*PI*(t.hg*t.hg + q.hg_j*q.hg_j)));
     }
     double r = div_rn(rate, t.m, t.inv_m);
     double mean = 0.0, second = 0.0, maximum = 0.0;
@@ -797,10 +866,10 @@ GDX_FN double outcome_factor(const owner_terms &t, double sj, bool high_speed)
     double ratio = div_rn(sj, si, t.inv_size);
     double q = ratio*ratio*ratio;
     double Gp = sticking_packet(q);
-    if (!high_speed) return Gp == 1.0 ? 1.0 : 1.0 / Gp;
+    if (!high_speed) return Gp == 1.0 ? 1.0 : recip(Gp);
     if (q <= 0.1)
     {
-        double remnant = Gp == 1.0 ? (1.0 - q) : (1.0 - q) / Gp;
+        double remnant = Gp == 1.0 ? (1.0 - q) : quot_any(1.0 - q, Gp);
         return remnant + q;
     }
     return 1.0;
@@ -832,7 +901,7 @@ GDX_FN pair_term eval_pair_rate(const owner_terms &t, const partner &q, double l
     {
         vrel = HELD ? vrel_pair_held(t, pt, size_j) : vrel_pair_terms(t, size_j);
         rate = numr_j*vrel*PI*(size_i + size_j)*(size_i + size_j) / 4.0;
-        if constexpr (N_Z == 1) rate /= sqrt(2.0*PI*(t.hg*t.hg + q.hg_j*q.hg_j));
+        if constexpr (N_Z == 1) rate = quot_any(rate, root(2.0*PI*(t.hg*t.hg + q.hg_j*q.hg_j)));
     }
     double r = div_rn(rate, t.m, t.inv_m);
     r *= outcome_factor(t, size_j, vrel >= V_FRAG);

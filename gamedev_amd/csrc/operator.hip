@@ -398,6 +398,9 @@ __global__ __launch_bounds__(BLOCK) void k_mark_stale(const gdx_gref *table, con
 // reference's upper-half fold, and higher levels combine through a carry stack whose branches
 // depend only on the chunk index (wavefront-uniform). The sums equal the fold bit for bit.
 // ---------------------------------------------------------------------------------------------
+// finite and >= 0: zeros of either sign, positive subnormal and normal numbers (one class test)
+__device__ __forceinline__ bool rate_ok(double r) { return __builtin_amdgcn_class(r, 0x1e0); }
+
 struct fold3
 {
     double r, a, b;
@@ -461,19 +464,19 @@ __device__ __forceinline__ rate_sums owner_rate_sums(const gdx_gref *GP, int s, 
         const partner q2 = load_partner(jj.z, res, hgs), q3 = load_partner(jj.w, res, hgs);
         pair_term p = eval(q0);
         fold3 a{p.rate, p.j1, p.j2};
-        V = V && isfinite(p.rate) && p.rate >= 0.0;
+        V = V && rate_ok(p.rate);
         JM = fmax(JM, p.jmax);
         p = eval(q1);
         a = add3(a, {p.rate, p.j1, p.j2});
-        V = V && isfinite(p.rate) && p.rate >= 0.0;
+        V = V && rate_ok(p.rate);
         JM = fmax(JM, p.jmax);
         p = eval(q2);
         fold3 b{p.rate, p.j1, p.j2};
-        V = V && isfinite(p.rate) && p.rate >= 0.0;
+        V = V && rate_ok(p.rate);
         JM = fmax(JM, p.jmax);
         p = eval(q3);
         b = add3(b, {p.rate, p.j1, p.j2});
-        V = V && isfinite(p.rate) && p.rate >= 0.0;
+        V = V && rate_ok(p.rate);
         JM = fmax(JM, p.jmax);
         fold3 part = add3(a, b);
         if (chunks) chunks[c] = part.r;
@@ -545,19 +548,19 @@ __device__ __forceinline__ rate_sums group_rate_sums(const gdx_gref *GP, int s, 
         const partner q2 = load_partner(jj.z, res, hgs), q3 = load_partner(jj.w, res, hgs);
         pair_term p = eval(q0);
         fold3 a{p.rate, p.j1, p.j2};
-        V = V && isfinite(p.rate) && p.rate >= 0.0;
+        V = V && rate_ok(p.rate);
         JM = fmax(JM, p.jmax);
         p = eval(q1);
         a = add3(a, {p.rate, p.j1, p.j2});
-        V = V && isfinite(p.rate) && p.rate >= 0.0;
+        V = V && rate_ok(p.rate);
         JM = fmax(JM, p.jmax);
         p = eval(q2);
         fold3 b{p.rate, p.j1, p.j2};
-        V = V && isfinite(p.rate) && p.rate >= 0.0;
+        V = V && rate_ok(p.rate);
         JM = fmax(JM, p.jmax);
         p = eval(q3);
         b = add3(b, {p.rate, p.j1, p.j2});
-        V = V && isfinite(p.rate) && p.rate >= 0.0;
+        V = V && rate_ok(p.rate);
         JM = fmax(JM, p.jmax);
         fold3 part = add3(a, b);
         if (chunks) chunks[c] = part.r;
@@ -1876,7 +1879,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain(gdx_wave w)
             double wait = 0.0;
             if (!now)
             {
-                wait = nx_nl / R;
+                wait = quot_any(nx_nl, R);
                 ++pool_used;
             }
             double remaining = end - time;
@@ -1927,7 +1930,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain(gdx_wave w)
                             evw[s].count[cat] += 1ull;
                             evw[s].log_mass[cat] += log_mass;
                         }
-                        numr_i = mass_before / (size_new*size_new*size_new);
+                        numr_i = quot_any(mass_before, size_new*size_new*size_new);
                         time = event_time;
                         ++events;
                         double mass_after = numr_i*size_new*size_new*size_new;

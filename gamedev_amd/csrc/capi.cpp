@@ -789,6 +789,7 @@ void run_swarms(std::vector<op_run *> &runs, run_buffers &rb, hipStream_t st, ke
             z.add(rb.hcount.p, sizeof(int)*ng);
             z.add(rb.ccount.p, sizeof(int)*ng);
             z.add(rb.wave_ctr.p, sizeof(unsigned long long)*GDX_WAVE_CTRS*nr);
+            z.add(rb.log_next.p, sizeof(int));
             phase_wave pw = upload_phase(rb, e, st, z, narrow_owners);
             timer.time(GDX_COL_KERNEL_SCREEN, pw.w256.total, [&] {
                 if (pw.narrow) launch_screen(st, pw.w256, pw.blocks256, true);
@@ -796,12 +797,18 @@ void run_swarms(std::vector<op_run *> &runs, run_buffers &rb, hipStream_t st, ke
             });
             if (pw.w256.learned && pw.blocks256)
                 timer.time(GDX_COL_KERNEL_CANDIDATES, pw.w256.total, [&] { launch_candidates(st, pw.w256, pw.blocks256, rb.cprefix.p); });
-            if (pw.blocks256)
+            // the chain's blocks form the prefixes of few groups themselves; under kernel timing they stay a launch
+            // of their own, timed as such
+            const bool own_prefix = pw.w256.n <= CHAIN_OWN_PREFIX && !timer.on();
+            if (pw.blocks256 && !own_prefix)
                 timer.time(GDX_COL_KERNEL_PREFIX, pw.w256.total, [&] { launch_queue_prefix(st, pw.w256, rb.qprefix.p); });
-            timer.time(GDX_COL_KERNEL_CHAIN, pw.w256.total, [&] { launch_chain(st, pw.w256, rb.resident); });
-            timer.time(GDX_COL_KERNEL_AUDIT, pw.w256.total, [&] { launch_chain_audit(st, pw.w1024, pw.blocks1024); });
+            timer.time(GDX_COL_KERNEL_CHAIN, pw.w256.total, [&] { launch_chain(st, pw.w256, rb, own_prefix); });
+            timer.time(GDX_COL_KERNEL_AUDIT, pw.w256.total, [&] { launch_chain_audit(st, pw.w1024, pw.blocks1024, rb); });
             rb.read_back(rb.off_wave, rb.back_bytes, st);          // wave counters, errors, audit bins
             wait_stream(st, "chain pass");
+            unsigned long long longest = 0;
+            for (op_run *r : now) longest = std::max(longest, r->wave_ctr[GDX_WAVE_LONGEST]);
+            rb.log_phases = longest >= (unsigned long long)LONG_CHAIN ? CHAIN_LOG_PHASES : std::max(0, rb.log_phases - 1);
             for (op_run *r : now) r->after_chain();
             upload_changed(now);
         }

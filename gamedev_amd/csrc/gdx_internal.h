@@ -134,6 +134,10 @@ struct view
     const T *data() const { return p; }
 };
 
+// a chain of this many events in one phase makes the next phases keep the solo owners' logs: 16 waves of short
+// chains lose 4 us each to the launch, a chain of LONG_CHAIN events gains 0.1 ms
+constexpr int LONG_CHAIN = 64, CHAIN_LOG_PHASES = 32;
+
 // buffers of operator runs: the group table, pinned staging and device copies of the due lists,
 // the chain's queue prefix
 struct run_buffers
@@ -157,6 +161,27 @@ struct run_buffers
     dbuf<int> nchanged;               // entries of each changed-slot list
     int changed_cap = 0;              // entries each changed-slot list can hold
     int resident = 0;                 // resident blocks of the persistent chain kernel
+    // the solo heavy owners' logs of one chain launch (gdx_chain_log)
+    gdx_chain_log log{};
+    dbuf<double2> log_entry;
+    dbuf<double4> log_part;
+    dbuf<int4> log_use;
+    dbuf<int> log_prev, log_last, log_next;
+    // chain phases that keep logs still to come after a chain of LONG_CHAIN events (CHAIN_LOG_PHASES each
+    // time). The logs cost a launch; without them a long chain costs its owner's moments at every event. The
+    // results do not depend on it.
+    int log_phases = CHAIN_LOG_PHASES;
+    void reserve_log(int owners)
+    {
+        const size_t chunks = size_t(owners) + CHAIN_EXTRA;
+        log_entry.alloc(chunks*CHAIN_CHUNK);
+        log_part.alloc(chunks);
+        log_use.alloc(chunks);
+        log_prev.alloc(chunks);
+        log_last.alloc(size_t(owners));
+        log = gdx_chain_log{log_entry.p, log_part.p, log_use.p, log_prev.p, log_last.p, log_next.p, owners,
+                            log_phases > 0, hcount.p, qcount.p};
+    }
     // controller sums, queue lengths, counters and errors of every group and swarm of the run. The
     // read-backs share one device block and one page-locked mirror laid out [raw_rate][wave_ctr][err]
     // [raw_audit], so that the rate phase reads [raw_rate, wave_ctr] and the chain phase [wave_ctr,
@@ -192,6 +217,7 @@ struct run_buffers
         qcount.alloc(groups);
         hcount.alloc(groups);
         ccount.alloc(groups);
+        log_next.alloc(1);
         counters.alloc(size_t(swarms)*GDX_CTRS);
         h_counters.resize(size_t(swarms)*GDX_CTRS);
     }
@@ -377,6 +403,8 @@ void launch_bath_rate_grouped(hipStream_t st, const gdx_wave &w, int blocks);
 // owners), else four per lane over block starts of 1024
 void launch_screen(hipStream_t st, const gdx_wave &w, int blocks, bool narrow);
 void launch_candidates(hipStream_t st, const gdx_wave &w, int blocks, int *vstart);
+// due groups whose queue prefixes the chain's blocks form themselves; more take a launch of their own
+constexpr int CHAIN_OWN_PREFIX = 256;
 void launch_queue_prefix(hipStream_t st, const gdx_wave &w, int *qprefix);
 void launch_majorant(hipStream_t st, const gdx_wave &w, int blocks);
 void launch_zero(hipStream_t st, const zero_ranges &z);
@@ -393,8 +421,8 @@ unsigned long long majorant_version(gdx_col_majorant m);
 void invalidate_bounds(context &c);
 void build_reverse(context &c);
 int chain_resident_blocks();
-void launch_chain(hipStream_t st, const gdx_wave &w, int resident);
-void launch_chain_audit(hipStream_t st, const gdx_wave &w, int blocks);
+void launch_chain(hipStream_t st, const gdx_wave &w, run_buffers &rb, bool own_prefix);
+void launch_chain_audit(hipStream_t st, const gdx_wave &w, int blocks, const run_buffers &rb);
 void launch_event_sum(context &c, hipStream_t st);
 void launch_gather_cached(context &c, double *out_particle_order);
 void launch_pair_rates(context &c, const gdx_gref &G, double *out_particle_order);

@@ -1598,6 +1598,132 @@ __global__ __launch_bounds__(256) void k_queue_prefix(gdx_wave w, int *qprefix)
     }
 }
 
+// ---- one owner on a whole wavefront (k_chain's solo heavy owners) ----
+// Lane l holds neighbour slot l % N_K: with fewer slots than lanes the wavefront holds copies, so that
+// every total is on every lane and nothing needs a segment mask, a lane broadcast or LDS.
+
+// the reference's upper-half fold over the slots (slot j with j + K/2 first), on every lane: lane swaps
+// between halves and rows, then rotations within a row, which meet the partner j +- 4 of a value already
+// the same at j and j + 8
+__device__ __forceinline__ double solo_fold(double v)
+{
+    auto lower = [](double x, bool half) {
+        const unsigned lo = __double2loint(x), hi = __double2hiint(x);
+        const auto a = half ? __builtin_amdgcn_permlane32_swap(lo, lo, false, false)
+                            : __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto b = half ? __builtin_amdgcn_permlane32_swap(hi, hi, false, false)
+                            : __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        return __hiloint2double(b[0], a[0]) + __hiloint2double(b[1], a[1]);
+    };
+    if constexpr (N_K == 64) v = lower(v, true);
+    if constexpr (N_K >= 32) v = lower(v, false);
+    v += dpp_move<0x128, 0xf, true>(v);            // row_ror:8
+    v += dpp_move<0x124, 0xf, true>(v);            // row_ror:4
+    v += dpp_move<0x4e, 0xf, true>(v);             // quad_perm [2,3,0,1]
+    v += dpp_move<0xb1, 0xf, true>(v);             // quad_perm [1,0,3,2]
+    return v;
+}
+
+// partner-only factors of a slot, fixed over the owner's chain
+struct solo_partner
+{
+    partner q;
+    partner_terms pt;
+    double overlap;
+    bool has;
+};
+
+__device__ __forceinline__ solo_partner make_solo_partner(const owner_terms &t, const partner &q)
+{
+    solo_partner s{q, partner_terms{0.0, 0.0, 0.0, 0.0}, 1.0, q.valid};
+    if constexpr (COAG_KERNEL == 3)
+    {
+        s.pt = make_partner_terms(t, q.size_j);
+        if constexpr (N_Z == 1) s.overlap = root(2.0*PI*(t.hg*t.hg + q.hg_j*q.hg_j));
+    }
+    return s;
+}
+
+// vrel_t_merged where the wavefront's lanes mostly share one regime, as the partners of one grain far larger
+// than them do: without lanes elsewhere, regimes 4 and 5 are one straight line (1 / (1 + y) is formed for
+// both: the same bits as regime 4's constant) and regime 6 another
+__device__ __forceinline__ double solo_vrel_t(double ris, double vg_sq, double stokes_i, double stokes_j)
+{
+    const bool mine = stokes_i >= stokes_j;
+    const double sl = mine ? stokes_i : stokes_j, ss = mine ? stokes_j : stokes_i;
+    const bool small = sl < 5.0*ris;
+    const unsigned long long outside = __ballot(small), middle = __ballot(sl < 1.0);
+    if (outside == 0ull && middle == ~0ull)
+    {
+        double y = 1.6015125;
+        y += -0.63119577*sl;
+        y +=  0.32938936*sl*sl;
+        y += -0.29847604*sl*sl*sl;
+        y = sl < 0.2 ? 1.6 : y;
+        const double eps = quot(ss, sl);
+        const double d2 = quot(2.0, 1.0 + eps);
+        const double d3 = quot(eps*eps*eps, y + eps);
+        const double inv = recip(1.0 + y);
+        double v = vg_sq*sl;
+        v *= (2.0*y - (1.0 + eps) + d2*(inv + d3));
+        return root(v);
+    }
+    if (outside == 0ull && middle == 0ull) return root(vg_sq*(recip(1.0 + sl) + recip(1.0 + ss)));
+    return vrel_t_merged(ris, vg_sq, stokes_i, stokes_j);
+}
+
+// eval_pair_rate, bit for bit, by selects; the sticking packet only where some lane has one above 1
+__device__ __forceinline__ double solo_pair_rate(const owner_terms &t, const solo_partner &s, double lambda_0, double &vrel)
+{
+    const double size_i = t.size_i, size_j = s.q.size_j, numr_j = s.q.numr_j;
+    double rate;
+    vrel = 0.0;
+    if constexpr (COAG_KERNEL == 0)
+    {
+        rate = lambda_0*numr_j;
+    }
+    else if constexpr (COAG_KERNEL == 1)
+    {
+        rate = lambda_0*numr_j*(grain_mass(size_i) + grain_mass(size_j));
+    }
+    else if constexpr (COAG_KERNEL == 2)
+    {
+        rate = lambda_0*numr_j*grain_mass(size_i)*grain_mass(size_j);
+    }
+    else
+    {
+        const double dvr = 2.0*t.vn*(t.ai - s.pt.aj);
+        const double dvphi = t.vn*(t.fi - s.pt.fj);
+        const double dvz = t.zo*(t.mi - s.pt.mj);
+        const double vt = solo_vrel_t(t.ris, t.vg_sq, t.si, s.pt.sj);
+        double square = dvr*dvr + dvphi*dvphi + dvz*dvz + vt*vt;
+#ifndef CODE_UNIT
+        const double mi = grain_mass(size_i), mj = grain_mass(size_j);
+        const double vb = fmin(sqrt(8.0*t.cs*t.cs*M_MOL*(mi + mj) / (PI*mi*mj)), t.cs);
+        square += vb*vb;
+#endif
+        vrel = root(square);
+        rate = numr_j*vrel*PI*(size_i + size_j)*(size_i + size_j) / 4.0;
+        if constexpr (N_Z == 1) rate = quot_any(rate, s.overlap);
+    }
+    double r = div_rn(rate, t.m, t.inv_m);
+    const double ratio = div_rn(size_j, size_i, t.inv_size);
+    const double q = ratio*ratio*ratio;
+    const bool high = vrel >= V_FRAG;
+    double low_factor = 1.0, remnant = 1.0 - q;
+    if (__ballot(q > 0.0 && q <= 1.0e-06))
+    {
+        const double Gp = sticking_packet(q);
+        const bool one = Gp == 1.0;
+        low_factor = one ? 1.0 : recip(Gp);
+        if constexpr (CAN_FRAGMENT) remnant = one ? remnant : quot_any(1.0 - q, Gp);
+    }
+    double factor = low_factor;
+    if constexpr (CAN_FRAGMENT) factor = high ? (q <= 0.1 ? remnant + q : 1.0) : low_factor;
+    r *= factor;
+    return s.has ? r : 0.0;
+}
+
 // event chains (col_chain_run.cu:127-382): a persistent grid over the queued owners. Each K-lane segment
 // of a wavefront runs one owner to its bath end, then takes the wavefront's next owner; the chain sums go
 // to the owner's queue position for the audit pass. The owners are dealt out without atomics: heavy
@@ -1607,7 +1733,7 @@ __global__ __launch_bounds__(256) void k_queue_prefix(gdx_wave w, int *qprefix)
 // not the chains, set the launch's length.
 constexpr int CHAIN_PREFIX_LDS = 4096;     // due groups whose queue prefix a chain block keeps in LDS
 
-__global__ __launch_bounds__(BLOCK) void k_chain(gdx_wave w)
+__global__ __launch_bounds__(BLOCK) void k_chain(gdx_wave w, gdx_chain_log clog, int *qprefix)
 {
     __shared__ double walk[WAVES][NSEG][N_K];
     __shared__ int qp[2*(CHAIN_PREFIX_LDS + 1)];
@@ -1619,10 +1745,49 @@ __global__ __launch_bounds__(BLOCK) void k_chain(gdx_wave w)
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     // the queue prefixes of the due groups (heavy, then light), searched at every refill: LDS when
     // they fit. Positions [0, heavy) of the run are the heavy queues, group after group; the rest are
-    // the light queues.
+    // the light queues. Of few groups every block forms them itself (a launch less on the way of a small
+    // wave), and the first block leaves them for the kernels after this one.
     const bool in_lds = w.n <= CHAIN_PREFIX_LDS;
-    if (in_lds)
+    if (qprefix)
+    {
+        static_assert(CHAIN_OWN_PREFIX <= BLOCK, "one group per thread");
+        __shared__ int part[2][WAVES];
+        const int i = threadIdx.x;
+        const int ref = w.ref[min(i, w.n - 1)];
+        const int mine[2] = {i < w.n ? clog.hcount[ref] : 0, i < w.n ? clog.qcount[ref] : 0};
+        int incl[2] = {mine[0], mine[1]};
+#pragma unroll
+        for (int d = 1; d < WAVE; d <<= 1)
+        {
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+            {
+                const int v = __shfl_up(incl[k], d, WAVE);
+                if (lane >= d) incl[k] += v;
+            }
+        }
+        if (lane == WAVE - 1) { part[0][wave] = incl[0]; part[1][wave] = incl[1]; }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+        {
+            int at = incl[k] - mine[k];
+            for (int v = 0; v < wave; ++v) at += part[k][v];
+            int *out = qp + k*(w.n + 1);
+            if (i <= w.n) out[i] = at;
+            if (i == BLOCK - 1 && w.n == BLOCK) out[BLOCK] = at + mine[k];
+            if (blockIdx.x == 0)
+            {
+                int *keep = qprefix + k*(w.n + 1);
+                if (i <= w.n) keep[i] = at;
+                if (i == BLOCK - 1 && w.n == BLOCK) keep[BLOCK] = at + mine[k];
+            }
+        }
+    }
+    else if (in_lds)
+    {
         for (int i = threadIdx.x; i < 2*(w.n + 1); i += BLOCK) qp[i] = w.qprefix[i];
+    }
     __syncthreads();
     const int *hprefix = in_lds ? qp : w.qprefix;
     const int *lprefix = hprefix + w.n + 1;
@@ -1691,20 +1856,206 @@ __global__ __launch_bounds__(BLOCK) void k_chain(gdx_wave w)
     const int nwaves = int(gridDim.x)*WAVES;
     const int gw = int(blockIdx.x)*WAVES + wave;
     const int light = total - heavy;
-    const bool solo = heavy <= nwaves / 2;
+    const bool solo = heavy <= clog.owners;   // half the grid's wavefronts
     const int hstride = solo && heavy > 0 ? nwaves / heavy : nwaves;
     int hn = solo ? ((gw % hstride == 0 && gw / hstride < heavy) ? gw / hstride : heavy) : gw;
-    const int hstep = solo ? heavy : nwaves;  // a solo wavefront's one heavy position, then none
+    const int hstep = nwaves;
     const int lb1 = int((long long)light*(blockIdx.x + 1) / gridDim.x);
     if (threadIdx.x == 0) lpool = int((long long)light*blockIdx.x / gridDim.x);
     __syncthreads();
+    // ---- a solo heavy owner on the whole wavefront, event after event ----
+    // The longest chains set the launch's length, and a chain is latency: on one wavefront an event of the
+    // general loop below took some 8,400 cycles, 630 vector instructions among 46 branches and a dozen LDS
+    // round trips. Here the lanes are copies in slot order (solo_fold), so totals, the partner walk and the
+    // chosen partner need no LDS; the pair rate is straight-line where the lanes share a regime; and the jump
+    // moments, which only the audit needs, are left out of the chain: each waiting interval goes to the
+    // owner's log and k_chain_moments forms their sums afterwards, every interval on its own. Whatever is
+    // not an ordinary event (an invalid rate or state, a walk too close to call, no log left) leaves the
+    // owner as it was before that event to the general loop, which forms everything again.
+    // Clumped swarm of 46,425, longest chains of 800 events: 8,400 -> 3,290 cycles an event, the launch
+    // 1,175 -> 515 us.
+    if (solo && hn < heavy)
+    {
+        const int h = hn;
+        hn = heavy;
+        int lo = 0, hi = w.n - 1;
+        while (lo < hi)
+        {
+            const int mid = (lo + hi + 1) >> 1;
+            if (hprefix[mid] <= h) lo = mid;
+            else hi = mid - 1;
+        }
+        gi = __builtin_amdgcn_readfirstlane(lo);
+        G = w.table + w.ref[gi];
+        ctr_of = G->counters;
+        wave_of = G->wave_ctr;
+        pos = w.beg[gi] + (h - hprefix[gi]);
+        s = G->queue[pos];
+        end = w.dt[gi];
+        seed = G->seed;
+        lambda_0 = G->lambda_0;
+        const double2 cur = G->st[s];
+        numr_i = cur.y;
+        ctr = G->rng[s];
+        pidx = uint32_t(G->slot_pidx[s]);
+        double hg_i = 0.0;
+        gdx_env e{};
+        if constexpr (COAG_KERNEL == 3) e = G->env[s];
+        if constexpr (PARTNER_HG) hg_i = G->hgs[s];
+        const double measure_i = G->measure[s];
+        const int *row = G->nbr + (long long)s*N_K;
+        const partner fresh = load_partner(row[bitrev_slot(lane % N_K)], G->res, G->hgs);
+        t = make_owner(e, cur.x, measure_i, hg_i);
+        moments = exact_owner(w, gi, s);
+        if (w.learned && w.sub[gi] >= 0)
+        {
+            const double2 qs = G->qstart[pos];
+            time = qs.x;
+            first_event = qs.y == 1.0;
+            if (qs.y == 2.0) events = 1;
+        }
+        heavy_owner = true;
+        walk_exact = G->exact_walk != 0;
+        evw = G->evw;
+        bool done = false;
+        uint64_t used = 0;                                   // draws taken
+        // the owner's log: its present chunk, -1 once there are no more, and the intervals in it. The next
+        // chunk is asked for when this one is half full, so that its number is there when it is needed.
+        int chunk = h, logged = 0, ahead = 0;
+        bool asked = false;
+        if (lane == 0 && clog.enabled) clog.prev[h] = -1;
+        auto note = [&](double size, double length) {
+            if (lane == 0) clog.entry[(long long)chunk*CHAIN_CHUNK + logged] = make_double2(size, length);
+            ++logged;
+            if (logged == CHAIN_CHUNK / 2)
+            {
+                if (lane == 0) ahead = atomicAdd(clog.next, 1);
+                asked = true;
+            }
+            if (logged < CHAIN_CHUNK) return;
+            const int c = __builtin_amdgcn_readfirstlane(ahead);
+            if (lane == 0)
+            {
+                clog.use[chunk] = make_int4(w.ref[gi], s, CHAIN_CHUNK, 0);
+                if (c < CHAIN_EXTRA) clog.prev[clog.owners + c] = chunk;
+                else clog.last[h] = chunk;
+            }
+            chunk = c < CHAIN_EXTRA ? clog.owners + c : -1;
+            logged = 0;
+            asked = false;
+        };
+        if (!first_event && !walk_exact && !evw && (!moments || clog.enabled))
+        {
+            __builtin_amdgcn_s_setprio(2);
+            const solo_partner me = make_solo_partner(t, fresh);
+            // the next 64 draws, one per lane, as the general loop's pool
+            int at = WAVE;
+            double draw_u = 0.0, draw_nl = 0.0;
+            while (true)
+            {
+                if (at > WAVE - 3)
+                {
+                    at = 0;
+                    draw_u = col_uniform_at(pidx, seed, ctr + used + uint64_t(lane));
+                    draw_nl = -log(draw_u);
+                }
+                double vrel;
+                const double rate = solo_pair_rate(t, me, lambda_0, vrel);
+                const double R = solo_fold(rate);
+                const double nl = lane_value(draw_nl, at), u1 = lane_value(draw_u, at + 1);
+                // the walk in slot order, decided by tree partials where they are clear of the target (see the
+                // general loop)
+                const double target = u1*R;
+                const double a = seg_scan(rate);
+                const bool above = a*(1.0 - 0x1p-44) - 0x1p-1000 > target;
+                const bool below = a*(1.0 + 0x1p-44) + 0x1p-1000 <= target;
+                const unsigned long long hit = __ballot(rate > 0.0 && above);
+                const unsigned long long odd = __ballot(!rate_ok(rate) || (rate > 0.0 && !above && !below));
+                const double wait = quot_any(nl, R), remaining = end - time;
+                const double event_time = time + wait;
+                // ordinary: every rate valid, the walk decided, a positive finite wait that moves the clock
+                const bool plain = odd == 0ull && hit != 0ull && wait > 0.0 && wait < __builtin_inf()
+                    && (!moments || chunk >= 0);
+                if (!__builtin_amdgcn_readfirstlane(plain)) break;
+                n_pairs += lane == 0 ? N_K : 0;
+                if (__builtin_amdgcn_readfirstlane(wait >= remaining))
+                {
+                    hazard += R*remaining;
+                    if (moments) note(t.size_i, remaining);
+                    ++used;
+                    time = end;
+                    done = true;
+                    break;
+                }
+                const int slot = int(__builtin_ctzll(hit));
+                const double size_j = lane_value(me.q.size_j, slot), v_j = lane_value(vrel, slot);
+                const double size_i = t.size_i;
+                const double mass_before = numr_i*size_i*size_i*size_i;
+                const bool high_speed = __builtin_amdgcn_readfirstlane(v_j >= V_FRAG);
+                const double sample = high_speed ? lane_value(draw_u, at + 2) : 0.0;
+                const double size_new = sample_outcome_owner(t, size_j, high_speed, sample);
+                const double numr_new = quot_any(mass_before, size_new*size_new*size_new);
+                const double mass_after = numr_new*size_new*size_new*size_new;
+                const double mass_scale = fmax(fabs(mass_before), fabs(mass_after));
+                const bool sound = size_new > 0.0 && size_new < __builtin_inf() && numr_new > 0.0
+                    && numr_new < __builtin_inf() && !(fabs(mass_after - mass_before) > 2.0e-12*mass_scale)
+                    && event_time > time && events + 1 < EVENT_LIMIT;
+                if (!__builtin_amdgcn_readfirstlane(sound))
+                {
+                    n_pairs -= lane == 0 ? N_K : 0;
+                    break;
+                }
+                hazard += R*wait;
+                if (moments) note(size_i, wait);
+                const int draws = high_speed ? 3 : 2;
+                at += draws;
+                used += draws;
+                numr_i = numr_new;
+                time = event_time;
+                ++events;
+                owner_resize(t, size_new);
+            }
+        }
+        if (lane == 0 && chunk >= 0 && clog.enabled)
+        {
+            clog.use[chunk] = make_int4(w.ref[gi], s, logged, 0);
+            clog.last[h] = moments ? chunk : -1;
+            // a chunk asked for and not begun
+            if (asked && ahead < CHAIN_EXTRA) clog.use[clog.owners + ahead] = make_int4(w.ref[gi], s, 0, 0);
+        }
+        if (done)
+        {
+            if (lane == 0)
+            {
+                if (events > 0)
+                {
+                    G->st[s] = make_double2(t.size_i, numr_i);
+                    G->dirty[s] = 1;
+                }
+                G->rng[s] = ctr + used;
+                G->qsum[pos] = make_double4(hazard, 0.0, 0.0, 0.0);
+                G->qevents[pos] = events;
+                longest = max(longest, events);
+                n_blocks += (unsigned long long)(events / COL_EVENT_CAP + 1);
+                n_events += events;
+                n_chain += 1;
+            }
+        }
+        else if (seg == 0)
+        {
+            // the general loop goes on from here on the first segment, lanes in row order
+            ctr += used;
+            refill(ctr);
+            q = load_partner(row[kl], G->res, G->hgs);
+            if constexpr (HOLD_PARTNER) pt = make_partner_terms(t, q.size_j);
+            active = true;
+        }
+    }
     while (true)
     {
         unsigned long long need = __ballot(!active) & seg_lead;
-        // a solo heavy owner runs alone: its wavefront takes nothing while it runs, and only that owner
-        // (on the first segment) at its first refill
+        // a solo heavy owner handed on by the block above runs alone: its wavefront takes nothing meanwhile
         if (solo && __ballot(active && heavy_owner)) need = 0ull;
-        if (solo && hn < heavy) need &= 1ull;
         if (need)
         {
             // free segments, in lane order, take the next heavy positions, then the next light ones
@@ -2003,13 +2354,100 @@ __global__ __launch_bounds__(BLOCK) void k_chain(gdx_wave w)
     }
 }
 
+// jump moments of the solo heavy owners' logged intervals: j1 and j2 are sums over intervals of the moment
+// sums at the owner's size times the interval, jmax their maximum (col_chain_run.cu:188-214). One block
+// per chunk, a quarter of its intervals per wavefront and NSEG at a time, as the general loop forms them; the
+// audit adds an owner's chunks.
+constexpr int MOMENT_GRID = 256;
+
+__global__ __launch_bounds__(BLOCK) void k_chain_moments(gdx_wave w, gdx_chain_log clog)
+{
+    __shared__ double sums[WAVES][NSEG][3];
+    const int heavy = w.qprefix[w.n];
+    if (heavy == 0 || heavy > clog.owners) return;
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    const int seg = lane / SEG, kl = lane % SEG;
+    const int items = heavy + min(*clog.next, CHAIN_EXTRA);
+    for (int item = blockIdx.x; item < items; item += gridDim.x)
+    {
+        const int chunk = item < heavy ? item : clog.owners + (item - heavy);
+        const int4 use = clog.use[chunk];
+        const int s = use.y, count = use.z;
+        if (count == 0)
+        {
+            if (threadIdx.x == 0) clog.part[chunk] = make_double4(0.0, 0.0, 0.0, 0.0);
+            continue;
+        }
+        const gdx_gref *G = w.table + use.x;
+        const double lambda_0 = G->lambda_0;
+        double hg_i = 0.0;
+        gdx_env e{};
+        if constexpr (COAG_KERNEL == 3) e = G->env[s];
+        if constexpr (PARTNER_HG) hg_i = G->hgs[s];
+        const double m = G->measure[s];
+        const partner q = load_partner(G->nbr[(long long)s*N_K + kl], G->res, G->hgs);
+        const double2 *entries = clog.entry + (long long)chunk*CHAIN_CHUNK;
+        double j1 = 0.0, j2 = 0.0, jmax = 0.0;
+        constexpr int SHARE = CHAIN_CHUNK / WAVES;
+        const int end = min(count, (wave + 1)*SHARE);
+        for (int i = wave*SHARE; i < end; i += NSEG)
+        {
+            const bool own = i + seg < end;
+            const double2 interval = own ? entries[i + seg] : make_double2(1.0, 0.0);
+            const owner_terms t = make_owner(e, interval.x, m, hg_i);
+            pair_term p = eval_pair_terms(t, cat_moments_deferred{}, q, lambda_0);
+            if constexpr (CAN_FRAGMENT)
+            {
+                const bool cat = own && q.valid && catastrophic_pair(t, q.size_j, p.vrel >= V_FRAG);
+                if (__ballot(cat))
+                {
+                    const cat_moments c = catastrophic_moments(t.size_i);
+                    if (cat)
+                    {
+                        p.j1 = p.rate*c.mean;
+                        p.j2 = p.rate*c.second;
+                        p.jmax = p.rate > 0.0 ? c.maximum : 0.0;
+                    }
+                }
+            }
+            const double J1 = seg_fold<false>(p.j1), J2 = seg_fold<false>(p.j2), JM = seg_fold<true>(p.jmax);
+            if (own)
+            {
+                j1 += J1*interval.y;
+                j2 += J2*interval.y;
+                jmax = fmax(jmax, JM);
+            }
+        }
+        // the segments' sums in a fixed order
+        if (kl == 0)
+        {
+            sums[wave][seg][0] = j1;
+            sums[wave][seg][1] = j2;
+            sums[wave][seg][2] = jmax;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0)
+        {
+            const double *v = &sums[0][0][0];
+            for (int k = 1; k < WAVES*NSEG; ++k)
+            {
+                j1 += v[3*k];
+                j2 += v[3*k + 1];
+                jmax = fmax(jmax, v[3*k + 2]);
+            }
+            clog.part[chunk] = make_double4(j1, j2, jmax, 0.0);
+        }
+        __syncthreads();
+    }
+}
+
 // audit of the chained owners, one lane per queue position of each due group (col_audit_bin.cu:13-60),
 // AUDIT_ROUNDS positions per lane: a block covers 1024 slots of its group, and blocks without a queued
 // position (most of them, the queues being short) leave after reading two counters
 constexpr int AUDIT_ROUNDS = 4;
 static_assert(BLOCK*AUDIT_ROUNDS == PUBLISH_OWNERS, "the audit uses the 1024-owner block starts");
 
-__global__ __launch_bounds__(BLOCK) void k_chain_audit(gdx_wave w)
+__global__ __launch_bounds__(BLOCK) void k_chain_audit(gdx_wave w, gdx_chain_log clog)
 {
     __shared__ audit_lds a;
     int gi, s0, s1;
@@ -2019,6 +2457,9 @@ __global__ __launch_bounds__(BLOCK) void k_chain_audit(gdx_wave w)
     const int h1 = w.beg[gi] + *G.hcount;
     const int l0 = w.beg[gi] + w.cnt[gi] - *G.qcount;
     if (s0 >= h1 && s1 <= l0) return;
+    // the heavy positions' logged jump moments (k_chain_moments), where the heavy owners ran alone
+    const bool logs = clog.enabled && w.qprefix[w.n] <= clog.owners;
+    const int hbase = w.qprefix[gi] - w.beg[gi];
     const double end = w.dt[gi];
     const double lo = *G.lower, up = *G.upper;
     const int *__restrict__ queue = G.queue;
@@ -2049,6 +2490,16 @@ __global__ __launch_bounds__(BLOCK) void k_chain_audit(gdx_wave w)
             rate0 = cached[s].x;
             sum = qsum[pos];
             events = qevents[pos];
+            if (logs && pos < h1)
+            {
+                for (int k = clog.last[hbase + pos]; k >= 0; k = clog.prev[k])
+                {
+                    const double4 v = clog.part[k];
+                    sum.y += v.x;
+                    sum.z += v.y;
+                    sum.w = fmax(sum.w, v.z);
+                }
+            }
         }
         if (take)
         {
@@ -2299,6 +2750,12 @@ void launch_candidates(hipStream_t st, const gdx_wave &w, int blocks, int *vstar
     hip_check(hipGetLastError(), "launch candidates");
 }
 
+// blocks of the chain's persistent grid: at most what the GPU holds, fewer for small waves
+static int chain_grid(const gdx_wave &w, int resident)
+{
+    return std::max(1, std::min(resident, (w.total + 4*NSEG - 1) / (4*NSEG)));
+}
+
 void launch_queue_prefix(hipStream_t st, const gdx_wave &w, int *qprefix)
 {
     k_queue_prefix<<<1, 256, 0, st>>>(w, qprefix);
@@ -2314,19 +2771,24 @@ int chain_resident_blocks()
     return std::max(1, per_cu*cus);
 }
 
-// a persistent grid of at most `resident` blocks, fewer for small waves
-void launch_chain(hipStream_t st, const gdx_wave &w, int resident)
+// after launch_queue_prefix of the same wave unless own_prefix (at most CHAIN_OWN_PREFIX due groups); then the
+// jump moments of the intervals that the chain's solo heavy owners logged
+void launch_chain(hipStream_t st, const gdx_wave &w, run_buffers &rb, bool own_prefix)
 {
     if (!w.total) return;
-    int grid = std::max(1, std::min(resident, (w.total + 4*NSEG - 1) / (4*NSEG)));
-    k_chain<<<grid, BLOCK, 0, st>>>(w);
+    const int grid = chain_grid(w, rb.resident);
+    rb.reserve_log(grid*WAVES / 2);
+    k_chain<<<grid, BLOCK, 0, st>>>(w, rb.log, own_prefix ? rb.qprefix.p : nullptr);
     hip_check(hipGetLastError(), "launch chain");
+    if (!rb.log.enabled) return;
+    k_chain_moments<<<MOMENT_GRID, BLOCK, 0, st>>>(w, rb.log);
+    hip_check(hipGetLastError(), "launch chain moments");
 }
 
-void launch_chain_audit(hipStream_t st, const gdx_wave &w, int blocks)
+void launch_chain_audit(hipStream_t st, const gdx_wave &w, int blocks, const run_buffers &rb)
 {
     if (!blocks) return;
-    k_chain_audit<<<xcd_grid(blocks), BLOCK, 0, st>>>(w);
+    k_chain_audit<<<xcd_grid(blocks), BLOCK, 0, st>>>(w, rb.log);
     hip_check(hipGetLastError(), "launch chain audit");
 }
 

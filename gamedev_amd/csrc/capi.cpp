@@ -1303,7 +1303,7 @@ int gdx_col_get_kdtree(gdx_col_handle h, int *node_idx, int *node_dim, float *wo
             {
                 int d;
                 std::memcpy(&d, &nodes[i].w, sizeof d);
-                node_dim[i] = d;
+                node_dim[i] = d & 3;     // above it: the site is active
             }
         }
         hip_check(hipStreamSynchronize(c.stream), "read k-d tree");

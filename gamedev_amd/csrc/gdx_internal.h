@@ -116,7 +116,7 @@ void swap_buf(dbuf<T> &a, dbuf<T> &b)
     std::swap(a.n, b.n);
 }
 
-// left-balanced k-d tree over all collision sites, node order: {x, y, z, split dim bits}
+// left-balanced k-d tree over all collision sites, node order: {x, y, z, bits: split dim | active site << 2}
 struct kd_tree
 {
     int n = 0;

@@ -14,7 +14,7 @@
 // moves its point into the left or right child subtree, or settles it as the subtree's pivot, and
 // sets its split dimension to the widest extent of the child subtree's domain.
 // Query: one lane per active owner, owners taken in Morton order so that neighbouring lanes walk
-// similar paths; heap and stack are per-lane private arrays. Rows are written in heap order.
+// similar paths; heap and path are columns of LDS. Rows are written in heap order.
 #include "gdx_internal.h"
 #include "gdx_device.h"
 
@@ -29,7 +29,7 @@ namespace {
 
 constexpr int KD_BLOCK = 256;
 constexpr int KD_QUERY_BLOCK = 64;
-constexpr int KD_STACK = 30;                 // depth of a left-balanced tree of up to 2^30 points
+constexpr int KD_ACTIVE = 4;                 // flag beside the split dimension in node.w
 constexpr int WAVE = 64;
 
 int blocks(long long n, int per) { return static_cast<int>((n + per - 1) / per); }
@@ -46,7 +46,12 @@ __device__ __forceinline__ uint32_t ordered(float x)
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-__device__ __forceinline__ float coord(const float4 &p, int d) { return d == 0 ? p.x : (d == 1 ? p.y : p.z); }
+__device__ __forceinline__ float pick(int d, float x, float y, float z)
+{
+    const float v = d == 1 ? y : x;
+    return d == 2 ? z : v;
+}
+__device__ __forceinline__ float coord(const float4 &p, int d) { return pick(d, p.x, p.y, p.z); }
 
 struct kd_box
 {
@@ -170,14 +175,18 @@ __global__ __launch_bounds__(KD_BLOCK) void k_kd_keys(const float4 *node, const 
 }
 
 __global__ __launch_bounds__(KD_BLOCK) void k_kd_gather(const uint64_t *key, const int *val, const float4 *node,
-                                                       const int *idx, int n, bool tag_only, float4 *node_out,
+                                                       const int *idx, int n, bool tag_only,
+                                                       const unsigned char *active, int n_phys, float4 *node_out,
                                                        int *idx_out, uint32_t *tag_out)
 {
     int i = blockIdx.x*KD_BLOCK + threadIdx.x;
     if (i >= n) return;
     int from = val[i];
-    node_out[i] = node[from];
-    idx_out[i] = idx[from];
+    float4 p = node[from];
+    const int r = idx[from];
+    if (tag_only && active[r % n_phys]) p.w = __int_as_float(__float_as_int(p.w) | KD_ACTIVE);
+    node_out[i] = p;
+    idx_out[i] = r;
     tag_out[i] = tag_only ? uint32_t(key[i]) : uint32_t(key[i] >> 32);
 }
 
@@ -223,6 +232,13 @@ __device__ __forceinline__ float d2_of(float ax, float ay, float az, float bx, f
 
 __device__ __forceinline__ float key_d2(uint64_t k) { return __uint_as_float(uint32_t(k >> 32)); }
 
+// nextafterf(x, inf) for x >= 0 or NaN
+__device__ __forceinline__ float above(float x)
+{
+    const uint32_t u = __float_as_uint(x);
+    return __uint_as_float(u + (u < 0x7f800000u ? 1u : 0u));
+}
+
 // col_site_init's wedge images (src/swarm/col_site_init.cu:42-62): physical points at [0, n), every point
 // rotated by -width (image 1) at [n, 2n) and by +width (image 2) at [2n, 3n)
 __global__ __launch_bounds__(KD_BLOCK) void k_kd_images(const float4 *pts, int n, float cw, float sw, float4 *out)
@@ -239,18 +255,91 @@ __global__ __launch_bounds__(KD_BLOCK) void k_kd_images(const float4 *pts, int n
     }
 }
 
+// max-heap columns in LDS: `cand` takes the place of the entry at `slot` and sinks. The larger child and its
+// children are read together, which halves the chain of dependent LDS reads.
+__device__ __forceinline__ void sift_from(uint64_t *heap, int slot, uint64_t cand)
+{
+    for (int child = 2*slot + 1; child < N_K; child = 2*slot + 1)
+    {
+        uint64_t cv = heap[child*WAVE];
+        if (child + 1 < N_K)
+        {
+            const uint64_t other = heap[(child + 1)*WAVE];
+            if (other > cv) { cv = other; ++child; }
+        }
+        if (cv < cand) break;
+        heap[slot*WAVE] = cv;
+        slot = child;
+    }
+    heap[slot*WAVE] = cand;
+}
+
+// the same from the root: slots 1 .. N_K - 2 fill their levels, slot N_K - 1 is the only one below them
+// returns the new root
+__device__ __forceinline__ uint64_t sift_root(uint64_t *heap, uint64_t cand)
+{
+    int slot = 0;
+    bool sinks = true;
+    uint64_t root = cand;
+#pragma unroll
+    for (int l = 1; l < LOG2K; l += 2)
+    {
+        if (!sinks) continue;
+        int child = 2*slot + 1;
+        const uint64_t *h = heap + child*WAVE, *g = h + (child + 1)*WAVE;      // children, grandchildren
+        const uint64_t a = h[0], b = h[WAVE];
+        uint64_t g0 = 0, g1 = 0, g2 = 0, g3 = 0;
+        if (l + 1 < LOG2K) { g0 = g[0]; g1 = g[WAVE]; g2 = g[2*WAVE]; g3 = g[3*WAVE]; }
+        const bool right = b > a;
+        const uint64_t cv = right ? b : a;
+        if (right) { ++child; g0 = g2; g1 = g3; }
+        sinks = !(cv < cand);
+        if (!sinks) continue;
+        if (l == 1) root = cv;
+        heap[slot*WAVE] = cv;
+        slot = child;
+        if (l + 1 == LOG2K) continue;
+        child = 2*slot + 1 + (g1 > g0 ? 1 : 0);
+        const uint64_t gv = g1 > g0 ? g1 : g0;
+        sinks = !(gv < cand);
+        if (!sinks) continue;
+        heap[slot*WAVE] = gv;
+        slot = child;
+    }
+    if (slot == N_K / 2 - 1)
+    {
+        const uint64_t cv = heap[(N_K - 1)*WAVE];
+        if (!(cv < cand)) { heap[slot*WAVE] = cv; slot = N_K - 1; }
+    }
+    heap[slot*WAVE] = cand;
+    return root;
+}
+
 // queries: the nq physical particles in Morton order; the tree holds nt records, record r being particle
 // r % n_phys at image r / n_phys when n_phys > 0 (a wedge), else particle r
-__global__ __launch_bounds__(KD_QUERY_BLOCK) void k_kd_topk(const float4 *node, const int *node_idx, int nt, int nq,
+//
+// A lane walks the tree alone, so what bounds it is the latency of a chain of node loads and the heap, both of
+// which are indexed differently in every lane. Heap and path values live in LDS, one column per lane (no bank
+// conflicts whatever the index); as private arrays they were scratch, whose 38 KB per wavefront did not fit the
+// caches. The path takes 8 bytes per level: the far child of a path node is the path's sibling one level down,
+// so a pending one is a bit, with the plane's coordinate and the distance of the closest corner behind it; the
+// corner itself follows from the planes of the far sides that the path is on. 1e6 points, 32 neighbours:
+// 13.1 -> 2.6 ms (262 visits and 217 heap insertions per wavefront, 6 wavefronts per CU).
+__global__ __launch_bounds__(KD_QUERY_BLOCK) void k_kd_topk(const float4 *__restrict__ node,
+                                                           const int *__restrict__ node_idx, int nt, int nq,
                                                            int n_phys, float image_dist_min,
                                                            const float *world, const int *sidx, const float4 *pts,
                                                            const unsigned char *active, const int *pidx_slot,
                                                            const unsigned char *group, bound_state u, int *nbr,
                                                            double *measure, unsigned long long *graph,
-                                                           unsigned int *overflow, unsigned char *nbr_image)
+                                                           unsigned char *nbr_image)
 {
+    static_assert(KD_QUERY_BLOCK == WAVE, "one wavefront per block: no column is shared");
+    extern __shared__ uint64_t kd_lds[];
     const int lane = threadIdx.x % WAVE;
-    const int m = blockIdx.x*KD_QUERY_BLOCK + threadIdx.x;
+    uint64_t *const heap = kd_lds + lane;                                            // [N_K] columns
+    float2 *const path = reinterpret_cast<float2 *>(kd_lds + N_K*WAVE) + lane;        // [levels of the tree]
+    const int m = xcd_block()*KD_QUERY_BLOCK + threadIdx.x;
     const int n = nt;
     const int p = m < nq ? sidx[m] : 0;
     const bool qactive = m < nq && active[p];
@@ -259,94 +348,107 @@ __global__ __launch_bounds__(KD_QUERY_BLOCK) void k_kd_topk(const float4 *node, 
     if (qactive)
     {
         const float4 qp = pts[p];
-        uint64_t heap[N_K];
         const uint64_t empty = (uint64_t(__float_as_uint(qp.w*qp.w)) << 32) | 0xffffffffull;
         // one entry per particle when two of its images can share this ball (_col_cache.cuh:38-41)
         const bool dedup = X_WEDGE && !(image_dist_min < 0.0f || image_dist_min > 2.0f*qp.w);
-#pragma unroll
-        for (int k = 0; k < N_K; ++k) heap[k] = empty;
-        int st_node[KD_STACK];
-        float st_c[KD_STACK][3];
-        int sp = 0;
-        float cull = nextafterf(key_d2(heap[0]), __builtin_inff());
-        float cx = fminf(fmaxf(qp.x, world[0]), world[3]);
-        float cy = fminf(fmaxf(qp.y, world[1]), world[4]);
-        float cz = fminf(fmaxf(qp.z, world[2]), world[5]);
+        for (int k = 0; k < N_K; ++k) heap[k*WAVE] = empty;
+        uint64_t top = empty;                                  // the heap's root
+        float cull = above(key_d2(top));
+        const float wx = fminf(fmaxf(qp.x, world[0]), world[3]);
+        const float wy = fminf(fmaxf(qp.y, world[1]), world[4]);
+        const float wz = fminf(fmaxf(qp.z, world[2]), world[5]);
+        float cx = wx, cy = wy, cz = wz;
+        // bit l: the far child of the path's node at level l is still to be visited (pending) or the path goes
+        // through it (taken); is_y, is_z: the node's split dimension
+        unsigned int pending = 0u, taken = 0u, is_y = 0u, is_z = 0u;
+        unsigned int id = 0u;
+        int level = 0;
         bool run = !(d2_of(cx, cy, cz, qp.x, qp.y, qp.z) > cull);
-        int id = 0;
+        float4 np = node[0];
+        int r = node_idx[0];
         while (run)
         {
-            if (id >= n)
-            {
-                bool found = false;
-                while (sp > 0)
-                {
-                    --sp;
-                    cx = st_c[sp][0]; cy = st_c[sp][1]; cz = st_c[sp][2];
-                    if (d2_of(cx, cy, cz, qp.x, qp.y, qp.z) >= cull) continue;
-                    id = st_node[sp];
-                    found = true;
-                    break;
-                }
-                if (!found) break;
-            }
-            const float4 np = node[id];
-            const int r = node_idx[id];
-            const int image = X_WEDGE ? r / n_phys : 0;
-            const int j = X_WEDGE ? r - image*n_phys : r;
+            const int bits = __float_as_int(np.w);
+            const int dim = bits & 3;
             const float d2 = d2_of(np.x, np.y, np.z, qp.x, qp.y, qp.z);
-            if (active[j])
-            {
-                uint64_t cand = (uint64_t(__float_as_uint(d2)) << 32) | uint32_t(3*j + image);
-                // a particle already in the heap is replaced only by a nearer image of itself
-                // (idx_old_heap::processCandidate, inc/swarm/kdtree/index_heap.cuh:112-175)
-                int slot = 0;
-                bool take = cand < heap[0];
-                if (X_WEDGE && dedup)
-                {
-                    int found = -1;
-#pragma unroll
-                    for (int k = 0; k < N_K; ++k)
-                    {
-                        const uint32_t ck = uint32_t(heap[k]);
-                        if (found < 0 && ck != 0xffffffffu && int(ck / 3u) == j) found = k;
-                    }
-                    if (found >= 0)
-                    {
-                        slot = found;
-                        take = cand < heap[found];
-                    }
-                }
-                if (take)
-                {
-                    while (true)
-                    {
-                        int child = 2*slot + 1;
-                        if (child >= N_K) { heap[slot] = cand; break; }
-                        uint64_t cv = heap[child];
-                        if (child + 1 < N_K && heap[child + 1] > cv) { cv = heap[child + 1]; ++child; }
-                        if (cv < cand) { heap[slot] = cand; break; }
-                        heap[slot] = cv;
-                        slot = child;
-                    }
-                }
-            }
-            cull = nextafterf(key_d2(heap[0]), __builtin_inff());
-            const int dim = __float_as_int(np.w);
             const float nd = coord(np, dim);
             const bool left_close = coord(qp, dim) < nd;
-            const int lc = 2*id + 1, rc = lc + 1;
-            const int far = left_close ? rc : lc;
-            float fx = cx, fy = cy, fz = cz;
-            if (dim == 0) fx = nd; else if (dim == 1) fy = nd; else fz = nd;
-            if (far < n && d2_of(fx, fy, fz, qp.x, qp.y, qp.z) < cull)
+            const unsigned int lc = 2u*id + 1u;
+            const unsigned int near = left_close ? lc : lc + 1u, far = left_close ? lc + 1u : lc;
+            // the near child's record is on its way while the heap takes this one
+            const unsigned int ahead = min(near, unsigned(n) - 1u);
+            const float4 next = node[ahead];
+            const int next_r = node_idx[ahead];
+            if ((bits & KD_ACTIVE) && __float_as_uint(d2) <= uint32_t(top >> 32))
             {
-                if (sp == KD_STACK) { atomicOr(overflow, 1u); run = false; break; }
-                st_node[sp] = far;
-                st_c[sp][0] = fx; st_c[sp][1] = fy; st_c[sp][2] = fz;
-                ++sp;
+                const int image = X_WEDGE ? r / n_phys : 0;
+                const int j = X_WEDGE ? r - image*n_phys : r;
+                const uint64_t cand = (uint64_t(__float_as_uint(d2)) << 32) | uint32_t(3*j + image);
+                // a particle already in the heap is replaced only by a nearer image of itself
+                // (idx_old_heap::processCandidate, inc/swarm/kdtree/index_heap.cuh:112-175)
+                int found = -1;
+                if (X_WEDGE && dedup)
+                {
+                    for (int k = 0; k < N_K; ++k)
+                    {
+                        const uint32_t ck = uint32_t(heap[k*WAVE]);
+                        if (found < 0 && ck != 0xffffffffu && int(ck / 3u) == j) found = k;
+                    }
+                }
+                if (X_WEDGE && found >= 0)
+                {
+                    if (cand < heap[found*WAVE]) sift_from(heap, found, cand);
+                    top = heap[0];
+                }
+                else if (cand < top)
+                {
+                    top = sift_root(heap, cand);
+                }
+                cull = above(key_d2(top));
             }
-            id = left_close ? lc : rc;
+            const float far_d2 = d2_of(dim == 0 ? nd : cx, dim == 1 ? nd : cy, dim == 2 ? nd : cz, qp.x, qp.y, qp.z);
+            if (far < unsigned(n) && far_d2 < cull)
+            {
+                const unsigned int bit = 1u << level;
+                path[level*WAVE] = make_float2(nd, far_d2);
+                pending |= bit;
+                is_y = dim == 1 ? is_y | bit : is_y & ~bit;
+                is_z = dim == 2 ? is_z | bit : is_z & ~bit;
+            }
+            id = near;
+            ++level;
+            np = next;
+            r = next_r;
+            if (id >= unsigned(n))
+            {
+                // the deepest far child that is still close enough
+                while (pending)
+                {
+                    const int l = 31 - __clz(static_cast<int>(pending));
+                    if (path[l*WAVE].y < cull) break;
+                    pending &= ~(1u << l);
+                }
+                run = pending != 0u;
+                if (run)
+                {
+                    const int l = 31 - __clz(static_cast<int>(pending));
+                    const unsigned int bit = 1u << l;
+                    pending &= ~bit;
+                    taken = (taken & (bit - 1u)) | bit;
+                    id = (((id + 1u) >> (level - l - 1)) ^ 1u) - 1u;
+                    level = l + 1;
+                    np = node[id];
+                    r = node_idx[id];
+                    // its closest corner: in each dimension the plane of the deepest far side that the path is on
+                    const unsigned int tx = taken & ~(is_y | is_z), ty = taken & is_y, tz = taken & is_z;
+                    cx = tx ? path[(31 - __clz(static_cast<int>(tx)))*WAVE].x : wx;
+                    cy = ty ? path[(31 - __clz(static_cast<int>(ty)))*WAVE].x : wy;
+                    cz = tz ? path[(31 - __clz(static_cast<int>(tz)))*WAVE].x : wz;
+                }
+            }
+            // one latch: lanes that go down and lanes that go back visit their next nodes together (as two nested
+            // loops, which the compiler makes of it otherwise, a wavefront takes 420 visits instead of 260)
+            __builtin_amdgcn_wave_barrier();
         }
         const int s = pidx_slot[p];
         float max_d2 = 0.0f;
@@ -354,10 +456,11 @@ __global__ __launch_bounds__(KD_QUERY_BLOCK) void k_kd_topk(const float4 *node, 
 #pragma unroll
         for (int k = 0; k < N_K; ++k)
         {
-            uint32_t code = uint32_t(heap[k]);
+            const uint64_t entry = heap[k*WAVE];
+            const uint32_t code = uint32_t(entry);
             if (code != 0xffffffffu)
             {
-                max_d2 = fmaxf(max_d2, key_d2(heap[k]));
+                max_d2 = fmaxf(max_d2, key_d2(entry));
                 int jj = int(code) / 3;
                 row[k] = pidx_slot[jj];
                 mask |= 1ull << group[jj];
@@ -377,7 +480,7 @@ __global__ __launch_bounds__(KD_QUERY_BLOCK) void k_kd_topk(const float4 *node, 
 #pragma unroll
             for (int t = 0; t < N_K; ++t)
             {
-                const uint32_t code = uint32_t(heap[bitrev_slot(t)]);
+                const uint32_t code = uint32_t(heap[bitrev_slot(t)*WAVE]);
                 nbr_image[(long long)s*N_K + t] = static_cast<unsigned char>(code != 0xffffffffu ? code % 3u : 0u);
             }
         }
@@ -452,7 +555,7 @@ void kd_build(context &c)
         int tag_bits = tag_only ? levels : L + 1;
         radix_sort_pairs(key.p, val.p, n, 0, (tag_only ? 0 : 32) + tag_bits, c.scratch, st);
         k_kd_gather<<<blocks(n, KD_BLOCK), KD_BLOCK, 0, st>>>(key.p, val.p, t.node.p, t.idx.p, n, tag_only,
-                                                             node_b.p, idx_b.p, tag_b.p);
+                                                             c.active.p, c.n, node_b.p, idx_b.p, tag_b.p);
         hip_check(hipGetLastError(), "launch k-d sort");
         swap_buf(t.node, node_b);
         swap_buf(t.idx, idx_b);
@@ -482,10 +585,12 @@ void kd_query(context &c)
             *std::fabs(sinf1(0.5f*(x_max - x_min)));
         c.nbr_image.alloc(size_t(std::max(1, c.n_active))*N_K);
     }
-    k_kd_topk<<<blocks(n, KD_QUERY_BLOCK), KD_QUERY_BLOCK, 0, c.stream>>>(
+    int levels = 0;
+    while ((1ll << levels) - 1 < c.kd.n) ++levels;
+    const size_t lds = size_t(WAVE)*(N_K*sizeof(uint64_t) + levels*sizeof(float2));
+    k_kd_topk<<<xcd_grid(blocks(n, KD_QUERY_BLOCK)), KD_QUERY_BLOCK, lds, c.stream>>>(
         c.kd.node.p, c.kd.idx.p, c.kd.n, n, X_WEDGE ? n : 0, image_dist_min, c.kd.world.p, c.index.idx.p, c.pts.p,
-        c.active.p, c.pidx_slot.p, c.group.p, c.user, c.nbr.p, c.measure.p, c.graph.p, c.overflow.p,
-        c.nbr_image.p);
+        c.active.p, c.pidx_slot.p, c.group.p, c.user, c.nbr.p, c.measure.p, c.graph.p, c.nbr_image.p);
     hip_check(hipGetLastError(), "launch k-d top-K");
 }
 

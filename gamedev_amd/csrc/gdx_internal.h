@@ -123,6 +123,9 @@ struct kd_tree
     dbuf<float4> node;
     dbuf<int> idx;             // particle index per node
     dbuf<float> world;         // data bounds {lo xyz, hi xyz}
+    // workspace of the build: points in two orders, subtree segments of two levels, digit counts and cursors
+    dbuf<float4> points[2];
+    dbuf<unsigned int> segments, counts;
 };
 
 // a typed view into one of run_buffers' shared allocations

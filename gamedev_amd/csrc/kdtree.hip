@@ -8,11 +8,12 @@
 // (inc/swarm/kdtree/index_heap.cuh:11-177) and the closest-corner-tracking traversal
 // (inc/swarm/kdtree/traverse-cct.h:26-100).
 //
-// Build: every level sorts (tag, coordinate along the point's split dimension) with the library's
-// stable LSD radix sort (the reference's thrust::sort is not stable, so its layout for equal
-// coordinates is unspecified; this layout is the stable one), then one thread per array position
-// moves its point into the left or right child subtree, or settles it as the subtree's pivot, and
-// sets its split dimension to the widest extent of the child subtree's domain.
+// Layout: a subtree's pivot is the point of rank `left size` among its points, ordered along its split dimension;
+// points that tie there keep the order that the level above gave them, and so on up to the input order (the
+// stable one; the reference's thrust::sort is not stable, so its layout for equal coordinates is unspecified).
+// That order is a comparison of a point's coordinates, the most recently used split dimension first, and of its
+// index at last, so no level has to be sorted: subtrees of more than KD_SLOTS points are split by a radix
+// selection of the pivot and a partition in any order, smaller ones are finished in LDS by one block each.
 // Query: one lane per active owner, owners taken in Morton order so that neighbouring lanes walk
 // similar paths; heap and path are columns of LDS. Rows are written in heap order.
 #include "gdx_internal.h"
@@ -74,62 +75,102 @@ __device__ __forceinline__ int widest(const kd_box &b)
     return best;
 }
 
-__device__ __forceinline__ int level_of(int node) { return 63 - __clzll(static_cast<long long>(node) + 1ll); }
-__device__ __forceinline__ int levels_for(int n) { return level_of(n - 1) + 1; }
-__device__ __forceinline__ int full_nodes(int levels) { return (1 << levels) - 1; }
-
-__device__ __forceinline__ int subtree_size(int n, int root)
+// points left of the pivot of a left-balanced subtree of m points
+__host__ __device__ __forceinline__ int kd_left(int m)
 {
-    int levels_sub = levels_for(n) - level_of(root);
-    int first = (root + 1) << (levels_sub - 1);
-    int on_last = 1 << (levels_sub - 1);
-    int last_on_last = first + on_last - 1;
-    int missing = min(max(last_on_last - n, 0), on_last);
-    return full_nodes(levels_sub) - missing;
-}
-
-// array position of a level-L subtree's pivot during step L
-__device__ __forceinline__ int pivot_pos(int L, int n, int subtree)
-{
-    int settled = full_nodes(L);
-    int levels_total = levels_for(n);
-    int remaining = levels_total - L;
-    int earlier = subtree - settled;
-    int left_if_full = earlier*full_nodes(remaining);
-    int left_on_last_if_full = earlier*(1 << (remaining - 1));
-    int total_on_last = n - full_nodes(levels_total - 1);
-    int missing = left_on_last_if_full - min(total_on_last, left_on_last_if_full);
-    int left_root = 2*subtree + 1;
-    return settled + left_if_full - missing + (left_root >= n ? 0 : subtree_size(n, left_root));
+    if (m < 2) return 0;
+    const int levels = 32 - __builtin_clz(static_cast<unsigned int>(m));
+    const int half = 1 << (levels - 2);
+    const int last = m - ((1 << (levels - 1)) - 1);
+    return half - 1 + (last < half ? last : half);
 }
 
 // ---------------------------------------------------------------------------------------------
 // build
 // ---------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(KD_BLOCK) void k_kd_init(const float4 *pts, int n, float4 *node, int *idx,
-                                                     unsigned int *world_bits)
+constexpr int KD_LDS_LEVELS = 12, KD_SLOTS = 1 << KD_LDS_LEVELS;      // largest subtree of the LDS part
+constexpr int KD_FINISH_BLOCK = 1024;
+constexpr int KD_SPLIT_BLOCK = 512, KD_CHUNK = 4096;
+constexpr int KD_BINS = 2048;                                         // 11 bits a digit, three digits a coordinate
+constexpr int KD_TIES = 1024;
+constexpr int KD_INIT_BLOCKS = 512;
+constexpr uint32_t KD_SITE = 0x80000000u;                             // active flag beside the point's index
+
+// a subtree before its split: the box of its domain as ordered keys, its points [start, start + size) and the
+// order of its points: split dimension | second << 2 | third << 4, 3 for none
+struct kd_seg
+{
+    uint32_t lo[3], hi[3];
+    int start, size, order;
+};
+
+// a digit's outcome: leading bits of the pivot's key, its rank among the points that share them, their number
+struct kd_sel
+{
+    uint32_t prefix;
+    int rank, count;
+};
+
+__device__ __forceinline__ float unordered(uint32_t u)
+{
+    return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
+}
+
+// the order of a subtree's points: its widest dimension, then the dimensions used above it, latest first
+__device__ __forceinline__ int order_of(const uint32_t lo[3], const uint32_t hi[3], int above)
+{
+    kd_box b;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) { b.lo[d] = unordered(lo[d]); b.hi[d] = unordered(hi[d]); }
+    const int dim = widest(b), a0 = above & 3, a1 = (above >> 2) & 3;
+    if (dim == a0) return above;
+    if (dim == a1) return dim | (a0 << 2) | (above & 0x30);
+    return dim | (a0 << 2) | (a1 << 4);
+}
+
+// whether p comes before q where they tie in the split dimension
+__device__ __forceinline__ bool tie_less(const float4 &p, const float4 &q, int order)
+{
+#pragma unroll
+    for (int k = 2; k < 6; k += 2)
+    {
+        const int d = (order >> k) & 3;
+        if (d == 3) break;
+        const uint32_t a = ordered(coord(p, d)), b = ordered(coord(q, d));
+        if (a != b) return a < b;
+    }
+    return (__float_as_uint(p.w) & ~KD_SITE) < (__float_as_uint(q.w) & ~KD_SITE);
+}
+
+__device__ __forceinline__ void put_node(const float4 &p, int dim, long long tag, float4 *node, int *idx)
+{
+    const uint32_t w = __float_as_uint(p.w);
+    node[tag] = make_float4(p.x, p.y, p.z, __int_as_float(dim | ((w & KD_SITE) ? KD_ACTIVE : 0)));
+    idx[tag] = int(w & ~KD_SITE);
+}
+
+__global__ __launch_bounds__(KD_BLOCK) void k_kd_init(const float4 *pts, const unsigned char *active, int n,
+                                                     int n_phys, float4 *out, unsigned int *world_bits)
 {
     __shared__ unsigned int red[6][KD_BLOCK / WAVE];
-    int i = blockIdx.x*KD_BLOCK + threadIdx.x;
-    float4 p = pts[min(i, n - 1)];
-    if (i < n)
+    // world box of the data: minima of the ordered keys and of their complements, one atomic per block and bound
+    unsigned int k[6] = {~0u, ~0u, ~0u, ~0u, ~0u, ~0u};
+    for (long long i = (long long)blockIdx.x*KD_BLOCK + threadIdx.x; i < n; i += (long long)gridDim.x*KD_BLOCK)
     {
-        node[i] = make_float4(p.x, p.y, p.z, __int_as_float(0));
-        idx[i] = i;
+        float4 p = pts[i];
+        const unsigned int o[3] = {ordered(p.x), ordered(p.y), ordered(p.z)};
+#pragma unroll
+        for (int d = 0; d < 3; ++d) { k[d] = min(k[d], o[d]); k[3 + d] = min(k[3 + d], ~o[d]); }
+        p.w = __uint_as_float(uint32_t(i) | (active[X_WEDGE ? int(i) % n_phys : int(i)] ? KD_SITE : 0u));
+        out[i] = p;
     }
-    // world box of the data: ordered-key minima and maxima, one atomic per block and bound
-    unsigned int k[6] = {ordered(p.x), ordered(p.y), ordered(p.z), ordered(p.x), ordered(p.y), ordered(p.z)};
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
 #pragma unroll
     for (int b = 0; b < 6; ++b)
     {
         unsigned int v = k[b];
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1)
-        {
-            unsigned int t = __shfl_xor(v, o, WAVE);
-            v = (b < 3) ? min(v, t) : max(v, t);
-        }
+        for (int o = 32; o > 0; o >>= 1) v = min(v, static_cast<unsigned int>(__shfl_xor(v, o, WAVE)));
         if (lane == 0) red[b][wave] = v;
     }
     __syncthreads();
@@ -137,88 +178,399 @@ __global__ __launch_bounds__(KD_BLOCK) void k_kd_init(const float4 *pts, int n, 
     {
         int b = threadIdx.x;
         unsigned int v = red[b][0];
-        for (int w = 1; w < KD_BLOCK / WAVE; ++w) v = (b < 3) ? min(v, red[b][w]) : max(v, red[b][w]);
-        if (b < 3) atomicMin(world_bits + b, v);
-        else atomicMax(world_bits + b, v);
+        for (int w = 1; w < KD_BLOCK / WAVE; ++w) v = min(v, red[b][w]);
+        atomicMin(world_bits + b, v);
     }
 }
 
-__device__ __forceinline__ float unordered(uint32_t u)
-{
-    return __uint_as_float((u & 0x80000000u) ? (u & 0x7fffffffu) : ~u);
-}
-
-__global__ void k_kd_world(const unsigned int *world_bits, float *world, int *dim0)
+__global__ void k_kd_root(const unsigned int *world_bits, int n, float *world, kd_seg *seg)
 {
     if (threadIdx.x != 0) return;
-    kd_box b;
-    for (int d = 0; d < 3; ++d) { b.lo[d] = unordered(world_bits[d]); b.hi[d] = unordered(world_bits[3 + d]); }
-    for (int d = 0; d < 3; ++d) { world[d] = b.lo[d]; world[3 + d] = b.hi[d]; }
-    *dim0 = widest(b);
-}
-
-__global__ __launch_bounds__(KD_BLOCK) void k_kd_dim0(float4 *node, int n, const int *dim0)
-{
-    int i = blockIdx.x*KD_BLOCK + threadIdx.x;
-    if (i < n) node[i].w = __int_as_float(*dim0);
-}
-
-__global__ __launch_bounds__(KD_BLOCK) void k_kd_keys(const float4 *node, const uint32_t *tag, int n, uint64_t *key,
-                                                     int *val, bool tag_only)
-{
-    int i = blockIdx.x*KD_BLOCK + threadIdx.x;
-    if (i >= n) return;
-    float4 p = node[i];
-    uint64_t t = tag[i];
-    key[i] = tag_only ? t : (t << 32) | ordered(coord(p, __float_as_int(p.w)));
-    val[i] = i;
-}
-
-__global__ __launch_bounds__(KD_BLOCK) void k_kd_gather(const uint64_t *key, const int *val, const float4 *node,
-                                                       const int *idx, int n, bool tag_only,
-                                                       const unsigned char *active, int n_phys, float4 *node_out,
-                                                       int *idx_out, uint32_t *tag_out)
-{
-    int i = blockIdx.x*KD_BLOCK + threadIdx.x;
-    if (i >= n) return;
-    int from = val[i];
-    float4 p = node[from];
-    const int r = idx[from];
-    if (tag_only && active[r % n_phys]) p.w = __int_as_float(__float_as_int(p.w) | KD_ACTIVE);
-    node_out[i] = p;
-    idx_out[i] = r;
-    tag_out[i] = tag_only ? uint32_t(key[i]) : uint32_t(key[i] >> 32);
-}
-
-// step L of the tag update: positions below the settled count are final; every other point moves
-// into its subtree's left or right child, or stays as the subtree's pivot (its node)
-__global__ __launch_bounds__(KD_BLOCK) void k_kd_update(float4 *node, uint32_t *tag, int n, int L,
-                                                       const float *world)
-{
-    int g = blockIdx.x*KD_BLOCK + threadIdx.x;
-    if (g >= n || g < full_nodes(L)) return;
-    int subtree = int(tag[g]);
-    kd_box b;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) { b.lo[d] = world[d]; b.hi[d] = world[3 + d]; }
-    for (int cur = subtree; cur > 0;)
+    kd_seg g;
+    for (int d = 0; d < 3; ++d)
     {
-        int parent = (cur + 1) / 2 - 1;
-        float4 pp = node[parent];
-        int d = __float_as_int(pp.w);
-        float split = coord(pp, d);
-        if (cur & 1) b.hi[d] = fminf(split, b.hi[d]);
-        else b.lo[d] = fmaxf(split, b.lo[d]);
-        cur = parent;
+        g.lo[d] = world_bits[d];
+        g.hi[d] = ~world_bits[3 + d];
+        world[d] = unordered(g.lo[d]);
+        world[3 + d] = unordered(g.hi[d]);
     }
-    int pivot = pivot_pos(L, n, subtree);
-    float4 pv = node[pivot];
-    int pd = __float_as_int(pv.w);
-    float pc = coord(pv, pd);
-    if (g < pivot) { subtree = 2*subtree + 1; b.hi[pd] = pc; }
-    else if (g > pivot) { subtree = 2*subtree + 2; b.lo[pd] = pc; }
-    if (g != pivot) node[g].w = __int_as_float(widest(b));
-    tag[g] = uint32_t(subtree);
+    g.start = 0;
+    g.size = n;
+    g.order = order_of(g.lo, g.hi, 63);
+    *seg = g;
+}
+
+// the bin that holds rank `rank` of `bins`, by the whole block
+template <int BLOCK>
+__device__ __forceinline__ kd_sel pick_bin(const unsigned int *bins, int rank)
+{
+    constexpr int PER = KD_BINS / BLOCK;
+    __shared__ int total[BLOCK / WAVE];
+    __shared__ kd_sel found;
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    int c[PER], sum = 0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) { c[k] = int(bins[threadIdx.x*PER + k]); sum += c[k]; }
+    int incl = sum;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1)
+    {
+        const int t = __shfl_up(incl, o, WAVE);
+        if (lane >= o) incl += t;
+    }
+    if (lane == WAVE - 1) total[wave] = incl;
+    __syncthreads();
+    int before = incl - sum;
+    for (int w = 0; w < wave; ++w) before += total[w];
+    if (rank >= before && rank < before + sum)
+    {
+        int k = 0;
+        while (rank >= before + c[k]) before += c[k++];
+        found.prefix = threadIdx.x*PER + k;
+        found.rank = rank - before;
+        found.count = c[k];
+    }
+    __syncthreads();
+    return found;
+}
+
+// the three digits of a key relative to its subtree's lower bound: the leading 11, the next 11 and the last 10
+// bits of the subtree's extent
+struct kd_digits
+{
+    int dim, s1, s2;
+    uint32_t lo;
+};
+
+__device__ __forceinline__ kd_digits digits_of(const kd_seg *g)
+{
+    kd_digits k;
+    k.dim = g->order & 3;
+    k.lo = g->lo[k.dim];
+    const int bits = 32 - __clz(static_cast<int>(g->hi[k.dim] - k.lo));
+    k.s1 = max(bits - 11, 0);
+    k.s2 = max(bits - 22, 0);
+    return k;
+}
+
+// One digit of the radix selection of every subtree's pivot. bins: [3][segs][KD_BINS], sel: [3][segs]; the blocks
+// of digit D each find digit D - 1's bin from its counts, which saves a launch between them. A level of 1e6 points
+// takes 6 launches and 37 us, against 300 us for the radix sort of (subtree, coordinate) keys: a selection needs
+// three reads of the points and one write, whatever the number of subtrees.
+template <int D>
+__global__ __launch_bounds__(KD_SPLIT_BLOCK) void k_kd_digit(const float4 *points, const kd_seg *seg, int segs,
+                                                            int chunks, unsigned int *bins, kd_sel *sel)
+{
+    __shared__ unsigned int count[KD_BINS];
+    const int s = blockIdx.x / chunks, chunk = blockIdx.x % chunks;
+    const int start = seg[s].start, size = seg[s].size;
+    if ((long long)chunk*KD_CHUNK >= size) return;
+    const kd_digits k = digits_of(seg + s);
+    uint32_t prefix = 0;
+    if constexpr (D > 0)
+    {
+        const kd_sel last = D == 1 ? kd_sel{0u, kd_left(size), 0} : sel[s];
+        kd_sel now = pick_bin<KD_SPLIT_BLOCK>(bins + ((long long)(D - 1)*segs + s)*KD_BINS, last.rank);
+        now.prefix |= D == 1 ? 0u : last.prefix << (k.s1 - k.s2);
+        prefix = now.prefix;
+        if (chunk == 0 && threadIdx.x == 0) sel[(D - 1)*segs + s] = now;
+    }
+    for (int b = threadIdx.x; b < KD_BINS; b += KD_SPLIT_BLOCK) count[b] = 0u;
+    __syncthreads();
+    const int begin = chunk*KD_CHUNK, end = min(begin + KD_CHUNK, size);
+    for (int i = begin + threadIdx.x; i < end; i += KD_SPLIT_BLOCK)
+    {
+        const uint32_t rel = ordered(coord(points[start + i], k.dim)) - k.lo;
+        if (D == 0) atomicAdd(count + (rel >> k.s1), 1u);
+        else if (D == 1 && rel >> k.s1 == prefix) atomicAdd(count + ((rel >> k.s2) & ((1u << (k.s1 - k.s2)) - 1u)), 1u);
+        else if (D == 2 && rel >> k.s2 == prefix) atomicAdd(count + (rel & ((1u << k.s2) - 1u)), 1u);
+    }
+    __syncthreads();
+    unsigned int *const to = bins + ((long long)D*segs + s)*KD_BINS;
+    for (int b = threadIdx.x; b < KD_BINS; b += KD_SPLIT_BLOCK)
+        if (count[b]) atomicAdd(to + b, count[b]);
+}
+
+// points below the pivot's coordinate to the front of their subtree's range, those that tie with it behind them,
+// the rest at the end, each part in any order; cursors: [segs][4]
+__global__ __launch_bounds__(KD_SPLIT_BLOCK) void k_kd_partition(const float4 *points, const kd_seg *seg, int segs,
+                                                                int chunks, const unsigned int *bins, kd_sel *sel,
+                                                                int *cursors, float4 *out)
+{
+    constexpr int PER = KD_CHUNK / KD_SPLIT_BLOCK, WAVES = KD_SPLIT_BLOCK / WAVE;
+    __shared__ int counts[WAVES][3], base[3];
+    const int s = blockIdx.x / chunks, chunk = blockIdx.x % chunks;
+    const int start = seg[s].start, size = seg[s].size;
+    if ((long long)chunk*KD_CHUNK >= size) return;
+    const kd_digits k = digits_of(seg + s);
+    const kd_sel last = sel[segs + s];
+    const kd_sel ties = pick_bin<KD_SPLIT_BLOCK>(bins + (2ll*segs + s)*KD_BINS, last.rank);
+    const uint32_t pivot = (last.prefix << k.s2) | ties.prefix;
+    if (chunk == 0 && threadIdx.x == 0) sel[2*segs + s] = ties;
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    const int begin = chunk*KD_CHUNK;
+    float4 p[PER];
+    int part[PER], mine[3] = {0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < PER; ++e)
+    {
+        const int i = begin + e*KD_SPLIT_BLOCK + int(threadIdx.x);
+        part[e] = 3;
+        if (i < size)
+        {
+            p[e] = points[start + i];
+            const uint32_t rel = ordered(coord(p[e], k.dim)) - k.lo;
+            part[e] = rel < pivot ? 0 : (rel == pivot ? 1 : 2);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) mine[c] += __popcll(__ballot(part[e] == c));
+    }
+    if (lane == 0)
+    {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) counts[wave][c] = mine[c];
+    }
+    __syncthreads();
+    if (threadIdx.x < 3)
+    {
+        int sum = 0;
+        for (int w = 0; w < WAVES; ++w) sum += counts[w][threadIdx.x];
+        base[threadIdx.x] = sum ? atomicAdd(cursors + 4*s + threadIdx.x, sum) : 0;
+    }
+    __syncthreads();
+    const int below = kd_left(size) - ties.rank;
+    int at[3] = {start + base[0], start + below + base[1], start + below + ties.count + base[2]};
+    for (int w = 0; w < wave; ++w)
+    {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) at[c] += counts[w][c];
+    }
+#pragma unroll
+    for (int e = 0; e < PER; ++e)
+    {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+        {
+            const unsigned long long m = __ballot(part[e] == c);
+            if (part[e] == c) out[at[c] + __popcll(m & ((1ull << lane) - 1ull))] = p[e];
+            at[c] += __popcll(m);
+        }
+    }
+}
+
+// Puts the points that tie with a pivot on their sides of it, settles the pivot and describes its children. One
+// block per subtree: usually the pivot is alone and nothing is left to order. Up to KD_TIES ties are ranked against
+// each other in LDS, more are selected by the digits of the further dimensions and of the index, through `spare`.
+__global__ __launch_bounds__(KD_TIES) void k_kd_settle(float4 *points, float4 *spare, const kd_seg *seg, int segs,
+                                                      const kd_sel *sel, kd_seg *children, float4 *node, int *idx)
+{
+    __shared__ float4 ties[KD_TIES];
+    __shared__ unsigned int count[KD_BINS];
+    __shared__ int side[2];
+    const int s = blockIdx.x;
+    const kd_seg g = seg[s];
+    const kd_sel tie = sel[2*segs + s];
+    const int left = kd_left(g.size), t = tie.count;
+    float4 *const first = points + g.start + (left - tie.rank);
+    if (t > 1 && t <= KD_TIES)
+    {
+        const int i = threadIdx.x;
+        if (i < t) ties[i] = first[i];
+        __syncthreads();
+        if (i < t)
+        {
+            const float4 p = ties[i];
+            int rank = 0;
+            for (int j = 0; j < t; ++j) rank += tie_less(ties[j], p, g.order) ? 1 : 0;
+            first[rank] = p;
+        }
+    }
+    else if (t > KD_TIES)
+    {
+        uint32_t found[3] = {0u, 0u, 0u};
+        int rank = tie.rank;
+        // key q of a point: the second and third dimension's coordinates, then the index
+        auto key = [&](const float4 &p, int q) {
+            const int d = q == 2 ? 3 : (g.order >> (2 + 2*q)) & 3;
+            if (q == 2) return __float_as_uint(p.w) & ~KD_SITE;
+            return d == 3 ? 0u : ordered(coord(p, d));
+        };
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+            for (int shift = 21, width = 11; shift >= 0; shift = shift == 21 ? 10 : shift - 10, width = shift ? 11 : 10)
+            {
+                for (int b = threadIdx.x; b < KD_BINS; b += KD_TIES) count[b] = 0u;
+                __syncthreads();
+                for (int i = threadIdx.x; i < t; i += KD_TIES)
+                {
+                    const float4 p = first[i];
+                    bool same = true;
+#pragma unroll
+                    for (int r = 0; r < q; ++r) same = same && key(p, r) == found[r];
+                    const uint32_t v = key(p, q);
+                    if (same && (shift == 21 || v >> (shift + width) == found[q]))
+                        atomicAdd(count + ((v >> shift) & ((1u << width) - 1u)), 1u);
+                }
+                __syncthreads();
+                const kd_sel now = pick_bin<KD_TIES>(count, rank);
+                found[q] = (found[q] << width) | now.prefix;
+                rank = now.rank;
+            }
+        if (threadIdx.x < 2) side[threadIdx.x] = 0;
+        __syncthreads();
+        float4 *const to = spare + g.start + (left - tie.rank);
+        for (int i = threadIdx.x; i < t; i += KD_TIES)
+        {
+            const float4 p = first[i];
+            int c = 0;      // -1 before the pivot, 1 behind it
+#pragma unroll
+            for (int q = 2; q >= 0; --q)
+            {
+                const uint32_t v = key(p, q);
+                if (v != found[q]) c = v < found[q] ? -1 : 1;
+            }
+            const int at = c == 0 ? tie.rank : (c < 0 ? atomicAdd(side, 1) : tie.rank + 1 + atomicAdd(side + 1, 1));
+            to[at] = p;
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < t; i += KD_TIES) first[i] = to[i];
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    const int dim = g.order & 3;
+    const float4 p = points[g.start + left];
+    put_node(p, dim, segs - 1 + s, node, idx);
+    kd_seg l = g, r = g;
+    const uint32_t cut = ordered(coord(p, dim));
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        if (d == dim) l.hi[d] = r.lo[d] = cut;
+    l.size = left;
+    r.size = g.size - 1 - left;
+    r.start = g.start + left + 1;
+    l.order = order_of(l.lo, l.hi, g.order);
+    r.order = order_of(r.lo, r.hi, g.order);
+    children[2*s] = l;
+    children[2*s + 1] = r;
+}
+
+// Every subtree of up to KD_SLOTS - 1 points, by one block in LDS. A subtree of r levels owns 2^r slots; they are
+// sorted (bitonically, all subtrees of a level at once), the pivot is written to its node and the two sides move
+// into the two halves of the slots. Strides of up to 64 stay within a wavefront's slots and need no barrier.
+// Bound by LDS latency: 364 compare steps for 12 levels, 229 us for 256 subtrees of 3900 points, one per CU; the
+// radix sorts of all points that it stands in for took 300 us for each of the 11 levels.
+__global__ __launch_bounds__(KD_FINISH_BLOCK) void k_kd_finish(const float4 *points, const kd_seg *seg, int segs,
+                                                              int levels, float4 *node, int *idx)
+{
+    constexpr uint32_t NONE = ~0u;
+    struct part { uint32_t lo[3], hi[3]; int order, size; };
+    __shared__ float4 pts[KD_SLOTS];
+    __shared__ uint64_t key[KD_SLOTS];                   // ordered coordinate << 32 | point
+    __shared__ uint32_t box[6][KD_SLOTS / 2];
+    __shared__ int info[KD_SLOTS / 2];                   // order | size << 6
+    const int t = threadIdx.x;
+    const kd_seg g = seg[blockIdx.x];
+    const int slots = 1 << levels;
+    for (int i = t; i < slots; i += KD_FINISH_BLOCK)
+    {
+        uint64_t k = ~0ull;
+        if (i < g.size)
+        {
+            const float4 p = points[g.start + i];
+            pts[i] = p;
+            k = (uint64_t(ordered(coord(p, g.order & 3))) << 32) | uint32_t(i);
+        }
+        key[i] = k;
+    }
+    if (t < 3) { box[t][0] = g.lo[t]; box[3 + t][0] = g.hi[t]; }
+    if (t == 0) info[0] = g.order | (g.size << 6);
+    __syncthreads();
+    for (int r = levels; r >= 1; --r)
+    {
+        const int span = 1 << r;
+        if (r > 1)
+            for (int k = 2; k <= span; k <<= 1)
+                for (int j = k >> 1; j > 0; j >>= 1)
+                {
+                    for (int p = t; p < slots / 2; p += KD_FINISH_BLOCK)
+                    {
+                        const int i = 2*p - (p & (j - 1));
+                        const bool up = (i & k) == 0 || k == span;
+                        const uint64_t a = key[i], b = key[i + j];
+                        bool less = b < a;
+                        if (uint32_t(a >> 32) == uint32_t(b >> 32) && uint32_t(a) != NONE && uint32_t(b) != NONE)
+                            less = tie_less(pts[uint32_t(b)], pts[uint32_t(a)], info[i >> r] & 63);
+                        if (less == up) { key[i] = b; key[i + j] = a; }
+                    }
+                    if (j > 64 || (j == 1 && k > 64)) __syncthreads();
+                    else
+                    {
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                    }
+                }
+        __syncthreads();
+        // settle the pivots; at r = 1 every subtree is one point and has no children
+        const int subtrees = slots >> r;
+        part l, h;
+        bool split = false;
+        for (int q = t; q < subtrees; q += KD_FINISH_BLOCK)
+        {
+            const int size = info[q] >> 6, order = info[q] & 63, dim = order & 3;
+            const int left = kd_left(size);
+            const float4 p = size ? pts[uint32_t(key[q*span + left])] : make_float4(0.f, 0.f, 0.f, 0.f);
+            if (size) put_node(p, dim, ((long long)(segs + blockIdx.x) << (levels - r)) - 1 + q, node, idx);
+            if (r == 1) continue;
+            split = true;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) { l.lo[d] = h.lo[d] = box[d][q]; l.hi[d] = h.hi[d] = box[3 + d][q]; }
+            const uint32_t cut = ordered(coord(p, dim));
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+                if (d == dim) l.hi[d] = h.lo[d] = cut;
+            l.size = left;
+            h.size = max(size - 1 - left, 0);
+            l.order = order_of(l.lo, l.hi, order);
+            h.order = order_of(h.lo, h.hi, order);
+        }
+        if (r == 1) break;
+        const int half = span >> 1;
+        uint32_t from[KD_SLOTS / KD_FINISH_BLOCK];
+#pragma unroll
+        for (int e = 0; e < KD_SLOTS / KD_FINISH_BLOCK; ++e)
+        {
+            const int i = t + e*KD_FINISH_BLOCK;
+            from[e] = NONE;
+            if (i >= slots) continue;
+            const int q = i >> r, pos = i & (half - 1), size = info[q] >> 6, left = kd_left(size);
+            const bool right = i & half;
+            if (pos < (right ? size - 1 - left : left)) from[e] = uint32_t(key[q*span + pos + (right ? left + 1 : 0)]);
+        }
+        __syncthreads();
+        if (split)
+        {
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+            {
+                box[d][2*t] = l.lo[d]; box[3 + d][2*t] = l.hi[d];
+                box[d][2*t + 1] = h.lo[d]; box[3 + d][2*t + 1] = h.hi[d];
+            }
+            info[2*t] = l.order | (l.size << 6);
+            info[2*t + 1] = h.order | (h.size << 6);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < KD_SLOTS / KD_FINISH_BLOCK; ++e)
+        {
+            const int i = t + e*KD_FINISH_BLOCK;
+            if (i >= slots) continue;
+            uint64_t k = ~0ull;
+            if (from[e] != NONE)
+                k = (uint64_t(ordered(coord(pts[from[e]], info[i >> (r - 1)] & 3))) << 32) | from[e];
+            key[i] = k;
+        }
+        __syncthreads();
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -524,51 +876,43 @@ void kd_build(context &c)
     t.node.alloc(n);
     t.idx.alloc(n);
     t.world.alloc(6);
-    dbuf<float4> node_b;
-    dbuf<int> idx_b;
-    dbuf<uint32_t> tag, tag_b;
-    dbuf<uint64_t> key;
-    dbuf<int> val;
-    dbuf<unsigned int> wbits;
-    dbuf<int> dim0;
-    node_b.alloc(n);
-    idx_b.alloc(n);
-    tag.alloc(n);
-    tag_b.alloc(n);
-    key.alloc(n);
-    val.alloc(n);
-    wbits.alloc(6);
-    dim0.alloc(1);
-    const unsigned int init[6] = {~0u, ~0u, ~0u, 0u, 0u, 0u};
-    hip_check(hipMemcpyAsync(wbits.p, init, sizeof(init), hipMemcpyHostToDevice, st), "k-d world init");
-    hip_check(hipMemsetAsync(tag.p, 0, sizeof(uint32_t)*n, st), "k-d tags");
-    k_kd_init<<<blocks(n, KD_BLOCK), KD_BLOCK, 0, st>>>(src, n, t.node.p, t.idx.p, wbits.p);
-    k_kd_world<<<1, 64, 0, st>>>(wbits.p, t.world.p, dim0.p);
-    k_kd_dim0<<<blocks(n, KD_BLOCK), KD_BLOCK, 0, st>>>(t.node.p, n, dim0.p);
-    hip_check(hipGetLastError(), "launch k-d init");
     int levels = 0;
     while ((1ll << levels) - 1 < n) ++levels;      // levels of a left-balanced tree of n nodes
-    const int deepest = levels - 1;
-    auto sort_level = [&](int L, bool tag_only) {
-        k_kd_keys<<<blocks(n, KD_BLOCK), KD_BLOCK, 0, st>>>(t.node.p, tag.p, n, key.p, val.p, tag_only);
-        // tags of step L are below 2^(L+1); the final pass sorts tags of up to `levels` bits
-        int tag_bits = tag_only ? levels : L + 1;
-        radix_sort_pairs(key.p, val.p, n, 0, (tag_only ? 0 : 32) + tag_bits, c.scratch, st);
-        k_kd_gather<<<blocks(n, KD_BLOCK), KD_BLOCK, 0, st>>>(key.p, val.p, t.node.p, t.idx.p, n, tag_only,
-                                                             c.active.p, c.n, node_b.p, idx_b.p, tag_b.p);
-        hip_check(hipGetLastError(), "launch k-d sort");
-        swap_buf(t.node, node_b);
-        swap_buf(t.idx, idx_b);
-        swap_buf(tag, tag_b);
-    };
-    for (int L = 0; L < deepest; ++L)
+    const int top = std::max(0, levels - KD_LDS_LEVELS);
+    const size_t seg_words = (size_t(1) << top)*(sizeof(kd_seg) / sizeof(unsigned int));
+    const size_t most = size_t(1) << std::max(0, top - 1);      // subtrees of the last level that is split
+    t.points[0].alloc(n);
+    t.points[1].alloc(top ? n : 0);
+    t.segments.alloc(2*seg_words);
+    t.counts.alloc(most*(3*KD_BINS + 4 + 3*sizeof(kd_sel) / sizeof(unsigned int)) + 6);
+    unsigned int *const wbits = t.counts.p;
+    hip_check(hipMemsetAsync(wbits, 0xff, 6*sizeof(unsigned int), st), "k-d world init");
+    kd_seg *seg = reinterpret_cast<kd_seg *>(t.segments.p), *next = reinterpret_cast<kd_seg *>(t.segments.p + seg_words);
+    k_kd_init<<<std::min(KD_INIT_BLOCKS, blocks(n, KD_BLOCK)), KD_BLOCK, 0, st>>>(src, c.active.p, n, c.n,
+                                                                                t.points[0].p, wbits);
+    k_kd_root<<<1, 64, 0, st>>>(wbits, n, t.world.p, seg);
+    hip_check(hipGetLastError(), "launch k-d init");
+    float4 *points = t.points[0].p, *other = t.points[1].p;
+    int largest = n;
+    for (int L = 0; L < top; ++L)
     {
-        sort_level(L, false);
-        k_kd_update<<<blocks(n, KD_BLOCK), KD_BLOCK, 0, st>>>(t.node.p, tag.p, n, L, t.world.p);
-        hip_check(hipGetLastError(), "launch k-d update");
+        const int segs = 1 << L, chunks = blocks(largest, KD_CHUNK);
+        unsigned int *const bins = t.counts.p + 6;
+        int *const cursors = reinterpret_cast<int *>(bins + size_t(segs)*3*KD_BINS);
+        kd_sel *const sel = reinterpret_cast<kd_sel *>(cursors + size_t(segs)*4);
+        hip_check(hipMemsetAsync(bins, 0, sizeof(unsigned int)*size_t(segs)*(3*KD_BINS + 4), st), "k-d counts");
+        k_kd_digit<0><<<segs*chunks, KD_SPLIT_BLOCK, 0, st>>>(points, seg, segs, chunks, bins, sel);
+        k_kd_digit<1><<<segs*chunks, KD_SPLIT_BLOCK, 0, st>>>(points, seg, segs, chunks, bins, sel);
+        k_kd_digit<2><<<segs*chunks, KD_SPLIT_BLOCK, 0, st>>>(points, seg, segs, chunks, bins, sel);
+        k_kd_partition<<<segs*chunks, KD_SPLIT_BLOCK, 0, st>>>(points, seg, segs, chunks, bins, sel, cursors, other);
+        k_kd_settle<<<segs, KD_TIES, 0, st>>>(other, points, seg, segs, sel, next, t.node.p, t.idx.p);
+        hip_check(hipGetLastError(), "launch k-d split");
+        std::swap(points, other);
+        std::swap(seg, next);
+        largest = kd_left(largest);
     }
-    sort_level(deepest, true);
-    hip_check(hipStreamSynchronize(st), "k-d build");
+    k_kd_finish<<<1 << top, KD_FINISH_BLOCK, 0, st>>>(points, seg, 1 << top, levels - top, t.node.p, t.idx.p);
+    hip_check(hipGetLastError(), "launch k-d finish");
 }
 
 void kd_query(context &c)

@@ -294,6 +294,8 @@ struct context
     dbuf<float4> pts;          // {x, y, z, search cap}
     dbuf<unsigned char> active;
     dbuf<unsigned char> group;
+    dbuf<unsigned char> bin;       // group, with the bit above it set where the particle is inactive
+    dbuf<unsigned int> slot_totals;   // particles per bin
     dbuf<int> bad;             // first non-finite particle + 1
     morton_index index;
     kd_tree kd;
@@ -379,7 +381,6 @@ struct context
 // the reverse neighbour lists of a swarm with a majorant address n_active * N_K entries with 32-bit offsets
 constexpr long long MAJORANT_MAX_OWNERS = 4294967295LL / N_K;
 void scan_exclusive_u32(const unsigned int *in, unsigned int *out, int n, sort_scratch &s, hipStream_t st);
-void radix_sort_pairs(uint64_t *keys, int *vals, int n, int begin_bit, int end_bit, sort_scratch &s, hipStream_t st);
 void morton_build(morton_index &ix, const float4 *points, const unsigned char *active, int n, float ox, float oy,
                   float oz, float width, int dim, int leaf_target, int max_level, sort_scratch &s, hipStream_t st,
                   const int *codes = nullptr);

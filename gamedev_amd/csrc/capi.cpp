@@ -1716,6 +1716,11 @@ int gdx_morton_build(const void *points4, const unsigned char *active, int n, fl
         m = new gdx_morton_ctx();
         morton_build(m->ix, static_cast<const float4 *>(points4), active, n, ox, oy, oz, width, dim, leaf_target,
                      max_level, m->scratch, nullptr);
+        unsigned int nodes = 0;
+        copy_d2h(&nodes, morton_total(m->ix), sizeof(nodes), nullptr);
+        hip_check(hipStreamSynchronize(nullptr), "complete Morton hierarchy");
+        morton_settle(m->ix, nodes, nullptr);
+        hip_check(hipStreamSynchronize(nullptr), "complete Morton hierarchy");
         m->overflow.alloc(1);
     });
     if (rc != GDX_COL_OK) { delete m; return rc; }

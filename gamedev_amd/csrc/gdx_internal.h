@@ -267,10 +267,22 @@ struct morton_index
     dbuf<int> idx;             // sorted record -> source index
     dbuf<float4> rec;          // sorted records {x, y, z, code}; code sign bit marks inactive
     dbuf<gdx_node> nodes;
+    dbuf<unsigned int> counts; // nodes begun per level and 256 records, scanned; then the nodes below the root
+    dbuf<unsigned int> masks;  // per node: the child codes that it has
     dbuf<gdx_box> boxes;       // per node: the box and children the search reads
     dbuf<gdx_box> chunks;      // per eight sorted records: the box of the active ones
     int node_count = 0;
     int leaf_count = 0;
+};
+
+// what the host reads of a geometry epoch
+constexpr int SLOT_BINS = 128;
+struct epoch_results
+{
+    int bad;
+    unsigned int nodes;
+    unsigned int bins[SLOT_BINS];
+    unsigned long long graph[LOCAL_GROUPS + 1];
 };
 
 struct context
@@ -297,13 +309,13 @@ struct context
     dbuf<unsigned char> bin;       // group, with the bit above it set where the particle is inactive
     dbuf<unsigned int> slot_totals;   // particles per bin
     dbuf<int> bad;             // first non-finite particle + 1
+    pinned<epoch_results> epoch_host;
     morton_index index;
     kd_tree kd;
     sort_scratch scratch;
     dbuf<int> pidx_slot;       // particle -> slot (-1 inactive)
     dbuf<int> slot_pidx;       // slot -> particle
     dbuf<unsigned long long> graph;   // per group: 64-bit dependency mask
-    dbuf<unsigned int> overflow;
     // azimuthal wedge: physical records then seam ghosts, their codes 3*i + image, ghost counts and offsets
     dbuf<float4> wedge_rec;
     dbuf<int> wedge_code;
@@ -388,6 +400,9 @@ void geometry_epoch(context &c);
 void load_state(context &c);
 void store_state(context &c);
 // test access: exact top-K over a built index for arbitrary queries and a runtime K
+void write_nodes(morton_index &ix, hipStream_t st);
+const unsigned int *morton_total(const morton_index &ix);
+void morton_settle(morton_index &ix, unsigned int total, hipStream_t st);
 void knn_query(const morton_index &ix, const float4 *queries, int nq, int k, int *codes, float *d2,
                unsigned int *overflow, hipStream_t st);
 

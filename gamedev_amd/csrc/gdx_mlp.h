@@ -41,6 +41,14 @@ struct pack
 
 // round to nearest even (finite inputs): the hardware conversion (v_cvt_pk_bf16_f32)
 __device__ __forceinline__ short bf16_rn(float f) { return __builtin_bit_cast(short, static_cast<__bf16>(f)); }
+// four at once, two to a conversion (one by one the compiler converts each alone and packs the halves)
+__device__ __forceinline__ v4s bf16_rn4(v4f f)
+{
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    struct { b2 lo, hi; } r{__builtin_convertvector(f2{f[0], f[1]}, b2), __builtin_convertvector(f2{f[2], f[3]}, b2)};
+    return __builtin_bit_cast(v4s, r);
+}
 __device__ __forceinline__ float bf16_f(short b) { return __uint_as_float(static_cast<unsigned int>(static_cast<unsigned short>(b)) << 16); }
 
 // the hardware exponential and reciprocal (about 1 ulp each): far below the BF16 rounding that
@@ -66,8 +74,10 @@ __device__ __forceinline__ v4s input_fragment(const pack *P, const float *x, boo
     v4s r = {0, 0, 0, 0};
     if (valid && g < F/4)
     {
+        v4f u;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) r[v] = bf16_rn((x[4*g + v] - P->mu[4*g + v])*P->inv_sigma[4*g + v]);
+        for (int v = 0; v < 4; ++v) u[v] = (x[4*g + v] - P->mu[4*g + v])*P->inv_sigma[4*g + v];
+        r = bf16_rn4(u);
     }
     return r;
 }
@@ -90,10 +100,10 @@ __device__ __forceinline__ float tile_forward(const pack *P, v4s x, forward_stat
         for (int v = 0; v < 4; ++v) acc[v] = P->b1[16*c + 4*g + v];
         acc = mfma(P->w1a[c][lane], x, acc);
         f.a1[c] = acc;
-        v4s h;
+        v4f h;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) h[v] = bf16_rn(silu(acc[v]));
-        f.h1[c] = h;
+        for (int v = 0; v < 4; ++v) h[v] = silu(acc[v]);
+        f.h1[c] = bf16_rn4(h);
     }
     float part = 0.0f;
 #pragma unroll

@@ -835,7 +835,6 @@ __device__ double owner_features(const gdx_gref &G, int s, float *f)
 __global__ __launch_bounds__(BLOCK) void k_majorant(gdx_wave w)
 {
     __shared__ float feat[BLOCK][mlp::F + 1];
-    __shared__ float ys[BLOCK];
     __shared__ int list[MAJ_SLOTS];
     __shared__ int wave_tot[WAVES];
     int gi, s0, s1;
@@ -890,20 +889,19 @@ __global__ __launch_bounds__(BLOCK) void k_majorant(gdx_wave w)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        // every lane keeps the output of its own row: one softplus for the four tiles
+        float z = 0.0f;
 #pragma unroll
         for (int tt = 0; tt < WAVE / 16; ++tt)
         {
             const int row = wv*WAVE + tt*16 + (lane & 15);
             mlp::forward_state fs;
-            float z = mlp::tile_forward(P, mlp::input_fragment(P, &feat[row][0], true), fs);
-            if (lane < 16) ys[row] = mlp::softplus(z);
+            const float v = mlp::tile_forward(P, mlp::input_fragment(P, &feat[row][0], true), fs);
+            z = lane / 16 == tt ? v : z;
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (has)
         {
-            G.lam[so] = S*static_cast<double>(ys[threadIdx.x]);
+            G.lam[so] = S*static_cast<double>(mlp::softplus(z));
             G.lam_add[so] = 0.0;
             if (G.stale) G.stale[so] = 0;
         }

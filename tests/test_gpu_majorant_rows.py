@@ -1,0 +1,46 @@
+"""The majorant's kernels at the row counts where they split their work differently: inference tiles of 16 rows,
+steps of four tiles from 65536 rows on, the last one ragged; gradient rows of eight tiles and their last tile.
+Compared with the CPU oracle, with the bounds of the other majorant tests: FP32 accumulation order inside the
+matrix cores and rare BF16 flips of a hidden value."""
+import numpy as np
+import pytest
+
+from oracle import majorant as M
+from test_gpu_majorant import dev, rand_data, rand_params
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 64, 65, 65535, 65536, 65537, 70001])
+def test_inference_rows(gpu, n):
+    from gamedev_amd import Majorant
+    print(f"[majorant] inference n={n}", flush=True)
+    X, _, norm = rand_data(n, n)
+    p = rand_params(n)
+    m = Majorant("fiducial_3d", seed=1)
+    m.set_params(p, norm)
+    x = dev(X, gpu)
+    y = m.infer(x).cpu().numpy()
+    yo = M.predict(p, norm, X)
+    rel = np.abs(y - yo)/yo
+    assert np.median(rel) < 2e-5 and rel.max() < 5e-3, (np.median(rel), rel.max())
+    # a row's output depends on its own inputs alone: the same bits in a block of another size
+    k = min(n, 200)
+    assert np.array_equal(m.infer(x[n - k:].contiguous()).cpu().numpy(), y[n - k:])
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 127, 128, 129, 1025])
+def test_gradient_rows(gpu, n):
+    from gamedev_amd import Majorant
+    print(f"[majorant] gradient n={n}", flush=True)
+    X, lt, norm = rand_data(100 + n, n)
+    p = rand_params(7)
+    m = Majorant("fiducial_3d", seed=1)
+    m.set_params(p, norm)
+    g, loss = m.grad(dev(X, gpu), dev(lt, gpu))
+    go, lo = M.loss_grad(p, norm, X, lt)
+    assert abs(loss - lo) <= 1e-4*abs(lo) + 1e-6
+    # one flip of a hidden value's last BF16 bit (2^-8) moves a sample's gradient by that share of it
+    scale = np.abs(go).max()
+    assert np.abs(g - go).max() <= max(2e-3, 2**-8/n)*scale + 1e-7
+    assert float(np.dot(g, go)/np.linalg.norm(g)/np.linalg.norm(go)) > 0.9999

@@ -1676,21 +1676,64 @@ void invalidate_bounds(context &c)
     c.model_version = majorant_version(c.model);
 }
 
-// reverse neighbour lists of the geometry epoch: for every slot j the owners whose rows hold j
-__global__ __launch_bounds__(256) void k_rev_count(const int *nbr, long long entries, unsigned *count)
+// reverse neighbour lists of the geometry epoch: for every slot j the owners whose rows hold j, in any order.
+// Bound by the atomics on the slots' counts and cursors, and by the scattered writes. A block's consecutive owners
+// are close in space and share most of their neighbours, so it first counts its entries per slot in a hash table
+// in LDS and then takes each slot's places by one global atomic: some 10,000 for 131,072 entries. An entry whose
+// slot finds no room in the table takes its place by itself. 1e7 owners of 32 neighbours: counts 4.6 -> 1.5 ms,
+// lists 7.4 -> 3.8 ms.
+constexpr int REV_BLOCK = 1024;
+constexpr int REV_SLOTS = 16384, REV_PROBES = 16;
+constexpr int REV_OWNERS = 4096, REV_OWNERS_SMALL = 1024;      // per block; the smaller below one block per CU
+
+// the table place of slot j, entering it if it is new; -1: no room within the probes
+__device__ __forceinline__ int rev_place(unsigned *keys, unsigned j)
 {
-    const long long i = (long long)blockIdx.x*blockDim.x + threadIdx.x;
-    if (i >= entries) return;
-    const int j = nbr[i];
-    if (j >= 0) atomicAdd(&count[j], 1u);
+    const unsigned h = (j*2654435761u) >> 18;
+    static_assert(REV_SLOTS == 1 << 14, "the hash keeps 14 bits");
+    for (int p = 0; p < REV_PROBES; ++p)
+    {
+        const unsigned at = (h + p) & (REV_SLOTS - 1);
+        unsigned k = keys[at];
+        if (k == 0u) k = atomicCAS(keys + at, 0u, j + 1u);
+        if (k == 0u || k == j + 1u) return int(at);
+    }
+    return -1;
 }
 
-__global__ __launch_bounds__(256) void k_rev_fill(const int *nbr, long long entries, unsigned *cursor, int *rev)
+template <bool FILL>
+__global__ __launch_bounds__(REV_BLOCK) void k_reverse(const int *nbr, int n, int owners, unsigned *cursor, int *rev)
 {
-    const long long i = (long long)blockIdx.x*blockDim.x + threadIdx.x;
-    if (i >= entries) return;
-    const int j = nbr[i];
-    if (j >= 0) rev[atomicAdd(&cursor[j], 1u)] = int(i / N_K);
+    __shared__ unsigned keys[REV_SLOTS], count[REV_SLOTS];
+    for (int i = threadIdx.x; i < REV_SLOTS; i += REV_BLOCK) keys[i] = count[i] = 0u;
+    __syncthreads();
+    const long long first = (long long)blockIdx.x*owners;
+    const int entries = int(min((long long)owners, n - first))*N_K;
+    const int *const row = nbr + first*N_K;
+    for (int i = threadIdx.x; i < entries; i += REV_BLOCK)
+    {
+        const int j = row[i];
+        if (j < 0) continue;
+        const int at = rev_place(keys, unsigned(j));
+        if (at >= 0) atomicAdd(count + at, 1u);
+        else if (!FILL) atomicAdd(cursor + j, 1u);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < REV_SLOTS; i += REV_BLOCK)
+        if (count[i])
+        {
+            const unsigned from = atomicAdd(cursor + (keys[i] - 1u), count[i]);
+            if (FILL) count[i] = from;
+        }
+    if (!FILL) return;
+    __syncthreads();
+    for (int i = threadIdx.x; i < entries; i += REV_BLOCK)
+    {
+        const int j = row[i];
+        if (j < 0) continue;
+        const int at = rev_place(keys, unsigned(j));      // every slot with room is in the table by now
+        rev[atomicAdd(at >= 0 ? count + at : cursor + j, 1u)] = int(first) + i / N_K;
+    }
 }
 
 void build_reverse(context &c)
@@ -1706,16 +1749,15 @@ void build_reverse(context &c)
     c.rev.alloc(na*N_K);
     if (n > 0)
     {
-        const long long entries = (long long)n*N_K;
-        const unsigned blocks = unsigned((entries + 255) / 256);
+        const int owners = n >= 256*REV_OWNERS ? REV_OWNERS : REV_OWNERS_SMALL, blocks = blocks_for(n, owners);
         hip_check(hipMemsetAsync(c.rev_end.p, 0, sizeof(unsigned)*na, st), "zero reverse counts");
-        k_rev_count<<<blocks, 256, 0, st>>>(c.nbr.p, entries, c.rev_end.p);
+        k_reverse<false><<<blocks, REV_BLOCK, 0, st>>>(c.nbr.p, n, owners, c.rev_end.p, nullptr);
         hip_check(hipGetLastError(), "launch reverse count");
         scan_exclusive_u32(c.rev_end.p, c.rev_beg.p, n, c.scratch, st);
         hip_check(hipMemcpyAsync(c.rev_end.p, c.rev_beg.p, sizeof(unsigned)*na, hipMemcpyDeviceToDevice, st),
                   "reverse cursors");
         // after the fill each cursor is the end of its slot's list
-        k_rev_fill<<<blocks, 256, 0, st>>>(c.nbr.p, entries, c.rev_end.p, c.rev.p);
+        k_reverse<true><<<blocks, REV_BLOCK, 0, st>>>(c.nbr.p, n, owners, c.rev_end.p, c.rev.p);
         hip_check(hipGetLastError(), "launch reverse fill");
     }
     c.rev_valid = true;

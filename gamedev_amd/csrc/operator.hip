@@ -602,13 +602,26 @@ __device__ __forceinline__ rate_sums group_rate_sums(const gdx_gref *GP, int s, 
 constexpr int RATE_LANES = 4;
 static_assert(BLOCK / RATE_LANES == RATE_SUB_OWNERS, "host block starts of the lane-group launch");
 
+// A block's bins in LDS, BIN_COPIES times over: the lanes of a wavefront mostly share a bin or two, and atomics on
+// one address run one after the other. Lane l adds to copy l mod BIN_COPIES, whose size is an odd number of doubles,
+// so that the copies of one field lie in different banks; the flush adds the copies up. Sixteen copies leave at most
+// four lanes on an address, for 14 KB a block. 64 realizations of 65536
+// owners: the screens of a step 5.6 -> 2.8 ms (one at a time).
+constexpr int BIN_COPIES = 16;
+
+struct rate_lds
+{
+    double d[COL_BIN_S][4];    // mass, weighted rate, change, second
+    int cnt[COL_BIN_S][2];     // owners, invalid ones
+    double pad;
+};
+
 template <int LANES>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void k_bath_rate(gdx_wave w)
 {
     constexpr bool GROUPED = LANES > 1;
     constexpr int OWNERS = BLOCK / LANES;
-    __shared__ double accd[COL_BIN_S][4];     // mass, weighted rate, change, second
-    __shared__ int acci[COL_BIN_S][3];        // count, owner count, invalid count
+    __shared__ rate_lds acc[BIN_COPIES];
     // blocks cover the group's rated owners (every owner, or a learned swarm's subsample)
     const int b = xcd_block();
     if (b >= w.bstart[w.n]) return;
@@ -632,8 +645,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void
     const double *measure = GP->measure;
     // the exact subsample of a learned swarm checks the bound of the same bath: block totals
     __shared__ unsigned checked[2];
-    if (threadIdx.x < COL_BIN_S*4) (&accd[0][0])[threadIdx.x] = 0.0;
-    if (threadIdx.x < COL_BIN_S*3) (&acci[0][0])[threadIdx.x] = 0;
+    for (int i = threadIdx.x; i < int(sizeof(acc) / sizeof(double)); i += BLOCK) reinterpret_cast<double *>(acc)[i] = 0.0;
     if (threadIdx.x < 2) checked[threadIdx.x] = 0u;
     __syncthreads();
     const int s = w.beg[gi] + (sub < 0 ? i : ((i / THIN_RUN)*GP->thin_stride + sub)*THIN_RUN + i % THIN_RUN);
@@ -681,18 +693,18 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void
         const double weight = me.y*grain_mass(me.x);
         const bool bad = !isfinite(weight) || !(weight > 0.0) || !isfinite(R) || R < 0.0 || !isfinite(J1)
             || J1 < 0.0 || !isfinite(J2) || J2 < 0.0;
-        atomicAdd(&acci[sb][0], 1);
-        atomicAdd(&acci[sb][1], 1);
+        rate_lds &bin = acc[lane % BIN_COPIES];
+        atomicAdd(&bin.cnt[sb][0], 1);
         if (bad)
         {
-            atomicAdd(&acci[sb][2], 1);
+            atomicAdd(&bin.cnt[sb][1], 1);
         }
         else
         {
-            atomicAdd(&accd[sb][0], weight);
-            atomicAdd(&accd[sb][1], weight*R);
-            atomicAdd(&accd[sb][2], weight*J1);
-            atomicAdd(&accd[sb][3], weight*J2);
+            atomicAdd(&bin.d[sb][0], weight);
+            atomicAdd(&bin.d[sb][1], weight*R);
+            atomicAdd(&bin.d[sb][2], weight*J1);
+            atomicAdd(&bin.d[sb][3], weight*J2);
         }
     }
     __syncthreads();
@@ -712,13 +724,18 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void
     if (threadIdx.x < COL_BIN_S*4)
     {
         int b = threadIdx.x / 4, f = threadIdx.x % 4;
-        double v = accd[b][f];
+        double v = 0.0;
+#pragma unroll
+        for (int c = 0; c < BIN_COPIES; ++c) v += acc[c].d[b][f];
         if (v != 0.0) atomicAdd(&(&G.raw_rate[b].mass)[f], v);
     }
     else if (threadIdx.x >= 64 && threadIdx.x < 64 + COL_BIN_S*3)
     {
+        // count, owner count, invalid count: every rated owner counts in the first two
         int b = (threadIdx.x - 64) / 3, f = (threadIdx.x - 64) % 3;
-        int v = acci[b][f];
+        int v = 0;
+#pragma unroll
+        for (int c = 0; c < BIN_COPIES; ++c) v += acc[c].cnt[b][f / 2];
         if (v != 0) atomicAdd(&(&G.raw_rate[b].count)[f], v);
     }
 }
@@ -931,37 +948,50 @@ struct audit_lds
     double d[COL_BIN_S][11];   // mass, pf, pe, pvf, pve, pg, pvg, touched, event_weight, growth, end_mass
     unsigned long long mx[COL_BIN_S][2];
     int cnt[COL_BIN_S][2];     // owner_count, invalid_count
+    double pad;
 };
+static_assert(sizeof(audit_lds) / sizeof(double) % 2 == 1, "the copies lie in different banks");
 
-__device__ __forceinline__ void clear_audit(audit_lds &a)
+__device__ __forceinline__ void clear_audit(audit_lds (&a)[BIN_COPIES])
 {
-    for (int i = threadIdx.x; i < COL_BIN_S*11; i += BLOCK) (&a.d[0][0])[i] = 0.0;
-    if (threadIdx.x < COL_BIN_S*2) { (&a.mx[0][0])[threadIdx.x] = 0ull; (&a.cnt[0][0])[threadIdx.x] = 0; }
+    double *const p = reinterpret_cast<double *>(a);
+    for (int i = threadIdx.x; i < int(sizeof(a) / sizeof(double)); i += BLOCK) p[i] = 0.0;
 }
 
-__device__ __forceinline__ void flush_audit(const audit_lds &a, gdx_raw_audit *dst)
+__device__ __forceinline__ void flush_audit(const audit_lds (&a)[BIN_COPIES], gdx_raw_audit *dst)
 {
     for (int i = threadIdx.x; i < COL_BIN_S*11; i += BLOCK)
     {
         int b = i / 11, f = i % 11;
-        double v = a.d[b][f];
+        double v = 0.0;
+#pragma unroll
+        for (int c = 0; c < BIN_COPIES; ++c) v += a[c].d[b][f];
         if (v == 0.0) continue;
         double *base = (f < 7) ? &dst[b].mass + f : &dst[b].touched + (f - 7);
         atomicAdd(base, v);
     }
-    if (threadIdx.x < COL_BIN_S*2)
+    // the last wavefront takes the maxima and counts, beside the sums
+    const int t = int(threadIdx.x) - (BLOCK - WAVE);
+    static_assert(COL_BIN_S*2 <= WAVE, "a wavefront holds every maximum and count");
+    if (t >= 0 && t < COL_BIN_S*2)
     {
-        int b = threadIdx.x / 2, f = threadIdx.x % 2;
-        unsigned long long v = a.mx[b][f];
+        int b = t / 2, f = t % 2;
+        unsigned long long v = 0ull;
+        int cnt = 0;
+#pragma unroll
+        for (int c = 0; c < BIN_COPIES; ++c)
+        {
+            v = max(v, a[c].mx[b][f]);
+            cnt += a[c].cnt[b][f];
+        }
         if (v) atomicMax(f == 0 ? &dst[b].maximum_weight_bits : &dst[b].maximum_g_jump_bits, v);
-        int cnt = a.cnt[b][f];
         if (cnt) atomicAdd(f == 0 ? &dst[b].owner_count : &dst[b].invalid_count, cnt);
     }
 }
 
 // audit terms of one owner per lane (col_audit_bin.cu:31-59): every field but the end mass goes to the
-// start bin bs, the end mass to the end bin be. Each lane adds its terms to the block's LDS bins with
-// native FP64 LDS atomics (lanes of one bin meet on one address and the LDS serialises them). Without
+// start bin bs, the end mass to the end bin be. Each lane adds its terms to its copy of the block's LDS
+// bins with native FP64 LDS atomics. Without
 // events (EVENTS false) the end bin is the start bin and the event fields are zero.
 template <bool EVENTS>
 __device__ __forceinline__ void audit_wave(audit_lds &a, bool take, int bs, int be, double weight,
@@ -1013,7 +1043,7 @@ static_assert(SCREEN_OWNERS == PUBLISH_OWNERS, "the screen and the publish share
 template <int ROUNDS>
 __global__ __launch_bounds__(BLOCK) void k_screen(gdx_wave w)
 {
-    __shared__ audit_lds a;
+    __shared__ audit_lds a[BIN_COPIES];
     __shared__ int block_tot[3], block_base[3];
     int gi, s0, s1;
     if (!due_block(w, BLOCK*ROUNDS, gi, s0, s1)) return;
@@ -1149,7 +1179,7 @@ __global__ __launch_bounds__(BLOCK) void k_screen(gdx_wave w)
             const bool bad = !isfinite(weight) || !(weight > 0.0) || !isfinite(probability) || !isfinite(hazard)
                 || hazard < 0.0 || !isfinite(j1) || j1 < 0.0 || !isfinite(j2) || j2 < 0.0 || !isfinite(jmax)
                 || jmax < 0.0 || !isfinite(old.x) || !(old.x > 0.0);
-            audit_wave<false>(a, true, bs, bs, weight, probability, hazard, j1, j2, jmax, 0.0, 0.0, bad);
+            audit_wave<false>(a[lane % BIN_COPIES], true, bs, bs, weight, probability, hazard, j1, j2, jmax, 0.0, 0.0, bad);
         }
         // owners with an event join the group's queue (heavy ones from the region's start, the others
         // from its end) and thinning candidates its candidate list: offsets within the block's share
@@ -2447,7 +2477,7 @@ static_assert(BLOCK*AUDIT_ROUNDS == PUBLISH_OWNERS, "the audit uses the 1024-own
 
 __global__ __launch_bounds__(BLOCK) void k_chain_audit(gdx_wave w, gdx_chain_log clog)
 {
-    __shared__ audit_lds a;
+    __shared__ audit_lds a[BIN_COPIES];
     int gi, s0, s1;
     if (!due_block(w, BLOCK*AUDIT_ROUNDS, gi, s0, s1)) return;
     const gdx_gref &G = w.table[w.ref[gi]];
@@ -2510,7 +2540,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_audit(gdx_wave w, gdx_chain_log
                 || sum.x < 0.0 || !isfinite(ev) || !isfinite(sum.y) || sum.y < 0.0 || !isfinite(sum.z)
                 || sum.z < 0.0 || !isfinite(sum.w) || sum.w < 0.0 || !isfinite(size_end) || !(size_end > 0.0);
             const double growth = fabs(log(size_end / old.x));
-            audit_wave<true>(a, true, bs, be, weight, probability, sum.x, sum.y, sum.z, sum.w, ev, growth, bad);
+            audit_wave<true>(a[threadIdx.x % BIN_COPIES], true, bs, be, weight, probability, sum.x, sum.y, sum.z, sum.w, ev, growth, bad);
         }
     }
     __syncthreads();

@@ -422,7 +422,7 @@ struct rate_sums
 // chunks (optional): the rate partial of every four consecutive row positions, (t0 + t1) + (t2 + t3)
 template <bool MOMENTS = true>
 __device__ __forceinline__ rate_sums owner_rate_sums(const gdx_gref *GP, int s, bool own, double2 me, double m,
-                                                     double *cat3, double *chunks = nullptr)
+                                                     double *cat3, const log_entry *logs, double *chunks = nullptr)
 {
     const int *nbr = GP->nbr;
     const double2 *res = GP->res;
@@ -442,7 +442,7 @@ __device__ __forceinline__ rate_sums owner_rate_sums(const gdx_gref *GP, int s, 
         cat3[1] = c.second;
         cat3[2] = c.maximum;
     }
-    const cat_moments_lds cm{cat3};
+    const cat_moments_lds cm{cat3, logs};
     auto eval = [&](const partner &q) {
         if constexpr (MOMENTS) return eval_pair_terms(t, cm, q, lambda_0);
         else return eval_pair_rate(t, q, lambda_0);
@@ -504,7 +504,7 @@ __device__ __forceinline__ rate_sums owner_rate_sums(const gdx_gref *GP, int s, 
 // chunks (optional) receives the rate partials of the lane's own chunks.
 template <int G, bool MOMENTS = true>
 __device__ __forceinline__ rate_sums group_rate_sums(const gdx_gref *GP, int s, bool own, double2 me, double m, int g,
-                                                     double *cat3, double *chunks = nullptr)
+                                                     double *cat3, const log_entry *logs, double *chunks = nullptr)
 {
     constexpr int P = N_K / G;                 // positions per lane
     constexpr int CP = P / 4;                  // chunks per lane
@@ -528,7 +528,7 @@ __device__ __forceinline__ rate_sums group_rate_sums(const gdx_gref *GP, int s, 
         cat3[1] = c.second;
         cat3[2] = c.maximum;
     }
-    const cat_moments_lds cm{cat3};
+    const cat_moments_lds cm{cat3, logs};
     auto eval = [&](const partner &q) {
         if constexpr (MOMENTS) return eval_pair_terms(t, cm, q, lambda_0);
         else return eval_pair_rate(t, q, lambda_0);
@@ -605,8 +605,8 @@ static_assert(BLOCK / RATE_LANES == RATE_SUB_OWNERS, "host block starts of the l
 // A block's bins in LDS, BIN_COPIES times over: the lanes of a wavefront mostly share a bin or two, and atomics on
 // one address run one after the other. Lane l adds to copy l mod BIN_COPIES, whose size is an odd number of doubles,
 // so that the copies of one field lie in different banks; the flush adds the copies up. Sixteen copies leave at most
-// four lanes on an address, for 14 KB a block. 64 realizations of 65536
-// owners: the screens of a step 5.6 -> 2.8 ms (one at a time).
+// four lanes on an address, for 14 KB a block. 64 realizations of 65536 owners: the screens of a step 5.6 -> 2.8 ms
+// (one at a time).
 constexpr int BIN_COPIES = 16;
 
 struct rate_lds
@@ -622,6 +622,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void
     constexpr bool GROUPED = LANES > 1;
     constexpr int OWNERS = BLOCK / LANES;
     __shared__ rate_lds acc[BIN_COPIES];
+    __shared__ log_entry logs[LOG_CELLS];
     // blocks cover the group's rated owners (every owner, or a learned swarm's subsample)
     const int b = xcd_block();
     if (b >= w.bstart[w.n]) return;
@@ -647,6 +648,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void
     __shared__ unsigned checked[2];
     for (int i = threadIdx.x; i < int(sizeof(acc) / sizeof(double)); i += BLOCK) reinterpret_cast<double *>(acc)[i] = 0.0;
     if (threadIdx.x < 2) checked[threadIdx.x] = 0u;
+    copy_log_table(logs, BLOCK);
     __syncthreads();
     const int s = w.beg[gi] + (sub < 0 ? i : ((i / THIN_RUN)*GP->thin_stride + sub)*THIN_RUN + i % THIN_RUN);
     const bool own = s < w.beg[gi] + w.cnt[gi];
@@ -655,8 +657,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3))) void
     __shared__ double cats[BLOCK][3];
     const bool live = own && m > 0.0;
     rate_sums rs;
-    if constexpr (LANES == 1) rs = owner_rate_sums(GP, s, own, me, m, &cats[threadIdx.x][0]);
-    else rs = group_rate_sums<LANES>(GP, s, own, me, m, g, &cats[threadIdx.x][0]);
+    if constexpr (LANES == 1) rs = owner_rate_sums(GP, s, own, me, m, &cats[threadIdx.x][0], logs);
+    else rs = group_rate_sums<LANES>(GP, s, own, me, m, g, &cats[threadIdx.x][0], logs);
     // the owner's sums are on every lane of its group: its first lane writes and counts
     const bool lead = own && g == 0;
     const fold3 total = rs.total;
@@ -1335,7 +1337,7 @@ __global__ __launch_bounds__(BLOCK) void k_candidates(gdx_wave w, const int *vst
     const double2 me = own ? GP->st[s] : make_double2(1.0, 0.0);
     const double m = own ? GP->measure[s] : 0.0;
     double chunks[CP];
-    const rate_sums rs = group_rate_sums<CAND_LANES, false>(GP, s, own, me, m, g, nullptr, chunks);
+    const rate_sums rs = group_rate_sums<CAND_LANES, false>(GP, s, own, me, m, g, nullptr, nullptr, chunks);
     const double R = rs.total.r;
 #pragma unroll
     for (int c = 0; c < CP; ++c) chunk_rate[g*CP + c][cand] = chunks[c];
@@ -1474,7 +1476,7 @@ __global__ __launch_bounds__(BLOCK) void k_candidates(gdx_wave w, const int *vst
                     {
                         // the K-sum at the new size and the next wait from the event
                         const rate_sums r2 = group_rate_sums<CAND_LANES, false>(
-                            GP, s, true, make_double2(size_new, numr_new), m, g, nullptr);
+                            GP, s, true, make_double2(size_new, numr_new), m, g, nullptr, nullptr);
                         extra_pairs += N_K;
                         const double R2 = r2.total.r;
                         const double remaining = end - t_event;
@@ -1768,6 +1770,8 @@ __global__ __launch_bounds__(BLOCK) void k_chain(gdx_wave w, gdx_chain_log clog,
     __shared__ unsigned long long end_key, end_sum[5];
     __shared__ unsigned long long *end_wave;
     __shared__ int lpool;                     // the block's next light position
+    __shared__ log_entry logs[LOG_CELLS];
+    copy_log_table(logs, BLOCK);
     if (threadIdx.x == 0) end_key = 0ull;
     if (threadIdx.x < 5) end_sum[threadIdx.x] = 0ull;
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
@@ -2172,7 +2176,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain(gdx_wave w, gdx_chain_log clog,
         const double nx_u1 = __shfl(pool_u, segbase + pool_used + 1, WAVE);
         const double nx_u2 = __shfl(pool_u, segbase + pool_used + 2, WAVE);
         // owners outside a learned swarm's audited subsample keep no compensators: rates alone
-        pair_term p = moments ? eval_pair_terms<cat_moments_deferred, HOLD_PARTNER>(t, cat_moments_deferred{}, q,
+        pair_term p = moments ? eval_pair_terms<cat_moments_deferred, HOLD_PARTNER>(t, cat_moments_deferred{logs}, q,
                                                                                     lambda_0, pt)
                               : eval_pair_rate<HOLD_PARTNER>(t, q, lambda_0, pt);
         // the catastrophic moments (owner-size logarithm and exponentials) only at events where some
@@ -2393,6 +2397,9 @@ __global__ __launch_bounds__(BLOCK) void k_chain_moments(gdx_wave w, gdx_chain_l
     __shared__ double sums[WAVES][NSEG][3];
     const int heavy = w.qprefix[w.n];
     if (heavy == 0 || heavy > clog.owners) return;
+    __shared__ log_entry logs[LOG_CELLS];
+    copy_log_table(logs, BLOCK);
+    __syncthreads();
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     const int seg = lane / SEG, kl = lane % SEG;
     const int items = heavy + min(*clog.next, CHAIN_EXTRA);
@@ -2423,7 +2430,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_moments(gdx_wave w, gdx_chain_l
             const bool own = i + seg < end;
             const double2 interval = own ? entries[i + seg] : make_double2(1.0, 0.0);
             const owner_terms t = make_owner(e, interval.x, m, hg_i);
-            pair_term p = eval_pair_terms(t, cat_moments_deferred{}, q, lambda_0);
+            pair_term p = eval_pair_terms(t, cat_moments_deferred{logs}, q, lambda_0);
             if constexpr (CAN_FRAGMENT)
             {
                 const bool cat = own && q.valid && catastrophic_pair(t, q.size_j, p.vrel >= V_FRAG);

@@ -192,6 +192,8 @@ struct run_buffers
     dbuf<unsigned char> back_d;
     pinned<unsigned char> back_h;
     size_t off_rate = 0, off_wave = 0, off_err = 0, off_audit = 0, back_bytes = 0;
+    unsigned long long back_number = 0;
+    unsigned long long *back_flag() { return reinterpret_cast<unsigned long long *>(back_h.p + back_bytes); }
     view<gdx_raw_rate> raw_rate, h_rate;
     view<gdx_raw_audit> raw_audit, h_audit;
     view<int> err, h_err;
@@ -207,8 +209,9 @@ struct run_buffers
         off_err = align(off_wave + sizeof(unsigned long long)*size_t(swarms)*GDX_WAVE_CTRS);
         off_audit = align(off_err + sizeof(int)*size_t(swarms));
         back_bytes = align(off_audit + sizeof(gdx_raw_audit)*size_t(groups)*COL_BIN_S);
-        back_d.alloc(back_bytes);
-        back_h.resize(back_bytes);
+        // behind the data: the count of the read-back's finished blocks, the number of the last read-back
+        back_d.alloc(back_bytes + 16);
+        back_h.resize(back_bytes + 16);
         raw_rate.p = reinterpret_cast<gdx_raw_rate *>(back_d.p + off_rate);
         wave_ctr.p = reinterpret_cast<unsigned long long *>(back_d.p + off_wave);
         err.p = reinterpret_cast<int *>(back_d.p + off_err);
@@ -428,7 +431,6 @@ void launch_queue_prefix(hipStream_t st, const gdx_wave &w, int *qprefix);
 void launch_majorant(hipStream_t st, const gdx_wave &w, int blocks);
 void launch_zero(hipStream_t st, const zero_ranges &z);
 // bytes (a multiple of 16) from device memory into page-locked host memory by a kernel on the stream
-void launch_to_host(hipStream_t st, void *host_dst, const void *src, size_t bytes);
 // the ranges cleared and `bytes` of host data (multiple of 4) written to dst by one launch: the data ride
 // in the kernel's arguments when they fit (STAGE_INLINE_BYTES), else a zero launch and a copy
 constexpr int STAGE_INLINE_BYTES = 3072;

@@ -2692,23 +2692,35 @@ void launch_zero(hipStream_t st, const zero_ranges &z)
     hip_check(hipGetLastError(), "launch zero");
 }
 
-__global__ __launch_bounds__(256) void k_to_host(uint4 *dst, const uint4 *src, int n)
+// The last block to finish sets the flag behind the data, so that the host reads a phase's results as soon as they
+// are in its memory, without waiting for the end of the launch to reach the runtime. The data are written through
+// to system scope and each wavefront waits for its own stores before its block arrives: the flag follows them
+// without a release, which would write back the L2 under the kernels of other streams.
+__global__ __launch_bounds__(256) void k_to_host(unsigned long long *dst, const unsigned long long *src, int n,
+                                                 unsigned int *arrived, unsigned long long *flag,
+                                                 unsigned long long number)
 {
-    for (int i = blockIdx.x*blockDim.x + threadIdx.x; i < n; i += gridDim.x*blockDim.x) dst[i] = src[i];
-}
-
-void launch_to_host(hipStream_t st, void *host_dst, const void *src, size_t bytes)
-{
-    const int n = int(bytes / 16);
-    if (!n) return;
-    k_to_host<<<std::min(16, (n + 255) / 256), 256, 0, st>>>(static_cast<uint4 *>(host_dst),
-                                                             static_cast<const uint4 *>(src), n);
-    hip_check(hipGetLastError(), "launch read-back");
+    for (int i = blockIdx.x*blockDim.x + threadIdx.x; i < n; i += gridDim.x*blockDim.x)
+        __hip_atomic_store(dst + i, src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    if (gridDim.x > 1)
+    {
+        if (__hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != gridDim.x - 1) return;
+        *arrived = 0u;
+    }
+    __hip_atomic_store(flag, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 void run_buffers::read_back(size_t from, size_t to, hipStream_t st)
 {
-    launch_to_host(st, back_h.p + from, back_d.p + from, to - from);
+    const int n = int((to - from) / sizeof(unsigned long long));
+    k_to_host<<<std::max(1, std::min(32, (n + 255) / 256)), 256, 0, st>>>(
+        reinterpret_cast<unsigned long long *>(back_h.p + from),
+        reinterpret_cast<const unsigned long long *>(back_d.p + from), n,
+        reinterpret_cast<unsigned int *>(back_d.p + back_bytes), back_flag(), ++back_number);
+    hip_check(hipGetLastError(), "launch read-back");
 }
 
 // a phase's due list (ints and bath ends) in the launch's arguments, written by the first block

@@ -969,7 +969,7 @@ __device__ __forceinline__ void topk_flush(uint64_t (&L)[K], const char *col, in
         const uint32_t hi = r < cnt ? uint32_t(v >> 32) : TOPK_NO_KEY;
         S[r] = (uint64_t(hi) << 32) | uint32_t(v);
     }
-    bitonic_sort<B>(S);
+    odd_even_sort<B>(S);
     topk_merge_sorted<K, B>(L, S);
 }
 

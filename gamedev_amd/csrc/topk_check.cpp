@@ -68,7 +68,7 @@ int run(long trials, lcg &g, long &merges)
         auto flush = [&] {
             uint64_t S[B];
             for (int r = 0; r < B; ++r) S[r] = r < cnt ? buf[r] : TOPK_EMPTY;
-            bitonic_sort<B>(S);
+            odd_even_sort<B>(S);
             topk_merge_sorted<K, B>(L, S);
             cnt = 0;
             ++merges;

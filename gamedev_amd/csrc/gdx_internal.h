@@ -403,6 +403,7 @@ void geometry_epoch(context &c);
 void load_state(context &c);
 void store_state(context &c);
 // test access: exact top-K over a built index for arbitrary queries and a runtime K
+void sort_keys(dbuf<uint64_t> &keys, dbuf<int> &idx, int n, int bits, bool flat, sort_scratch &s, hipStream_t st);
 void write_nodes(morton_index &ix, hipStream_t st);
 const unsigned int *morton_total(const morton_index &ix);
 void morton_settle(morton_index &ix, unsigned int total, hipStream_t st);

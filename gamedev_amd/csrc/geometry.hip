@@ -1309,9 +1309,9 @@ void scan_exclusive_u32(const unsigned int *in, unsigned int *out, int n, sort_s
     hip_check(hipGetLastError(), "launch scan");
 }
 
-// keys sorted in place, idx becomes the stable permutation; 3*max_level bits in use, every third zero for dim 2
-static void sort_morton_keys(dbuf<uint64_t> &keys, dbuf<int> &idx, int n, int max_level, int dim, sort_scratch &s,
-                             hipStream_t st)
+// keys sorted in place, idx becomes the stable permutation; `bits` bits in use, of which every third is zero in
+// flat keys (two-dimensional Morton keys)
+void sort_keys(dbuf<uint64_t> &keys, dbuf<int> &idx, int n, int bits, bool flat, sort_scratch &s, hipStream_t st)
 {
     const int items = sort_items(n), nb = blocks_for(n, SORT_BLOCK*items);
     s.keys_alt.alloc(size_t(n));
@@ -1319,9 +1319,9 @@ static void sort_morton_keys(dbuf<uint64_t> &keys, dbuf<int> &idx, int n, int ma
     s.hist.alloc(size_t(RADIX)*nb + RADIX);
     unsigned int *const totals = s.hist.p + size_t(RADIX)*nb;
     bool first = true;
-    for (int shift = 0; shift < 3*max_level; shift += dim == 2 ? 12 : 8)
+    for (int shift = 0; shift < bits; shift += flat ? 12 : 8)
     {
-        const key_digit digit{shift, dim == 2};
+        const key_digit digit{shift, flat};
         const int *vals = first ? nullptr : idx.p;
         if (items == SORT_ITEMS) k_radix_hist<SORT_ITEMS><<<nb, SORT_BLOCK, 0, st>>>(keys.p, n, digit, s.hist.p, nb);
         else k_radix_hist<SORT_ITEMS_SMALL><<<nb, SORT_BLOCK, 0, st>>>(keys.p, n, digit, s.hist.p, nb);
@@ -1375,7 +1375,7 @@ void morton_build(morton_index &ix, const float4 *points, const unsigned char *a
     ix.chunks.alloc(size_t(blocks_for(n, CHUNK) + BOX_GROUP));
     k_morton_keys<<<blocks_for(n, 256), 256, 0, st>>>(points, n, ox, oy, oz, width, max_level, dim, ix.keys.p);
     hip_check(hipGetLastError(), "launch morton keys");
-    sort_morton_keys(ix.keys, ix.idx, n, max_level, dim, s, st);
+    sort_keys(ix.keys, ix.idx, n, 3*max_level, dim == 2, s, st);
     k_records<<<blocks_for(n, 256), 256, 0, st>>>(ix.idx.p, points, active, codes, n, ix.rec.p,
                                                      ix.chunks.p);
     hip_check(hipGetLastError(), "launch morton records");

@@ -331,16 +331,60 @@ __global__ __launch_bounds__(ADAM_BLOCK) void k_mlp_adam(float *__restrict__ p, 
     else P->b3 = q;
 }
 
-uint64_t splitmix(uint64_t &s)
+constexpr uint64_t SPLITMIX_STEP = 0x9e3779b97f4a7c15ull;
+__host__ __device__ inline uint64_t splitmix_of(uint64_t z)
 {
-    uint64_t z = (s += 0x9e3779b97f4a7c15ull);
     z = (z ^ (z >> 30))*0xbf58476d1ce4e5b9ull;
     z = (z ^ (z >> 27))*0x94d049bb133111ebull;
     return z ^ (z >> 31);
 }
+uint64_t splitmix(uint64_t &s) { return splitmix_of(s += SPLITMIX_STEP); }
 double unit(uint64_t &s) { return double(splitmix(s) >> 11)*0x1.0p-53; }
 
 }  // namespace
+
+// ---- the training order: the Fisher-Yates shuffle of one epoch, for i = n - 1 ... 1 a swap of positions i and
+// k_i = draw mod (i + 1), without its n dependent steps ----
+// Position x holds, just before step i, what the latest earlier step i' > i with k_i' = x moved there: what
+// position i' held just before step i'. So position i ends with the value found from the successor of i among the
+// steps with the same k, ascending, by following next(y), the first step after y with k = y, to its end (k_i itself
+// where there is no successor). The steps are grouped by one stable sort; the walks end, since they ascend, after
+// one link on average and ln n or so at most. 262144 samples: 1.7 ms on the host and 1 MB copied -> 65 us.
+constexpr int SHUFFLE_BLOCK = 256;
+// the host shuffles larger sets: the sort takes 28 bytes a sample
+constexpr long long SHUFFLE_MAX = 1ll << 26;
+
+// first: state before the epoch's first draw, which step n - 1 takes
+__global__ __launch_bounds__(SHUFFLE_BLOCK) void k_shuffle_draws(uint64_t first, int n, uint64_t *key, int *next)
+{
+    const int i = blockIdx.x*SHUFFLE_BLOCK + threadIdx.x;
+    if (i >= n) return;
+    key[i] = splitmix_of(first + uint64_t(n - i)*SPLITMIX_STEP) % uint64_t(i + 1);      // 0 for i = 0
+    next[i] = -1;
+}
+
+// after the sort: link[i] = i's successor among the steps with its k, or -1 - k
+__global__ __launch_bounds__(SHUFFLE_BLOCK) void k_shuffle_links(const uint64_t *key, const int *step, int n, int *link,
+                                                                int *next)
+{
+    const int p = blockIdx.x*SHUFFLE_BLOCK + threadIdx.x;
+    if (p >= n) return;
+    const int i = step[p], k = int(key[p]);
+    const int succ = p + 1 < n && int(key[p + 1]) == k ? step[p + 1] : -1;
+    link[i] = succ >= 0 ? succ : -1 - k;
+    if (p == 0 || int(key[p - 1]) != k) next[k] = i == k ? succ : i;
+}
+
+__global__ __launch_bounds__(SHUFFLE_BLOCK) void k_shuffle_order(const int *link, const int *next, int n, int *perm)
+{
+    const int i = blockIdx.x*SHUFFLE_BLOCK + threadIdx.x;
+    if (i >= n) return;
+    int y = link[i];
+    if (y < 0) y = -1 - y;
+    else
+        for (int z = next[y]; z >= 0; z = next[y]) y = z;
+    perm[i] = y;
+}
 
 // one majorant model: FP32 parameters and Adam moments, the packed fragments, the input normalization
 struct model
@@ -348,6 +392,10 @@ struct model
     dbuf<float> p, m1, m2, norm, partial, grad, loss;
     dbuf<pack> P;
     dbuf<int> perm;
+    // workspace of the shuffles
+    dbuf<uint64_t> draw;
+    dbuf<int> step_of, link, next;
+    sort_scratch scratch;
     long long steps = 0;
     unsigned long long version = 0;     // advanced by every change of the parameters or normalization
     std::vector<float> h_norm = std::vector<float>(2*F);
@@ -614,7 +662,14 @@ int gdx_col_majorant_train(gdx_col_majorant h, const float *features, const floa
         M.partial.alloc(size_t(rows)*P_STRIDE);
         M.perm.alloc(size_t(n));
         M.loss.alloc(size_t(std::max<long long>(1, batches)));
-        std::vector<int> perm(static_cast<size_t>(n));
+        std::vector<int> perm(n > SHUFFLE_MAX ? static_cast<size_t>(n) : 0);
+        if (n <= SHUFFLE_MAX)
+        {
+            M.draw.alloc(size_t(n));
+            M.step_of.alloc(size_t(n));
+            M.link.alloc(size_t(n));
+            M.next.alloc(size_t(n));
+        }
         std::vector<float> losses(static_cast<size_t>(std::max<long long>(1, batches)));
         uint64_t s = cfg->seed;
         const double b1 = cfg->beta1 > 0 ? cfg->beta1 : 0.9, b2 = cfg->beta2 > 0 ? cfg->beta2 : 0.999;
@@ -622,14 +677,30 @@ int gdx_col_majorant_train(gdx_col_majorant h, const float *features, const floa
         for (int ep = 0; ep < cfg->epochs; ++ep)
         {
             // Fisher-Yates shuffle of the sample order, one per epoch
-            for (long long i = 0; i < n; ++i) perm[size_t(i)] = int(i);
-            for (long long i = n - 1; i > 0; --i)
+            if (n <= SHUFFLE_MAX)
             {
-                long long k = (long long)(splitmix(s) % uint64_t(i + 1));
-                std::swap(perm[size_t(i)], perm[size_t(k)]);
+                const int m = int(n);
+                const dim3 grid(unsigned((m + SHUFFLE_BLOCK - 1) / SHUFFLE_BLOCK));
+                int bits = 1;
+                while (bits < 31 && (1 << bits) < m) ++bits;
+                k_shuffle_draws<<<grid, SHUFFLE_BLOCK>>>(s, m, M.draw.p, M.next.p);
+                gdx::sort_keys(M.draw, M.step_of, m, bits, false, M.scratch, nullptr);
+                k_shuffle_links<<<grid, SHUFFLE_BLOCK>>>(M.draw.p, M.step_of.p, m, M.link.p, M.next.p);
+                k_shuffle_order<<<grid, SHUFFLE_BLOCK>>>(M.link.p, M.next.p, m, M.perm.p);
+                gdx::hip_check(hipGetLastError(), "training order");
+                s += uint64_t(n - 1)*SPLITMIX_STEP;
             }
-            gdx::hip_check(hipMemcpy(M.perm.p, perm.data(), sizeof(int)*size_t(n), hipMemcpyHostToDevice),
-                           "training order");
+            else
+            {
+                for (long long i = 0; i < n; ++i) perm[size_t(i)] = int(i);
+                for (long long i = n - 1; i > 0; --i)
+                {
+                    long long k = (long long)(splitmix(s) % uint64_t(i + 1));
+                    std::swap(perm[size_t(i)], perm[size_t(k)]);
+                }
+                gdx::hip_check(hipMemcpy(M.perm.p, perm.data(), sizeof(int)*size_t(n), hipMemcpyHostToDevice),
+                               "training order");
+            }
             for (long long b = 0; b < batches; ++b)
             {
                 ++M.steps;

@@ -44,3 +44,22 @@ def test_gradient_rows(gpu, n):
     scale = np.abs(go).max()
     assert np.abs(g - go).max() <= max(2e-3, 2**-8/n)*scale + 1e-7
     assert float(np.dot(g, go)/np.linalg.norm(g)/np.linalg.norm(go)) > 0.9999
+
+
+@pytest.mark.parametrize("n,batch", [(1, 1), (2, 1), (3, 2), (255, 50), (256, 64), (257, 64), (513, 100), (5000, 1000)])
+def test_training_order(gpu, n, batch):
+    """Two epochs of minibatches in the oracle's shuffled order, one Adam step at 1e-2 each: a sample in another
+    minibatch would move parameters by a good part of the step."""
+    from gamedev_amd import Majorant
+    print(f"[majorant] training order n={n} batch={batch}", flush=True)
+    X, lt, norm = rand_data(300 + n, n)
+    p0 = rand_params(11)
+    m = Majorant("fiducial_3d", seed=1)
+    m.set_params(p0, norm)
+    losses = m.train(dev(X, gpu), dev(lt, gpu), epochs=2, batch=batch, lr=1e-2, seed=77)
+    p, _ = m.params()
+    po, lo = M.train(p0, norm, X, lt, epochs=2, batch=batch, lr=1e-2, seed=77)
+    # epoch losses to the rounding of a minibatch's BF16 activations; parameters except where a gradient near
+    # zero changes sign under that rounding
+    np.testing.assert_allclose(losses, lo, rtol=2e-3, atol=1e-6)
+    assert np.quantile(np.abs(p - po), 0.9) < 2e-3

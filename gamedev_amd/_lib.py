@@ -109,6 +109,7 @@ _SIGS = {
     "gdx_col_majorant_destroy": [P],
     "gdx_col_majorant_get_params": [P, P, P],
     "gdx_col_majorant_set_params": [P, P, P],
+    "gdx_col_majorant_feature_stats": [P, P, C.c_longlong, P, P],
     "gdx_col_majorant_infer": [P, P, C.c_longlong, P],
     "gdx_col_majorant_grad": [P, P, P, I, P, C.POINTER(D)],
     "gdx_col_majorant_grad_noalloc": [P, P, P, I, P, C.POINTER(D)],

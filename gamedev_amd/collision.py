@@ -373,13 +373,27 @@ class Majorant:
 
     def fit_normalization(self, features) -> np.ndarray:
         """Set the input normalization to the per-feature mean and standard deviation (1 where constant)."""
-        x = features.detach().double().cpu().numpy() if hasattr(features, "detach") else np.asarray(features)
-        mu = x.mean(axis=0)
-        sd = x.std(axis=0)
+        mu, sd = self._column_stats(features)
         sd = np.where(sd > 1e-12, sd, 1.0)
         norm = np.concatenate([mu, sd]).astype(np.float32)
         self.set_params(None, norm)
         return norm
+
+    def _column_stats(self, features) -> tuple[np.ndarray, np.ndarray]:
+        import torch
+        if not hasattr(features, "detach"):
+            x = np.asarray(features)
+        elif (features.is_cuda and features.dtype == torch.float32 and features.ndim == 2 and len(features)
+              and features.shape[1] == _lib.MAJORANT_FEATURES and features.device.index == torch.cuda.current_device()):
+            x = features.detach().contiguous()
+            # the rows may come from another stream than the library's
+            torch.cuda.current_stream().synchronize()
+            mu, sd = np.empty(_lib.MAJORANT_FEATURES), np.empty(_lib.MAJORANT_FEATURES)
+            self._call(self.lib.gdx_col_majorant_feature_stats, _ptr(x), len(x), _np_ptr(mu), _np_ptr(sd))
+            return mu, sd
+        else:
+            x = features.detach().double().cpu().numpy()
+        return x.mean(axis=0), x.std(axis=0)
 
     def fit_output(self, log_target) -> float:
         """Start the output bias at the mean log target, softplus(b3) = exp(mean), so that training

@@ -300,6 +300,9 @@ const char *gdx_col_majorant_last_error(gdx_col_majorant m);
  * set_params resets the Adam moments */
 int gdx_col_majorant_get_params(gdx_col_majorant m, float *params, float *norm16);
 int gdx_col_majorant_set_params(gdx_col_majorant m, const float *params, const float *norm16);
+/* mean and standard deviation (host, GDX_COL_MAJORANT_FEATURES each) of the columns of n > 0 device rows */
+int gdx_col_majorant_feature_stats(gdx_col_majorant m, const float *features, long long n, double *mean,
+                                   double *deviation);
 /* device rows in, device softplus outputs out */
 int gdx_col_majorant_infer(gdx_col_majorant m, const float *features, long long n, float *out);
 /* gradient (host, GDX_COL_MAJORANT_PARAMS) and value of the mean loss (ln softplus(z) - log_target)^2 */

@@ -63,3 +63,22 @@ def test_training_order(gpu, n, batch):
     # zero changes sign under that rounding
     np.testing.assert_allclose(losses, lo, rtol=2e-3, atol=1e-6)
     assert np.quantile(np.abs(p - po), 0.9) < 2e-3
+
+
+@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 16383, 16385, 200001])
+def test_feature_statistics(gpu, n):
+    """Column means and deviations of device rows against NumPy in FP64: sums of n rounded terms in two orders, the
+    constant column exactly constant."""
+    from gamedev_amd import Majorant
+    X, _, _ = rand_data(500 + n, n)
+    X[:, 3] = 2.5
+    X[:, 5] = 1e6 + X[:, 5]
+    m = Majorant("fiducial_3d", seed=1)
+    mu, sd = m._column_stats(dev(X, gpu))
+    x = X.astype(np.float64)
+    scale = np.abs(x).max(axis=0)
+    assert np.all(np.abs(mu - x.mean(axis=0)) <= n*2**-53*scale)
+    assert np.all(np.abs(sd - x.std(axis=0)) <= 4*n*2**-53*scale)
+    assert mu[3] == 2.5 and sd[3] == 0.0
+    norm = m.fit_normalization(dev(X, gpu))
+    assert norm[8 + 3] == 1.0

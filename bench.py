@@ -48,7 +48,8 @@ K = 32
 #                 + published (s, N) 16
 #   candidates:   per thinning candidate: candidate record 16 + owner state 16 + measure 8; per pair term of its
 #                 K-sums: code 4 + partner (s, N) 16
-#   queue_prefix: one block per phase over the group counters (not counted)
+#   queue_prefix: one block per phase over the group counters (not counted); a kernel of its own only while kernels
+#                 are timed or for more than 256 due groups, else formed by the chain's blocks
 #   chain:        per chained owner 140 (state, clock, draw counter, sums), per pair term: code 4 + partner (s, N) 16
 #   chain_audit:  per chained owner: queue entry 4 + chain sums 36 + published and final state 24
 #   majorant:     per due owner: stale flag 1; per evaluated owner: codes 4K + FP32 partner records 8K + owner

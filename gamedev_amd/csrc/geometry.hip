@@ -1203,8 +1203,8 @@ __global__ __launch_bounds__(WPB*WAVE) void k_col_topk(const float4 *__restrict_
 
 // runtime-K exact top-K for arbitrary query points (test access to the search contract)
 template <int K>
-__global__ __launch_bounds__(TOPK_BLOCK) void k_knn(const float4 *rec, const gdx_box *boxes, const float4 *queries, int nq, int *codes, float *dist,
-                                                   unsigned int *overflow)
+__global__ __launch_bounds__(TOPK_BLOCK) void k_knn(const float4 *rec, const gdx_box *boxes, const float4 *queries,
+                                                   int nq, int *codes, float *dist, unsigned int *overflow)
 {
     __shared__ int2 stacks[TOPK_BLOCK / WAVE][TOPK_STACK];
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;

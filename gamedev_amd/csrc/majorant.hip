@@ -346,7 +346,7 @@ double unit(uint64_t &s) { return double(splitmix(s) >> 11)*0x1.0p-53; }
 // ---- mean and standard deviation of each feature over the rows, in FP64 and two passes ----
 // Bound by the read of the rows, 32 bytes each; a block's threads take a column each, eight to a row, and leave one
 // sum per column, which one block adds up in a fixed order. 262144 rows: 22 us, where the rows were copied to
-// the host as FP64 and summed there in 9 ms.
+// the host as FP64 and summed there in 11 ms.
 constexpr int STATS_BLOCKS = 512, STATS_BLOCK = 256;
 
 template <bool CENTRED>

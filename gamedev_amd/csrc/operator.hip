@@ -11,6 +11,7 @@
 //   k_screen       col_skip_scan (col_skip_scan.cu): no-event owners finish and enter the audit sums,
 //                  the others are queued per group
 //   k_chain        col_chain_run (col_chain_run.cu): every queued owner's chain to its bath end
+//   k_chain_moments  the jump moments of the intervals that long chains logged
 //   k_chain_audit  col_audit_bin (col_audit_bin.cu) for the chained owners
 // Merged-bin sums are sums of raw-bin sums, so the host merges after the binmap is known.
 // Every kernel reads its groups through a table of per-group array pointers, so one launch serves

@@ -212,6 +212,8 @@ struct run_buffers
         // behind the data: the count of the read-back's finished blocks, the number of the last read-back
         back_d.alloc(back_bytes + 16);
         back_h.resize(back_bytes + 16);
+        // new memory, or another place in the old: whatever lies there is not a read-back's number (they begin at 1)
+        *back_flag() = 0ull;
         raw_rate.p = reinterpret_cast<gdx_raw_rate *>(back_d.p + off_rate);
         wave_ctr.p = reinterpret_cast<unsigned long long *>(back_d.p + off_wave);
         err.p = reinterpret_cast<int *>(back_d.p + off_err);

@@ -1,7 +1,8 @@
 // Learned rate majorant: training and inference kernels of the 8-64-64-1 perceptron (gdx_mlp.h) and the
 // C ABI of a majorant model (gdx_col_majorant_*). No counterpart in the reference.
 //
-//   k_mlp_infer   y = softplus(net(x)) for n feature rows, one or four 16-row tiles per wavefront step
+//   k_mlp_infer   y = softplus(net(x)) for n feature rows, four 16-row tiles per wavefront step; few rows
+//                 take k_mlp_infer_few, one tile per wavefront
 //   k_mlp_grad    forward + backward of a minibatch: each block takes ROW_TILES tiles, one per wavefront,
 //                 and writes one partial gradient row (deterministic, no atomics); weight gradients are
 //                 MFMA products over the sample dimension, their operands transposed through LDS
@@ -75,30 +76,45 @@ __global__ void k_mlp_pack(const float *p, const float *norm, pack *P)
     build_pack(p, norm, norm + F, P, threadIdx.x, blockDim.x);
 }
 
-// bound by the vector units: 128 SiLU a row, an exponential and a reciprocal each at half the rate.
+// Up to INFER_FEW rows, one tile a wavefront: bound by the latency of one pass, so the row's own inputs are read
+// first and each layer's weights where they are used. In a loop over tiles the compiler reads all weights ahead of
+// the loop and the inputs behind them, which a single tile has to wait for: 4.4 us a launch of 10,000 rows, 3.7 so.
+__global__ __launch_bounds__(BLOCK, 4) void k_mlp_infer_few(const pack *P, const float *X, int n, float *y)
+{
+    const int lane = threadIdx.x & 63, j = lane & 15;
+    const int first = 16*(int(blockIdx.x)*WAVES + int(threadIdx.x)/64);
+    if (first >= n) return;
+    const bool valid = first + j < n;
+    forward_state f;
+    const float z = tile_forward(P, input_fragment(P, X + (long long)(valid ? first + j : 0)*F, valid), f);
+    if (lane < 16 && valid) y[first + lane] = softplus(z);
+}
+
+// Many rows: bound by the vector units, 128 SiLU a row, an exponential and a reciprocal each at half the rate.
 // The weights stay in registers (a wavefront keeps them for all its tiles: nothing the kernel writes can
 // alias them), so the grid is what the GPU holds at once, four wavefronts per SIMD at 122 registers; the
 // bound of four keeps the accumulators out of the accumulation registers, which cost a move for each value
 // read. A tile leaves its results in 16 lanes, four times over: with four tiles a step every lane takes one
-// row through the softplus, some 120 instructions that every tile paid before. A million rows: 58 -> 47.5 us. Below
-// a tile for each wavefront a tile a step spreads the rows wider: 16.7 us a call for 16,384 rows against 19.2 with
-// four, 19.7 against 19.3 for 65,536, 22.1 against 21.3 for 131,072.
+// row through the softplus, some 120 instructions that every tile paid before. A million rows: 58 -> 47.5 us.
+constexpr int INFER_TILES = 4;
 constexpr int INFER_BLOCKS = 1024;
-constexpr long long INFER_WIDE = 16ll*WAVES*INFER_BLOCKS;
+// The most rows that go one tile a wavefront: their time grows with every tile a SIMD gets, 16,384 rows, the loop's
+// with every step, 65,536 rows. 65,600 rows: 7.4 us against 7.9 with the loop, 81,920: 8.2 against 9.0, 90,112: 9.2
+// against 9.1, 106,496: 10.3 against 9.0.
+constexpr long long INFER_FEW = 5*16*1024;
 
-template <int TILES>
 __global__ __launch_bounds__(BLOCK, 4) void k_mlp_infer(const pack *__restrict__ P, const float *__restrict__ X,
                                                        long long n, float *__restrict__ y)
 {
-    static_assert(TILES == 1 || TILES == 4, "a lane holds the row of its own tile");
+    static_assert(16*INFER_TILES == 64, "a lane holds the row of its own tile");
     const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
-    const long long steps = (n + 16*TILES - 1) / (16*TILES);
+    const long long steps = (n + 63) / 64;
     for (long long t = (long long)blockIdx.x*WAVES + threadIdx.x/64; t < steps; t += (long long)gridDim.x*WAVES)
     {
-        const long long first = t*16*TILES;
+        const long long first = t*64;
         float z = 0.0f;
 #pragma unroll
-        for (int k = 0; k < TILES; ++k)
+        for (int k = 0; k < INFER_TILES; ++k)
         {
             const long long r = first + 16*k + j;
             const bool valid = r < n;
@@ -108,7 +124,7 @@ __global__ __launch_bounds__(BLOCK, 4) void k_mlp_infer(const pack *__restrict__
             z = g == k ? v : z;
         }
         const long long row = first + lane;
-        if (lane < 16*TILES && row < n) y[row] = softplus(z);
+        if (row < n) y[row] = softplus(z);
     }
 }
 
@@ -489,11 +505,17 @@ const pack *model_pack(const model &M) { return M.P.p; }
 void launch_mlp_infer(const pack *P, const float *X, long long n, float *y, hipStream_t st)
 {
     if (n <= 0) return;
-    const int per = n >= INFER_WIDE ? 4 : 1;
-    const long long steps = (n + 16*per - 1) / (16*per);
-    const dim3 blocks(unsigned(std::min<long long>((steps + WAVES - 1) / WAVES, INFER_BLOCKS)));
-    if (per == 4) k_mlp_infer<4><<<blocks, BLOCK, 0, st>>>(P, X, n, y);
-    else k_mlp_infer<1><<<blocks, BLOCK, 0, st>>>(P, X, n, y);
+    if (n <= INFER_FEW)
+    {
+        const long long tiles = (n + 15) / 16;
+        k_mlp_infer_few<<<dim3(unsigned((tiles + WAVES - 1) / WAVES)), BLOCK, 0, st>>>(P, X, int(n), y);
+    }
+    else
+    {
+        const long long steps = (n + 63) / 64;
+        const long long blocks = std::min<long long>((steps + WAVES - 1) / WAVES, INFER_BLOCKS);
+        k_mlp_infer<<<dim3(unsigned(blocks)), BLOCK, 0, st>>>(P, X, n, y);
+    }
     hip_check(hipGetLastError(), "majorant inference launch");
 }
 

@@ -29,6 +29,27 @@ def test_inference_rows(gpu, n):
     assert np.array_equal(m.infer(x[n - k:].contiguous()).cpu().numpy(), y[n - k:])
 
 
+@pytest.mark.parametrize("n", [81903, 81919, 81920, 81921, 81985])
+def test_inference_rows_either_kernel(gpu, n):
+    """Both sides of the row count from which a wavefront takes four tiles in a loop instead of one, and the same
+    bits from either kernel."""
+    from gamedev_amd import Majorant
+    print(f"[majorant] inference n={n}", flush=True)
+    X, _, norm = rand_data(n, n)
+    p = rand_params(n)
+    m = Majorant("fiducial_3d", seed=1)
+    m.set_params(p, norm)
+    x = dev(X, gpu)
+    y = m.infer(x).cpu().numpy()
+    yo = M.predict(p, norm, X)
+    rel = np.abs(y - yo)/yo
+    assert np.median(rel) < 2e-5 and rel.max() < 5e-3, (np.median(rel), rel.max())
+    for k in (17, 16384):
+        assert np.array_equal(m.infer(x[n - k:].contiguous()).cpu().numpy(), y[n - k:])
+    double = m.infer(x.repeat(2, 1)).cpu().numpy()
+    assert np.array_equal(double[:n], y) and np.array_equal(double[n:], y)
+
+
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 127, 128, 129, 1025])
 def test_gradient_rows(gpu, n):
     from gamedev_amd import Majorant

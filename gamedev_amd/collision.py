@@ -237,6 +237,17 @@ class CollisionOperator:
         not depend on it."""
         self._call(self.lib.gdx_col_set_exact_walk, int(bool(on)))
 
+    def set_chain_log_chunks(self, chunks: int) -> None:
+        """Test access: chunks beyond an owner's first that the chain's interval logs may take (default all)."""
+        self._call(self.lib.gdx_col_set_chain_log_chunks, int(chunks))
+
+    def chain_sums(self) -> tuple[np.ndarray, np.ndarray, int]:
+        """Test access: {hazard, first and second jump moment, largest jump} and events per particle of the last
+        chain phase of the last call, and the log chunks asked for."""
+        sums, events, asked = np.empty((self.n, 4)), np.empty(self.n, np.int32), C.c_int()
+        self._call(self.lib.gdx_col_get_chain_sums, _np_ptr(sums), _np_ptr(events), C.byref(asked))
+        return sums, events, asked.value
+
     def set_narrow_waves(self, owners: int) -> None:
         """Refresh waves of at most `owners` due owners take the narrow launch shapes (four lanes per
         plain owner in the rate pass, one owner per lane in the screen); 0 always takes the wide ones.

@@ -199,6 +199,7 @@ phase_wave upload_phase(run_buffers &rb, const std::vector<phase_entry> &e, hipS
 {
     const int n = int(e.size());
     rb.reserve(n);
+    rb.chain_blocks = 0;
     int *ref = rb.h_int, *beg = ref + n, *cnt = beg + n, *sub = cnt + n, *b1024 = sub + n, *b256 = b1024 + n + 1;
     int *bsub = b256 + n + 1, *bmaj = bsub + n + 1, *blsub = bmaj + n + 1;
     int total = 0, x = 0, y = 0, z = 0, u = 0, v = 0, learned = 0;
@@ -712,6 +713,9 @@ void run_swarms(std::vector<op_run *> &runs, run_buffers &rb, hipStream_t st, ke
     const int ng = nr*LOCAL_GROUPS;
     const int narrow_owners = runs[0]->c.narrow_owners;
     rb.size_run(ng, nr);
+    rb.log_extra = runs[0]->c.log_chunks;
+    rb.chain_of = nr == 1 ? &runs[0]->c : nullptr;
+    rb.chain_epoch = runs[0]->c.epochs;
     rb.h_table.clear();
     for (op_run *r : runs)
     {
@@ -813,6 +817,8 @@ void run_swarms(std::vector<op_run *> &runs, run_buffers &rb, hipStream_t st, ke
                 timer.time(GDX_COL_KERNEL_PREFIX, pw.w256.total, [&] { launch_queue_prefix(st, pw.w256, rb.qprefix.p); });
             timer.time(GDX_COL_KERNEL_CHAIN, pw.w256.total, [&] { launch_chain(st, pw.w256, rb, own_prefix); });
             timer.time(GDX_COL_KERNEL_AUDIT, pw.w256.total, [&] { launch_chain_audit(st, pw.w1024, pw.blocks1024, rb); });
+            rb.chain_wave = pw.w256;
+            rb.chain_blocks = pw.blocks256;
             rb.read_back(rb.off_wave, rb.back_bytes, st);          // wave counters, errors, audit bins
             wait_results(rb, st, "chain pass");
             unsigned long long longest = 0;
@@ -1568,6 +1574,37 @@ int gdx_col_set_exact_walk(gdx_col_handle h, int on)
 {
     if (!h) return GDX_COL_ERR_ARG;
     return guard(&h->c, [&] { h->c.exact_walk = on ? 1 : 0; });
+}
+
+int gdx_col_set_chain_log_chunks(gdx_col_handle h, int chunks)
+{
+    if (!h) return GDX_COL_ERR_ARG;
+    return guard(&h->c, [&] {
+        require(chunks >= 0 && chunks <= CHAIN_EXTRA, GDX_COL_ERR_ARG, "chain log chunks out of range");
+        h->c.log_chunks = chunks;
+    });
+}
+
+int gdx_col_get_chain_sums(gdx_col_handle h, double *sums4, int *events, int *asked)
+{
+    if (!h || !sums4 || !events || !asked) return GDX_COL_ERR_ARG;
+    return guard(&h->c, [&] {
+        context &c = h->c;
+        run_buffers &rb = h->rb;
+        require(rb.chain_blocks > 0 && rb.chain_of == &c && rb.chain_epoch == c.epochs, GDX_COL_ERR_STATE,
+                "no chain phase of an operator call to read");
+        dbuf<double4> sums;
+        dbuf<int> ev;
+        sums.alloc(size_t(c.n));
+        ev.alloc(size_t(c.n));
+        hip_check(hipMemsetAsync(sums.p, 0, sizeof(double4)*size_t(c.n), c.stream), "zero chain sums");
+        hip_check(hipMemsetAsync(ev.p, 0, sizeof(int)*size_t(c.n), c.stream), "zero chain events");
+        launch_chain_sums(c.stream, rb, sums.p, ev.p);
+        copy_d2h(sums4, sums.p, sizeof(double4)*size_t(c.n), c.stream);
+        copy_d2h(events, ev.p, sizeof(int)*size_t(c.n), c.stream);
+        copy_d2h(asked, rb.log_next.p, sizeof(int), c.stream);
+        hip_check(hipStreamSynchronize(c.stream), "read chain sums");
+    });
 }
 
 int gdx_col_set_narrow_waves(gdx_col_handle h, int owners)

@@ -141,6 +141,8 @@ struct view
 // chains lose 4 us each to the launch, a chain of LONG_CHAIN events gains 0.1 ms
 constexpr int LONG_CHAIN = 64, CHAIN_LOG_PHASES = 32;
 
+struct context;
+
 // buffers of operator runs: the group table, pinned staging and device copies of the due lists,
 // the chain's queue prefix
 struct run_buffers
@@ -174,6 +176,12 @@ struct run_buffers
     // time). The logs cost a launch; without them a long chain costs its owner's moments at every event. The
     // results do not depend on it.
     int log_phases = CHAIN_LOG_PHASES;
+    int log_extra = CHAIN_EXTRA;      // chunks beyond the owners' first that the logs may take
+    // the last chain phase of the last run, if that was of one swarm (test access)
+    gdx_wave chain_wave{};
+    int chain_blocks = 0;
+    const context *chain_of = nullptr;
+    unsigned long long chain_epoch = 0;
     void reserve_log(int owners)
     {
         const size_t chunks = size_t(owners) + CHAIN_EXTRA;
@@ -183,7 +191,7 @@ struct run_buffers
         log_prev.alloc(chunks);
         log_last.alloc(size_t(owners));
         log = gdx_chain_log{log_entry.p, log_part.p, log_use.p, log_prev.p, log_last.p, log_next.p, owners,
-                            log_phases > 0, hcount.p, qcount.p};
+                            log_extra, log_phases > 0, hcount.p, qcount.p};
     }
     // controller sums, queue lengths, counters and errors of every group and swarm of the run. The
     // read-backs share one device block and one page-locked mirror laid out [raw_rate][wave_ctr][err]
@@ -373,6 +381,8 @@ struct context
     int thin_stride = THIN_STRIDE;   // learned: exact subsample stride (THIN_STRIDE_LARGE for large swarms)
     int majorant_min_owners = GDX_COL_MAJORANT_MIN_OWNERS;   // smaller swarms keep the plain method
     double fixed_bath = 0.0;   // > 0: every bath lasts this long (test access; the controller still audits)
+    int log_chunks = CHAIN_EXTRA;     // extra chunks of the chain's interval logs (test access)
+    unsigned long long epochs = 0;    // geometry epochs built
     int exact_walk = 0;        // 1: the chain's partner walk from sequential partials only (test access)
     bool diag = false;         // GDX_COL_DIAGNOSTICS
     dbuf<gdx_event_work> evw;  // per-slot event statistics of the current call
@@ -447,6 +457,7 @@ void build_reverse(context &c);
 int chain_resident_blocks();
 void launch_chain(hipStream_t st, const gdx_wave &w, run_buffers &rb, bool own_prefix);
 void launch_chain_audit(hipStream_t st, const gdx_wave &w, int blocks, const run_buffers &rb);
+void launch_chain_sums(hipStream_t st, const run_buffers &rb, double4 *sums, int *events);
 void launch_event_sum(context &c, hipStream_t st);
 void launch_gather_cached(context &c, double *out_particle_order);
 void launch_pair_rates(context &c, const gdx_gref &G, double *out_particle_order);

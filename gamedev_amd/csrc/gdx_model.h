@@ -208,11 +208,11 @@ struct gdx_wave
 };
 
 // waiting intervals {size, length} of the heavy owners that one chain launch ran alone on a wavefront each,
-// in chunks of CHAIN_CHUNK intervals of one owner: chunk h is heavy owner h's first, the CHAIN_EXTRA chunks
+// in chunks of CHAIN_CHUNK intervals of one owner: chunk h is heavy owner h's first, the `extra` chunks
 // from `owners` on go to the owners that need more, in order of `next`. An owner's chunks are linked from its
 // last one back, and each gets the jump-moment sums {j1, j2, jmax} of its intervals.
 constexpr int CHAIN_CHUNK = 64;
-constexpr int CHAIN_EXTRA = 8192;
+constexpr int CHAIN_EXTRA = 8192;   // extra chunks reserved
 struct gdx_chain_log
 {
     double2 *entry;              // CHAIN_CHUNK per chunk
@@ -222,6 +222,7 @@ struct gdx_chain_log
     int *last;                   // per heavy owner: its last chunk, -1 none logged
     int *next;                   // extra chunks asked for
     int owners;                  // heavy owners that run alone at most; with more there are no logs
+    int extra;                   // at most CHAIN_EXTRA
     int enabled;                 // 0: no logs, owners that need jump moments take the general loop
     const int *hcount, *qcount;  // heavy and light queue lengths by group-table entry
 };

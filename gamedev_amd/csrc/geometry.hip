@@ -1510,6 +1510,7 @@ void geometry_epoch(context &c)
     hipStream_t st = c.stream;
     c.geometry_valid = false;
     c.state_loaded = false;
+    ++c.epochs;
     c.pts.alloc(n);
     c.active.alloc(n);
     c.group.alloc(n);

@@ -1970,10 +1970,10 @@ __global__ __launch_bounds__(BLOCK) void k_chain(gdx_wave w, gdx_chain_log clog,
             if (lane == 0)
             {
                 clog.use[chunk] = make_int4(w.ref[gi], s, CHAIN_CHUNK, 0);
-                if (c < CHAIN_EXTRA) clog.prev[clog.owners + c] = chunk;
+                if (c < clog.extra) clog.prev[clog.owners + c] = chunk;
                 else clog.last[h] = chunk;
             }
-            chunk = c < CHAIN_EXTRA ? clog.owners + c : -1;
+            chunk = c < clog.extra ? clog.owners + c : -1;
             logged = 0;
             asked = false;
         };
@@ -2054,7 +2054,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain(gdx_wave w, gdx_chain_log clog,
             clog.use[chunk] = make_int4(w.ref[gi], s, logged, 0);
             clog.last[h] = moments ? chunk : -1;
             // a chunk asked for and not begun
-            if (asked && ahead < CHAIN_EXTRA) clog.use[clog.owners + ahead] = make_int4(w.ref[gi], s, 0, 0);
+            if (asked && ahead < clog.extra) clog.use[clog.owners + ahead] = make_int4(w.ref[gi], s, 0, 0);
         }
         if (done)
         {
@@ -2403,7 +2403,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_moments(gdx_wave w, gdx_chain_l
     __syncthreads();
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     const int seg = lane / SEG, kl = lane % SEG;
-    const int items = heavy + min(*clog.next, CHAIN_EXTRA);
+    const int items = heavy + min(*clog.next, clog.extra);
     for (int item = blockIdx.x; item < items; item += gridDim.x)
     {
         const int chunk = item < heavy ? item : clog.owners + (item - heavy);
@@ -2477,6 +2477,18 @@ __global__ __launch_bounds__(BLOCK) void k_chain_moments(gdx_wave w, gdx_chain_l
     }
 }
 
+// the logged jump moments of heavy position h (k_chain_moments) added to its owner's chain sums
+__device__ __forceinline__ void add_logged(const gdx_chain_log &clog, int h, double4 &sum)
+{
+    for (int k = clog.last[h]; k >= 0; k = clog.prev[k])
+    {
+        const double4 v = clog.part[k];
+        sum.y += v.x;
+        sum.z += v.y;
+        sum.w = fmax(sum.w, v.z);
+    }
+}
+
 // audit of the chained owners, one lane per queue position of each due group (col_audit_bin.cu:13-60),
 // AUDIT_ROUNDS positions per lane: a block covers 1024 slots of its group, and blocks without a queued
 // position (most of them, the queues being short) leave after reading two counters
@@ -2493,7 +2505,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_audit(gdx_wave w, gdx_chain_log
     const int h1 = w.beg[gi] + *G.hcount;
     const int l0 = w.beg[gi] + w.cnt[gi] - *G.qcount;
     if (s0 >= h1 && s1 <= l0) return;
-    // the heavy positions' logged jump moments (k_chain_moments), where the heavy owners ran alone
+    // whether the heavy owners ran alone and logged
     const bool logs = clog.enabled && w.qprefix[w.n] <= clog.owners;
     const int hbase = w.qprefix[gi] - w.beg[gi];
     const double end = w.dt[gi];
@@ -2526,16 +2538,7 @@ __global__ __launch_bounds__(BLOCK) void k_chain_audit(gdx_wave w, gdx_chain_log
             rate0 = cached[s].x;
             sum = qsum[pos];
             events = qevents[pos];
-            if (logs && pos < h1)
-            {
-                for (int k = clog.last[hbase + pos]; k >= 0; k = clog.prev[k])
-                {
-                    const double4 v = clog.part[k];
-                    sum.y += v.x;
-                    sum.z += v.y;
-                    sum.w = fmax(sum.w, v.z);
-                }
-            }
+            if (logs && pos < h1) add_logged(clog, hbase + pos, sum);
         }
         if (take)
         {
@@ -2553,6 +2556,23 @@ __global__ __launch_bounds__(BLOCK) void k_chain_audit(gdx_wave w, gdx_chain_log
     }
     __syncthreads();
     flush_audit(a, G.raw_audit);
+}
+
+// the chain sums that the audit reads and the events of a phase's chained owners, in particle order (test access)
+__global__ __launch_bounds__(BLOCK) void k_chain_sums(gdx_wave w, gdx_chain_log clog, double4 *sums, int *events)
+{
+    int gi, s0, s1;
+    if (!due_block(w, BLOCK, gi, s0, s1)) return;
+    const gdx_gref &G = w.table[w.ref[gi]];
+    const int h1 = w.beg[gi] + *G.hcount, l0 = w.beg[gi] + w.cnt[gi] - *G.qcount;
+    const int pos = s0 + int(threadIdx.x);
+    if (pos >= s1 || (pos >= h1 && pos < l0)) return;
+    double4 sum = G.qsum[pos];
+    if (clog.enabled && w.qprefix[w.n] <= clog.owners && pos < h1)
+        add_logged(clog, w.qprefix[gi] - w.beg[gi] + pos, sum);
+    const int p = G.slot_pidx[G.queue[pos]];
+    sums[p] = sum;
+    events[p] = G.qevents[pos];
 }
 
 __global__ __launch_bounds__(256) void k_cached_to_particles(const double4 *cached, const int *slot_pidx, int n_active,
@@ -2838,6 +2858,14 @@ void launch_chain_audit(hipStream_t st, const gdx_wave &w, int blocks, const run
     if (!blocks) return;
     k_chain_audit<<<xcd_grid(blocks), BLOCK, 0, st>>>(w, rb.log);
     hip_check(hipGetLastError(), "launch chain audit");
+}
+
+// of the run's last chain phase; sums and events cleared by the caller
+void launch_chain_sums(hipStream_t st, const run_buffers &rb, double4 *sums, int *events)
+{
+    if (!rb.chain_blocks) return;
+    k_chain_sums<<<xcd_grid(rb.chain_blocks), BLOCK, 0, st>>>(rb.chain_wave, rb.log, sums, events);
+    hip_check(hipGetLastError(), "launch chain sums");
 }
 
 void launch_gather_cached(context &c, double *out)

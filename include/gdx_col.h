@@ -175,16 +175,25 @@ int gdx_col_reset_controller(gdx_col_handle h);
  * min(duration, horizon) instead of the controller's choice (audits still run); 0 restores the
  * controller. Two operators with the same fixed bath follow the same schedule whatever their rates. */
 int gdx_col_set_fixed_bath(gdx_col_handle h, double duration);
-/* launch shapes, no reference counterpart: refresh waves with at most `owners` due owners rate each
- * plain owner with a group of four lanes and screen one owner per lane, so that the few owners of a small
- * wave spread over the whole GPU; larger waves take one lane per owner and four owners per lane
- * (default GDX_COL_NARROW_OWNERS; 0 always takes the wide shapes, < 0 is rejected). In a batch or an
- * ensemble the first handle's value applies. Results do not depend on it. */
 /* test access, no reference counterpart: on makes the chain pick every partner from the walk's
  * sequential partial sums; off (default) decides each slot from tree-summed partials wherever they are
  * provably on the same side of the target and falls back to the sequential ones otherwise. Results do
  * not depend on it. */
 int gdx_col_set_exact_walk(gdx_col_handle h, int on);
+/* test access, no reference counterpart: how many chunks of 64 waiting intervals beyond an owner's first the
+ * chain's interval logs may take, 0 ... 8192 (default 8192). An owner that gets no more forms its jump moments in
+ * the chain, in another order of sums; states, draws and events are the same. In a batch the first handle's
+ * value applies. */
+int gdx_col_set_chain_log_chunks(gdx_col_handle h, int chunks);
+/* test access, no reference counterpart: the sums {hazard, first and second jump moment, largest jump} (host n x 4,
+ * particle order) and the events of the owners chained in the last chain phase of h's last operator call, 0 for
+ * the others, and the chunks that its logs asked for */
+int gdx_col_get_chain_sums(gdx_col_handle h, double *sums4, int *events, int *asked);
+/* launch shapes, no reference counterpart: refresh waves with at most `owners` due owners rate each
+ * plain owner with a group of four lanes and screen one owner per lane, so that the few owners of a small
+ * wave spread over the whole GPU; larger waves take one lane per owner and four owners per lane
+ * (default GDX_COL_NARROW_OWNERS; 0 always takes the wide shapes, < 0 is rejected). In a batch or an
+ * ensemble the first handle's value applies. Results do not depend on it. */
 #define GDX_COL_NARROW_OWNERS 65536
 int gdx_col_set_narrow_waves(gdx_col_handle h, int owners);
 int gdx_col_synchronize(gdx_col_handle h);

@@ -241,12 +241,12 @@ class CollisionOperator:
         """Test access: chunks beyond an owner's first that the chain's interval logs may take (default all)."""
         self._call(self.lib.gdx_col_set_chain_log_chunks, int(chunks))
 
-    def chain_sums(self) -> tuple[np.ndarray, np.ndarray, int]:
+    def chain_sums(self) -> tuple[np.ndarray, np.ndarray, np.ndarray]:
         """Test access: {hazard, first and second jump moment, largest jump} and events per particle of the last
-        chain phase of the last call, and the log chunks asked for."""
-        sums, events, asked = np.empty((self.n, 4)), np.empty(self.n, np.int32), C.c_int()
-        self._call(self.lib.gdx_col_get_chain_sums, _np_ptr(sums), _np_ptr(events), C.byref(asked))
-        return sums, events, asked.value
+        chain phase of the last call, and the log chunks asked for and reserved."""
+        sums, events, chunks = np.empty((self.n, 4)), np.empty(self.n, np.int32), np.empty(2, np.int32)
+        self._call(self.lib.gdx_col_get_chain_sums, _np_ptr(sums), _np_ptr(events), _np_ptr(chunks))
+        return sums, events, chunks
 
     def set_narrow_waves(self, owners: int) -> None:
         """Refresh waves of at most `owners` due owners take the narrow launch shapes (four lanes per

@@ -740,7 +740,7 @@ void run_swarms(std::vector<op_run *> &runs, run_buffers &rb, hipStream_t st, ke
               "group table");
     hip_check(hipMemsetAsync(rb.counters.p, 0, sizeof(unsigned long long)*GDX_CTRS*nr, st), "zero counters");
     hip_check(hipMemsetAsync(rb.back_d.p + rb.back_bytes, 0, 16, st), "zero read-back count");
-    if (!rb.resident) rb.resident = chain_resident_blocks();
+    prepare_chain(rb);
     for (op_run *r : runs) r->start(st, rb);
     launch_reset_scratch(st, rb.table.p, ng);
     // swarms whose bound scale changed: their table entries again, before the next rate pass
@@ -1585,9 +1585,9 @@ int gdx_col_set_chain_log_chunks(gdx_col_handle h, int chunks)
     });
 }
 
-int gdx_col_get_chain_sums(gdx_col_handle h, double *sums4, int *events, int *asked)
+int gdx_col_get_chain_sums(gdx_col_handle h, double *sums4, int *events, int *chunks2)
 {
-    if (!h || !sums4 || !events || !asked) return GDX_COL_ERR_ARG;
+    if (!h || !sums4 || !events || !chunks2) return GDX_COL_ERR_ARG;
     return guard(&h->c, [&] {
         context &c = h->c;
         run_buffers &rb = h->rb;
@@ -1602,7 +1602,8 @@ int gdx_col_get_chain_sums(gdx_col_handle h, double *sums4, int *events, int *as
         launch_chain_sums(c.stream, rb, sums.p, ev.p);
         copy_d2h(sums4, sums.p, sizeof(double4)*size_t(c.n), c.stream);
         copy_d2h(events, ev.p, sizeof(int)*size_t(c.n), c.stream);
-        copy_d2h(asked, rb.log_next.p, sizeof(int), c.stream);
+        copy_d2h(chunks2, rb.log_next.p, sizeof(int), c.stream);
+        chunks2[1] = int(rb.log_part.n);
         hip_check(hipStreamSynchronize(c.stream), "read chain sums");
     });
 }

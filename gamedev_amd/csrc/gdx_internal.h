@@ -182,16 +182,18 @@ struct run_buffers
     int chain_blocks = 0;
     const context *chain_of = nullptr;
     unsigned long long chain_epoch = 0;
-    void reserve_log(int owners)
+    // before a run's first launch, for the largest grid (`most` owners): growing with the waves would free and
+    // allocate between their launches, and a free waits for the device, other streams' work included
+    void reserve_log(int most)
     {
-        const size_t chunks = size_t(owners) + CHAIN_EXTRA;
+        const size_t chunks = size_t(most) + CHAIN_EXTRA;
         log_entry.alloc(chunks*CHAIN_CHUNK);
         log_part.alloc(chunks);
         log_use.alloc(chunks);
         log_prev.alloc(chunks);
-        log_last.alloc(size_t(owners));
-        log = gdx_chain_log{log_entry.p, log_part.p, log_use.p, log_prev.p, log_last.p, log_next.p, owners,
-                            log_extra, log_phases > 0, hcount.p, qcount.p};
+        log_last.alloc(size_t(most));
+        log = gdx_chain_log{log_entry.p, log_part.p, log_use.p, log_prev.p, log_last.p, log_next.p, most,
+                            log_extra, 0, hcount.p, qcount.p};
     }
     // controller sums, queue lengths, counters and errors of every group and swarm of the run. The
     // read-backs share one device block and one page-locked mirror laid out [raw_rate][wave_ctr][err]
@@ -454,7 +456,7 @@ const void *majorant_pack(gdx_col_majorant m);
 unsigned long long majorant_version(gdx_col_majorant m);
 void invalidate_bounds(context &c);
 void build_reverse(context &c);
-int chain_resident_blocks();
+void prepare_chain(run_buffers &rb);
 void launch_chain(hipStream_t st, const gdx_wave &w, run_buffers &rb, bool own_prefix);
 void launch_chain_audit(hipStream_t st, const gdx_wave &w, int blocks, const run_buffers &rb);
 void launch_chain_sums(hipStream_t st, const run_buffers &rb, double4 *sums, int *events);

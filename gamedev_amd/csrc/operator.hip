@@ -2830,13 +2830,18 @@ void launch_queue_prefix(hipStream_t st, const gdx_wave &w, int *qprefix)
     hip_check(hipGetLastError(), "launch queue prefix");
 }
 
-int chain_resident_blocks()
+// the persistent grid's size and the logs of a run, after size_run
+void prepare_chain(run_buffers &rb)
 {
-    int per_cu = 0, cus = 0, dev = 0;
-    hip_check(hipGetDevice(&dev), "get device");
-    hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_chain, BLOCK, 0), "chain occupancy");
-    hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "CU count");
-    return std::max(1, per_cu*cus);
+    if (!rb.resident)
+    {
+        int per_cu = 0, cus = 0, dev = 0;
+        hip_check(hipGetDevice(&dev), "get device");
+        hip_check(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_chain, BLOCK, 0), "chain occupancy");
+        hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev), "CU count");
+        rb.resident = std::max(1, per_cu*cus);
+    }
+    rb.reserve_log(rb.resident*WAVES / 2);
 }
 
 // after launch_queue_prefix of the same wave unless own_prefix (at most CHAIN_OWN_PREFIX due groups); then the
@@ -2845,7 +2850,8 @@ void launch_chain(hipStream_t st, const gdx_wave &w, run_buffers &rb, bool own_p
 {
     if (!w.total) return;
     const int grid = chain_grid(w, rb.resident);
-    rb.reserve_log(grid*WAVES / 2);
+    rb.log.owners = grid*WAVES / 2;
+    rb.log.enabled = rb.log_phases > 0;
     k_chain<<<grid, BLOCK, 0, st>>>(w, rb.log, own_prefix ? rb.qprefix.p : nullptr);
     hip_check(hipGetLastError(), "launch chain");
     if (!rb.log.enabled) return;

@@ -187,8 +187,9 @@ int gdx_col_set_exact_walk(gdx_col_handle h, int on);
 int gdx_col_set_chain_log_chunks(gdx_col_handle h, int chunks);
 /* test access, no reference counterpart: the sums {hazard, first and second jump moment, largest jump} (host n x 4,
  * particle order) and the events of the owners chained in the last chain phase of h's last operator call, 0 for
- * the others, and the chunks that its logs asked for */
-int gdx_col_get_chain_sums(gdx_col_handle h, double *sums4, int *events, int *asked);
+ * the others; chunks2: the chunks beyond the owners' first that the phase's logs asked for, and those reserved
+ * in all */
+int gdx_col_get_chain_sums(gdx_col_handle h, double *sums4, int *events, int *chunks2);
 /* launch shapes, no reference counterpart: refresh waves with at most `owners` due owners rate each
  * plain owner with a group of four lanes and screen one owner per lane, so that the few owners of a small
  * wave spread over the whole GPU; larger waves take one lane per owner and four owners per lane

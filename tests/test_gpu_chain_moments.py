@@ -25,7 +25,7 @@ def _calls(n, h, gpu, exact=False, chunks=ALL, diagnostics=False):
     for step in range(2):
         print(f"[moments] n={n} exact={exact} chunks={chunks} step {step}", flush=True)
         s = op.evolve(h)
-        sums, events, asked = op.chain_sums()
+        sums, events, (asked, _) = op.chain_sums()
         out.append(dict(calls=(s["events"], s["waves"]), sums=sums, events=events, asked=asked,
                         state=(d["size"].cpu().numpy().tobytes(), d["numr"].cpu().numpy().tobytes(), op.rng().tobytes())))
     return out, op.event_totals() if diagnostics else None

@@ -100,6 +100,7 @@ _SIGS = {
     "gdx_col_host_choose": [P, I, D, D, P],
     "gdx_col_host_finish": [P, I, P, P],
     "gdx_col_host_schedule": [I, D, P, P, I, P, P, P, P],
+    "gdx_col_host_image_distance": [D, D, D, D, D, C.POINTER(C.c_float)],
     "gdx_morton_build": [P, P, I, C.c_float, C.c_float, C.c_float, C.c_float, I, I, I, C.POINTER(P)],
     "gdx_morton_destroy": [P],
     "gdx_morton_node_count": [P, C.POINTER(I)],

@@ -1640,6 +1640,13 @@ int gdx_col_majorant_max_owners(long long *out)
 }
 
 // ---- host controller and scheduler ----
+int gdx_col_host_image_distance(double x_min, double x_max, double y_min, double z_min, double z_max, float *out)
+{
+    if (!out) return GDX_COL_ERR_ARG;
+    *out = image_distance(x_min, x_max, y_min, z_min, z_max);
+    return GDX_COL_OK;
+}
+
 int gdx_col_host_binmap(const int *raw_count, int raw_bins, int *raw_to_merged, int *merged)
 {
     if (!raw_count || !raw_to_merged || !merged || raw_bins <= 0 || raw_bins % COL_BIN_S) return GDX_COL_ERR_ARG;

@@ -5,6 +5,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cfloat>
+#include <cmath>
 #include <cstddef>
 #include <cstdint>
 #include <stdexcept>
@@ -289,6 +292,19 @@ struct morton_index
     int node_count = 0;
     int leaf_count = 0;
 };
+
+// A distance that no two images of one particle lie nearer to each other than: they are rotated by the wedge's
+// width from each other, or, the two ghosts, by twice that. The records are FP32: the width is the one that the
+// rotation uses, and a ghost's coordinate, two rounded products of a rounded sine and cosine and their sum, is off by
+// up to 5 half ulps of the radius R, so a pair of ghosts by up to 7.1 FLT_EPSILON R. 10 of them are taken off; in
+// a wedge as narrow as that rounding the distance is zero and every list goes through the removal.
+inline float image_distance(double x_min, double x_max, double y_min, double z_min, double z_max)
+{
+    const double width = static_cast<float>(x_max) - static_cast<float>(x_min);
+    const double turn = std::fmin(std::fabs(std::sin(0.5*width)), std::fabs(std::sin(width)));
+    const double chord = std::fmax(2.0*turn - 10.0*FLT_EPSILON, 0.0);
+    return static_cast<float>(y_min*std::fmax(std::fmin(std::sin(z_min), std::sin(z_max)), 0.0)*chord);
+}
 
 // what the host reads of a geometry epoch
 constexpr int SLOT_BINS = 128;

@@ -1441,15 +1441,6 @@ void knn_query(const morton_index &ix, const float4 *queries, int nq, int k, int
     hip_check(hipGetLastError(), "launch knn");
 }
 
-// the least distance any two images of one particle can have: rotated by the wedge's width from each
-// other, or, the two ghosts, by twice that
-static float image_distance()
-{
-    const double width = static_cast<double>(X_MAX) - static_cast<double>(X_MIN);
-    const double turn = std::fmin(std::fabs(std::sin(0.5*width)), std::fabs(std::sin(width)));
-    return static_cast<float>(2.0*Y_MIN*std::fmin(std::sin(Z_MIN), std::sin(Z_MAX))*turn);
-}
-
 // the largest search cap and the unique-identifier test of swarm_runtime.cu:331-340, 413-415
 static void wedge_cap(context &c)
 {
@@ -1585,7 +1576,7 @@ void geometry_epoch(context &c)
     {
         int waves = blocks_for(nr, WAVE);
         if (X_WEDGE) c.nbr_image.alloc(na*N_K);
-        const float image_d2 = X_WEDGE ? image_distance()*image_distance() : 0.0f;
+        const float image_dist = image_distance(X_MIN, X_MAX, Y_MIN, Z_MIN, Z_MAX), image_d2 = image_dist*image_dist;
 #define GDX_TOPK_SHAPED(DEDUP, TILE, WPB)                                                                    \
     k_col_topk<DEDUP, TILE, WPB><<<xcd_grid(blocks_for(waves, WPB)), WPB*WAVE, 0, st>>>(                     \
         c.index.rec.p, c.index.boxes.p, c.index.chunks.p, nr, c.index.idx.p, c.pts.p, c.pidx_slot.p,         \

@@ -272,6 +272,11 @@ int gdx_col_host_schedule_adaptive(int n, double horizon, const double *requeste
                                    int max_waves, const double *wave_requested, const unsigned char *wave_passed,
                                    unsigned long long *ticks, int *due_counts, int *wave_levels, int *waves);
 
+/* a distance that no two images of one particle in a wedge of these limits lie nearer to each other than, as the
+ * search's FP32 records place them: lists that do not reach across it need no image removal. No reference
+ * counterpart. */
+int gdx_col_host_image_distance(double x_min, double x_max, double y_min, double z_min, double z_max, float *out);
+
 /* ---- stand-alone adaptive Morton index: morton_index::build / view (inc/swarm/morton/morton_index.cuh:160-293) ---- */
 typedef struct gdx_morton_ctx *gdx_morton_handle;
 /* points: device float4 {x, y, z, unused} x n; active: device flags or NULL */

@@ -1639,6 +1639,19 @@ int gdx_col_majorant_max_owners(long long *out)
     return GDX_COL_OK;
 }
 
+int gdx_col_check_arithmetic(long long n, const double *a, const double *b, double *device8, double *host3)
+{
+    if (n <= 0 || n > INT_MAX || !a || !b || !device8) return GDX_COL_ERR_ARG;
+    return guard(nullptr, [&] { check_arithmetic(a, b, n, device8, host3); });
+}
+
+int gdx_col_check_solo_rates(int owners, const double *owner5, const double *slots3, double *rates, double *speeds,
+                             int *route)
+{
+    if (owners <= 0 || !owner5 || !slots3 || !rates || !speeds || !route) return GDX_COL_ERR_ARG;
+    return guard(nullptr, [&] { check_solo_rates(owners, owner5, slots3, rates, speeds, route); });
+}
+
 // ---- host controller and scheduler ----
 int gdx_col_host_image_distance(double x_min, double x_max, double y_min, double z_min, double z_max, float *out)
 {

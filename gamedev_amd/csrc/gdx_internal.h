@@ -475,6 +475,8 @@ void build_reverse(context &c);
 void prepare_chain(run_buffers &rb);
 void launch_chain(hipStream_t st, const gdx_wave &w, run_buffers &rb, bool own_prefix);
 void launch_chain_audit(hipStream_t st, const gdx_wave &w, int blocks, const run_buffers &rb);
+void check_arithmetic(const double *a, const double *b, long long n, double *device8, double *host3);
+void check_solo_rates(int owners, const double *owner5, const double *slots3, double *rates, double *speeds, int *route);
 void launch_chain_sums(hipStream_t st, const run_buffers &rb, double4 *sums, int *events);
 void launch_event_sum(context &c, hipStream_t st);
 void launch_gather_cached(context &c, double *out_particle_order);

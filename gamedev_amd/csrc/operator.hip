@@ -1703,7 +1703,8 @@ __device__ __forceinline__ double solo_vrel_t(double ris, double vg_sq, double s
     return vrel_t_merged(ris, vg_sq, stokes_i, stokes_j);
 }
 
-// eval_pair_rate, bit for bit, by selects; the sticking packet only where some lane has one above 1
+// eval_pair_rate, bit for bit (tests/test_gpu_pair_arithmetic.py), by selects; the sticking packet only where some
+// lane has one above 1
 __device__ __forceinline__ double solo_pair_rate(const owner_terms &t, const solo_partner &s, double lambda_0, double &vrel)
 {
     const double size_i = t.size_i, size_j = s.q.size_j, numr_j = s.q.numr_j;
@@ -1753,6 +1754,55 @@ __device__ __forceinline__ double solo_pair_rate(const owner_terms &t, const sol
     if constexpr (CAN_FRAGMENT) factor = high ? (q <= 0.1 ? remnant + q : 1.0) : low_factor;
     r *= factor;
     return s.has ? r : 0.0;
+}
+
+// ---- test access to the forms that exist on the device only ----
+__global__ __launch_bounds__(BLOCK) void k_check_arithmetic(const double *a, const double *b, long long n, double *out)
+{
+    __shared__ log_entry logs[LOG_CELLS];
+    copy_log_table(logs, BLOCK);
+    __syncthreads();
+    const long long i = (long long)blockIdx.x*BLOCK + threadIdx.x;
+    if (i >= n) return;
+    const double x = a[i], y = b[i];
+    const double v[8] = {quot(x, y), quot_any(x, y), recip(y), root(x), ulog1p_finite(x, log_source{logs}),
+                         ulog(y, log_source{logs}), ulog1p(x), ulog(y)};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) out[k*n + i] = v[k];
+}
+
+// per owner, a wavefront each: solo_pair_rate beside eval_pair_rate with and without held partner factors; route: 1
+// where the lanes share regimes 4 and 5, 2 where they share regime 6, plus 4 with a sticking packet
+__global__ __launch_bounds__(WAVE) void k_check_solo_rates(const double *owner, const double *slots, int owners,
+                                                          double *rates, double *speeds, int *route)
+{
+    const int o = blockIdx.x, k = threadIdx.x % N_K;
+    const double *me = owner + 5ll*o, *slot = slots + 3ll*((long long)o*N_K + k);
+    gdx_env e{};
+    if constexpr (COAG_KERNEL == 3) e = make_env(me[0], me[1]);
+    const double lambda_0 = me[4];
+    const owner_terms t = make_owner(e, me[2], me[3], slots[3ll*o*N_K + 2]);
+    const partner q{slot[0], slot[1], slot[2], slot[1] >= 0.0};
+    const solo_partner s = make_solo_partner(t, q);
+    double vrel;
+    const double rate = solo_pair_rate(t, s, lambda_0, vrel);
+    const pair_term p = eval_pair_rate(t, q, lambda_0), h = eval_pair_rate<true>(t, q, lambda_0, s.pt);
+    int r = 0;
+    if constexpr (COAG_KERNEL == 3)
+    {
+        const double sl = fmax(t.si, s.pt.sj);
+        if (__ballot(sl < 5.0*t.ris) == 0ull) r = __ballot(sl < 1.0) == ~0ull ? 1 : (__ballot(sl < 1.0) == 0ull ? 2 : 0);
+    }
+    const double ratio = div_rn(q.size_j, t.size_i, t.inv_size), cube = ratio*ratio*ratio;
+    if (__ballot(cube > 0.0 && cube <= 1.0e-06)) r |= 4;
+    if (threadIdx.x == 0) route[o] = r;
+    if (threadIdx.x >= N_K) return;
+    const long long at = (long long)o*N_K + k, all = (long long)owners*N_K;
+    rates[at] = rate;
+    rates[all + at] = p.rate;
+    rates[2*all + at] = h.rate;
+    speeds[at] = vrel;
+    speeds[all + at] = p.vrel;
 }
 
 // event chains (col_chain_run.cu:127-382): a persistent grid over the queued owners. Each K-lane segment
@@ -2864,6 +2914,44 @@ void launch_chain_audit(hipStream_t st, const gdx_wave &w, int blocks, const run
     if (!blocks) return;
     k_chain_audit<<<xcd_grid(blocks), BLOCK, 0, st>>>(w, rb.log);
     hip_check(hipGetLastError(), "launch chain audit");
+}
+
+// host arrays: device8 as k_check_arithmetic leaves them, host3 the host's ulog1p_finite(a), ulog(b), ulog1p(a)
+void check_arithmetic(const double *a, const double *b, long long n, double *device8, double *host3)
+{
+    dbuf<double> in, out;
+    in.alloc(size_t(2*n));
+    out.alloc(size_t(8*n));
+    hip_check(hipMemcpy(in.p, a, sizeof(double)*size_t(n), hipMemcpyHostToDevice), "operands");
+    hip_check(hipMemcpy(in.p + n, b, sizeof(double)*size_t(n), hipMemcpyHostToDevice), "operands");
+    k_check_arithmetic<<<unsigned((n + BLOCK - 1) / BLOCK), BLOCK>>>(in.p, in.p + n, n, out.p);
+    hip_check(hipGetLastError(), "launch arithmetic check");
+    hip_check(hipMemcpy(device8, out.p, sizeof(double)*size_t(8*n), hipMemcpyDeviceToHost), "arithmetic check");
+    for (long long i = 0; host3 && i < n; ++i)
+    {
+        host3[i] = ulog1p_finite(a[i]);
+        host3[n + i] = ulog(b[i]);
+        host3[2*n + i] = ulog1p(a[i]);
+    }
+}
+
+void check_solo_rates(int owners, const double *owner5, const double *slots3, double *rates, double *speeds, int *route)
+{
+    const size_t all = size_t(owners)*N_K;
+    dbuf<double> own, slots, r, v;
+    dbuf<int> way;
+    own.alloc(size_t(5)*owners);
+    slots.alloc(3*all);
+    r.alloc(3*all);
+    v.alloc(2*all);
+    way.alloc(size_t(owners));
+    hip_check(hipMemcpy(own.p, owner5, sizeof(double)*size_t(5)*owners, hipMemcpyHostToDevice), "owners");
+    hip_check(hipMemcpy(slots.p, slots3, sizeof(double)*3*all, hipMemcpyHostToDevice), "partners");
+    k_check_solo_rates<<<owners, WAVE>>>(own.p, slots.p, owners, r.p, v.p, way.p);
+    hip_check(hipGetLastError(), "launch solo rate check");
+    hip_check(hipMemcpy(rates, r.p, sizeof(double)*3*all, hipMemcpyDeviceToHost), "solo rate check");
+    hip_check(hipMemcpy(speeds, v.p, sizeof(double)*2*all, hipMemcpyDeviceToHost), "solo rate check");
+    hip_check(hipMemcpy(route, way.p, sizeof(int)*size_t(owners), hipMemcpyDeviceToHost), "solo rate check");
 }
 
 // of the run's last chain phase; sums and events cleared by the caller

@@ -254,6 +254,18 @@ int gdx_col_rate_pass(gdx_col_handle h);
  * first, so the reservoir is published from the owners' states. */
 int gdx_col_pair_rates(gdx_col_handle h, double *rates);
 
+/* ---- the kernels' own arithmetic on given operands (host arrays); test access, no reference counterpart ---- */
+/* device8, n each: a/b by the form for finite operands, by the form for any, 1/b, sqrt(a), log1p(a) (finite a > -1)
+ * and log(b) with the table in LDS, log1p(a) and log(b) for any operand; host3 (may be NULL), n each: the host's
+ * log1p(a) for finite a, log(b), log1p(a) */
+int gdx_col_check_arithmetic(long long n, const double *a, const double *b, double *device8, double *host3);
+/* owner5: {y, z, size, measure, lambda_0} per owner; slots3: {size, number (negative: empty), scale height} per owner
+ * and neighbour slot; rates, one per slot each: as the chain's solo loop, the rate pass and the general loop with held
+ * partner factors form them; speeds: as the first two; route per owner: 1 all partners in turbulence regimes 4
+ * and 5, 2 all in regime 6, plus 4 with a sticking packet */
+int gdx_col_check_solo_rates(int owners, const double *owner5, const double *slots3, double *rates, double *speeds,
+                             int *route);
+
 /* ---- host controller and scheduler, callable without a GPU (same code the operator runs) ---- */
 /* _build_col_binmap (inc/swarm/_col_bound.cuh:45-98): returns the merged-bin count */
 int gdx_col_host_binmap(const int *raw_count, int raw_bins, int *raw_to_merged, int *merged);

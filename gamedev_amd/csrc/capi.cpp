@@ -740,7 +740,6 @@ void run_swarms(std::vector<op_run *> &runs, run_buffers &rb, hipStream_t st, ke
               "group table");
     hip_check(hipMemsetAsync(rb.counters.p, 0, sizeof(unsigned long long)*GDX_CTRS*nr, st), "zero counters");
     hip_check(hipMemsetAsync(rb.back_d.p + rb.back_bytes, 0, 16, st), "zero read-back count");
-    prepare_chain(rb);
     for (op_run *r : runs) r->start(st, rb);
     launch_reset_scratch(st, rb.table.p, ng);
     // swarms whose bound scale changed: their table entries again, before the next rate pass
@@ -757,6 +756,12 @@ void run_swarms(std::vector<op_run *> &runs, run_buffers &rb, hipStream_t st, ke
     };
     std::vector<phase_entry> e;
     std::vector<op_run *> now;
+    // the chain's pool, allocated by a handle's first run while the GPU rates
+    bool prepared = false;
+    auto prepare = [&] {
+        if (!prepared) prepare_chain(rb);
+        prepared = true;
+    };
     while (true)
     {
         bool work = false;
@@ -783,6 +788,7 @@ void run_swarms(std::vector<op_run *> &runs, run_buffers &rb, hipStream_t st, ke
                 launch_bath_rate_grouped(st, pw.wlsub, pw.blocks_lsub);
             });
             rb.read_back(rb.off_rate, rb.off_err, st);             // rate bins and wave counters
+            prepare();
             wait_results(rb, st, "rating pass");
             for (op_run *r : now) r->after_rate();
             upload_changed(now);
@@ -795,6 +801,7 @@ void run_swarms(std::vector<op_run *> &runs, run_buffers &rb, hipStream_t st, ke
         if (!now.empty())
         {
             work = true;
+            prepare();
             zero_ranges z;
             z.add(rb.raw_audit.p, sizeof(gdx_raw_audit)*COL_BIN_S*ng);
             z.add(rb.err.p, sizeof(int)*nr);
@@ -1603,7 +1610,7 @@ int gdx_col_get_chain_sums(gdx_col_handle h, double *sums4, int *events, int *ch
         copy_d2h(sums4, sums.p, sizeof(double4)*size_t(c.n), c.stream);
         copy_d2h(events, ev.p, sizeof(int)*size_t(c.n), c.stream);
         copy_d2h(chunks2, rb.log_next.p, sizeof(int), c.stream);
-        chunks2[1] = int(rb.log_part.n);
+        chunks2[1] = rb.log_chunks;
         hip_check(hipStreamSynchronize(c.stream), "read chain sums");
     });
 }

@@ -169,15 +169,15 @@ struct run_buffers
     dbuf<int> nchanged;               // entries of each changed-slot list
     int changed_cap = 0;              // entries each changed-slot list can hold
     int resident = 0;                 // resident blocks of the persistent chain kernel
-    // the solo heavy owners' logs of one chain launch (gdx_chain_log)
+    // the solo heavy owners' logs of one chain launch (gdx_chain_log), their pool one allocation
     gdx_chain_log log{};
-    dbuf<double2> log_entry;
-    dbuf<double4> log_part;
-    dbuf<int4> log_use;
-    dbuf<int> log_prev, log_last, log_next;
+    dbuf<unsigned char> log_pool;
+    dbuf<int> log_next;
+    int log_chunks = 0;
     // chain phases that keep logs still to come after a chain of LONG_CHAIN events (CHAIN_LOG_PHASES each
-    // time). The logs cost a launch; without them a long chain costs its owner's moments at every event. The
-    // results do not depend on it.
+    // time). The logs cost a launch; without them a long chain costs its owner's moments at every event. A bath's
+    // states, draws and events do not depend on it; the jump-moment sums that the audit takes are added in another
+    // order, so their last bits do (the audit adds them by atomics, in no order either).
     int log_phases = CHAIN_LOG_PHASES;
     int log_extra = CHAIN_EXTRA;      // chunks beyond the owners' first that the logs may take
     // the last chain phase of the last run, if that was of one swarm (test access)
@@ -185,17 +185,19 @@ struct run_buffers
     int chain_blocks = 0;
     const context *chain_of = nullptr;
     unsigned long long chain_epoch = 0;
-    // before a run's first launch, for the largest grid (`most` owners): growing with the waves would free and
+    // before a run's first chain, for the largest grid (`most` owners): growing with the waves would free and
     // allocate between their launches, and a free waits for the device, other streams' work included
     void reserve_log(int most)
     {
-        const size_t chunks = size_t(most) + CHAIN_EXTRA;
-        log_entry.alloc(chunks*CHAIN_CHUNK);
-        log_part.alloc(chunks);
-        log_use.alloc(chunks);
-        log_prev.alloc(chunks);
-        log_last.alloc(size_t(most));
-        log = gdx_chain_log{log_entry.p, log_part.p, log_use.p, log_prev.p, log_last.p, log_next.p, most,
+        log_chunks = most + CHAIN_EXTRA;
+        const size_t chunks = size_t(log_chunks);
+        log_pool.alloc(chunks*(CHAIN_CHUNK*sizeof(double2) + sizeof(double4) + sizeof(int4) + sizeof(int))
+                       + sizeof(int)*size_t(most));
+        double4 *const part = reinterpret_cast<double4 *>(log_pool.p);
+        double2 *const entry = reinterpret_cast<double2 *>(part + chunks);
+        int4 *const use = reinterpret_cast<int4 *>(entry + chunks*CHAIN_CHUNK);
+        int *const prev = reinterpret_cast<int *>(use + chunks);
+        log = gdx_chain_log{entry, part, use, prev, prev + chunks, log_next.p, most,
                             log_extra, 0, hcount.p, qcount.p};
     }
     // controller sums, queue lengths, counters and errors of every group and swarm of the run. The
@@ -432,11 +434,11 @@ void morton_build(morton_index &ix, const float4 *points, const unsigned char *a
 void geometry_epoch(context &c);
 void load_state(context &c);
 void store_state(context &c);
-// test access: exact top-K over a built index for arbitrary queries and a runtime K
 void sort_keys(dbuf<uint64_t> &keys, dbuf<int> &idx, int n, int bits, bool flat, sort_scratch &s, hipStream_t st);
 void write_nodes(morton_index &ix, hipStream_t st);
 const unsigned int *morton_total(const morton_index &ix);
 void morton_settle(morton_index &ix, unsigned int total, hipStream_t st);
+// test access: exact top-K over a built index for arbitrary queries and a runtime K
 void knn_query(const morton_index &ix, const float4 *queries, int nq, int k, int *codes, float *d2,
                unsigned int *overflow, hipStream_t st);
 
@@ -461,7 +463,6 @@ constexpr int CHAIN_OWN_PREFIX = 256;
 void launch_queue_prefix(hipStream_t st, const gdx_wave &w, int *qprefix);
 void launch_majorant(hipStream_t st, const gdx_wave &w, int blocks);
 void launch_zero(hipStream_t st, const zero_ranges &z);
-// bytes (a multiple of 16) from device memory into page-locked host memory by a kernel on the stream
 // the ranges cleared and `bytes` of host data (multiple of 4) written to dst by one launch: the data ride
 // in the kernel's arguments when they fit (STAGE_INLINE_BYTES), else a zero launch and a copy
 constexpr int STAGE_INLINE_BYTES = 3072;

@@ -79,8 +79,8 @@ __device__ __forceinline__ double col_uniform(uint32_t pidx, uint64_t seed, uint
 // operand nor quotient nor remainder leaves the normal range, |b| within 2^+-1021 and |a| above 2^-960.
 // tests/test_gpu_pair_arithmetic.py compares them with IEEE division and square root over 2^24 random operand pairs
 // of exponents up to +-480, all-ones and all-zero mantissas among them: no bit differs. On the host they are the
-// operators. With them the rate pass at 1e7 owners (K = 32) fell from 378 to 325 vector instructions a pair, 1.70 to 1.48 ms
-// a launch.
+// operators. With them the rate pass at 1e7 owners (K = 32) fell from 378 to 325 vector instructions a pair, 1.70 to
+// 1.48 ms a launch.
 #ifdef __HIP_DEVICE_COMPILE__
 __device__ __forceinline__ double near_recip(double b)
 {
@@ -419,15 +419,19 @@ GDX_FN double ball_measure(double y, double z, double radius)
 // logarithms of the pair outcome moments, table-driven (Tang, ACM TOMS 16, 1990): 1 + x = 2^k z with z in
 // [0.703125, 1.40625), r = z inv - 1 by one fused operation with the reciprocal `inv` of the middle of z's
 // cell, |r| <= 2^-8, and log(1 + x) = (k ln 2 - log inv) + log(1 + r), the first sum exact in its leading part,
-// the second the Taylor series to r^7 (its remainder is below 2^-59 of it). Around 1 the cells have inv = 1,
-// so that small x keep their accuracy. Branch-free (every lane runs one instruction stream), at most 0.75 ulp
-// off and misrounded once in 200 at worst; 34 instructions and a table read, which the pair kernels make from
-// LDS, against 77 for fdlibm's division and degree-14 polynomial (at most 0.86 ulp, misrounded once in eight
-// between 1 and 2). The rates of 5.5e6 owners of the physical kernel: 1.43 -> 1.31 ms; of 75e6 of the constant
-// one, whose partner loads bound it: 9.8 -> 9.2 ms.
+// the second the Taylor series to r^7, the next term's share spread over r^6 (what remains is below 2^-62 of it).
+// The reciprocals are short, 9 fractional bits, so that r is exact for z > 1 and off by 2^-63 at most below: with
+// 11 bits its rounding cost up to 0.25 ulp near 1. In the two cells at 1 inv = 1, so that small x keep their
+// accuracy. Branch-free (every lane runs one instruction stream), within 0.51 ulp from |x| = 1e-6 on and misrounded once
+// in 1,000 at worst (around |x| = 1e-16, where what 1 + x rounds away is as large as x, 0.66 ulp); 34 instructions
+// and a table read, which the pair kernels make from LDS, against 77 for fdlibm's division and degree-14 polynomial
+// (at most 0.86 ulp, misrounded once in eight between 1 and 2). The rates of 5.5e6 owners of the physical kernel:
+// 1.43 -> 1.31 ms; of 75e6 of the constant one, whose partner loads bound it: 9.8 -> 9.2 ms.
 // ---------------------------------------------------------------------------------------------
 constexpr double LN2_HI = 6.93147180369123816490e-01;   // 32 significant bits: k LN2_HI + hi is exact
 constexpr double LN2_LO = 1.90821492927058770002e-10;
+// r^8 / 8 ~ LOG_EIGHTH r^6 for |r| <= 2^-8: the factor of 2^-16 / 8 that makes the larger of both ends' errors least
+constexpr double LOG_EIGHTH = 0.923*0x1p-16 / 8.0;
 
 struct log_entry
 {
@@ -504,7 +508,7 @@ GDX_FN double log_kernel(double u, double e, int k0, const log_source &table)
     double l = (y - h) + r;
     const double c = ldexp(e, -k)*inv;                   // e / u = c / (1 + r)
     l += fma(-c, r, c) + fma(dk, LN2_LO, static_cast<double>(cell.lo));
-    double p = fma_const(r, 1.0 / 7.0, -1.0 / 6.0);
+    double p = fma_const(r, 1.0 / 7.0, -1.0 / 6.0 - LOG_EIGHTH);
     p = fma_const(r, p, 1.0 / 5.0);
     p = fma_const(r, p, -1.0 / 4.0);
     p = fma_const(r, p, 1.0 / 3.0);

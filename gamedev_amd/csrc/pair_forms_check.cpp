@@ -83,31 +83,49 @@ double ulp_error(double y, long double t)
     return static_cast<double>(std::fabs(static_cast<long double>(y) - t) / ulp);
 }
 
+// the lower end of one of the logarithm's LOG_CELLS cells, [0.703125, 1.40625)
+double cell_border(lcg &g)
+{
+    const uint64_t b = uint64_t(0x3fe68000 + (int(g.next()*LOG_CELLS) << 12)) << 32;
+    double v;
+    std::memcpy(&v, &b, sizeof v);
+    return v;
+}
+
 int check_logs(long long trials, lcg &g)
 {
     double worst1 = 0.0, worst2 = 0.0, x1 = 0.0, x2 = 0.0;
+    double pair_worst = 0.0;             // over the arguments that the outcome moments take: 1e-6 <= |x|
     long long differ1 = 0, differ2 = 0;
     for (long long n = 0; n < trials; ++n)
     {
-        // log1p arguments: tiny to huge magnitudes of both signs above -1, and the reduction edges
+        // log1p arguments: tiny to huge magnitudes of both signs above -1, the octave's ends 0.703125 and 1.40625,
+        // the cells around 1 (reciprocal 1) and the borders of any cell
         double x;
         double r = g.next();
         if (r < 0.3) x = std::ldexp(g.next(), -int(60*g.next()));
         else if (r < 0.5) x = -std::ldexp(g.next(), -int(60*g.next()));
         else if (r < 0.7) x = -0.3 + 0.75*g.next();
-        else if (r < 0.8) x = std::sqrt(0.5) - 1.0 + (g.next() - 0.5)*1e-6;
-        else if (r < 0.9) x = std::sqrt(2.0) - 1.0 + (g.next() - 0.5)*1e-6;
+        else if (r < 0.75) x = (g.next() < 0.5 ? 0.703125 : 1.40625) - 1.0 + (g.next() - 0.5)*1e-6;
+        else if (r < 0.8) x = (g.next() - 0.5)*(2.0/128);
+        else if (r < 0.9) x = cell_border(g)*std::ldexp(1.0, int(20*g.next()) - 10)*(1.0 + (g.next() - 0.5)*0x1p-46) - 1.0;
         else x = std::pow(10.0, 300.0*g.next());
         double y = ulog1p(x);
         double err = ulp_error(y, log1pl(static_cast<long double>(x)));
         if (err > worst1) { worst1 = err; x1 = x; }
+        if (std::fabs(x) >= 1e-6) pair_worst = std::fmax(pair_worst, err);
+        const double near = (g.next() < 0.5 ? -1.0 : 1.0)*std::pow(10.0, -6.0 + 5.0*g.next());   // q or Gp q
+        pair_worst = std::fmax(pair_worst, ulp_error(ulog1p(near), log1pl(static_cast<long double>(near))));
         differ1 += y != std::log1p(x);
-        // log arguments: mass ratios over the whole normal range
+        // log arguments: mass ratios over the whole normal range, and cell borders
         double q = std::pow(10.0, -300.0 + 600.0*g.next());
+        if (g.next() < 0.2) q = cell_border(g)*std::ldexp(1.0, int(20*g.next()) - 10)*(1.0 + (g.next() - 0.5)*0x1p-46);
         double yq = ulog(q);
         double eq = ulp_error(yq, logl(static_cast<long double>(q)));
         if (eq > worst2) { worst2 = eq; x2 = q; }
         differ2 += yq != std::log(q);
+        const double ratio = 1.0 - 0.1*std::pow(g.next(), 4.0);
+        pair_worst = std::fmax(pair_worst, std::fmax(eq, ulp_error(ulog(ratio), logl(static_cast<long double>(ratio)))));
     }
     bool special = ulog1p(0.0) == 0.0 && std::isinf(ulog1p(-1.0)) && ulog1p(-1.0) < 0 && std::isnan(ulog1p(-2.0))
         && std::isnan(ulog1p(__builtin_nan(""))) && std::isinf(ulog1p(__builtin_inf())) && ulog1p(1e-300) == 1e-300
@@ -115,6 +133,7 @@ int check_logs(long long trials, lcg &g)
     std::printf("log1p worst_ulp %.4f at %.17g differs_from_libm %lld\n", worst1, x1, differ1);
     std::printf("log worst_ulp %.4f at %.17g differs_from_libm %lld\n", worst2, x2, differ2);
     std::printf("special %d\n", int(special));
+    std::printf("pair_arguments worst %.4f\n", pair_worst);
     return (worst1 < 1.0 && worst2 < 1.0 && special) ? 0 : 1;
 }
 

@@ -98,6 +98,7 @@ _SIGS = {
     "gdx_col_rate_pass": [P],
     "gdx_col_check_arithmetic": [C.c_longlong, P, P, P, P],
     "gdx_col_check_solo_rates": [I, P, P, P, P, P],
+    "gdx_col_check_reverse": [I, P, P, P, P],
     "gdx_col_host_binmap": [P, I, P, P],
     "gdx_col_host_choose": [P, I, D, D, P],
     "gdx_col_host_finish": [P, I, P, P],

@@ -1659,6 +1659,16 @@ int gdx_col_check_solo_rates(int owners, const double *owner5, const double *slo
     return guard(nullptr, [&] { check_solo_rates(owners, owner5, slots3, rates, speeds, route); });
 }
 
+int gdx_col_check_reverse(int n, const int *nbr, unsigned int *beg, unsigned int *end, int *rev)
+{
+    if (n <= 0 || !nbr || !beg || !end || !rev) return GDX_COL_ERR_ARG;
+    return guard(nullptr, [&] {
+        for (long long i = 0; i < (long long)n*N_K; ++i)
+            require(nbr[i] >= -1 && nbr[i] < n, GDX_COL_ERR_ARG, "neighbour slot out of range");
+        check_reverse(nbr, n, beg, end, rev);
+    });
+}
+
 // ---- host controller and scheduler ----
 int gdx_col_host_image_distance(double x_min, double x_max, double y_min, double z_min, double z_max, float *out)
 {

@@ -473,6 +473,7 @@ const void *majorant_pack(gdx_col_majorant m);
 unsigned long long majorant_version(gdx_col_majorant m);
 void invalidate_bounds(context &c);
 void build_reverse(context &c);
+void check_reverse(const int *nbr, int n, unsigned *beg, unsigned *end, int *rev);
 void prepare_chain(run_buffers &rb);
 void launch_chain(hipStream_t st, const gdx_wave &w, run_buffers &rb, bool own_prefix);
 void launch_chain_audit(hipStream_t st, const gdx_wave &w, int blocks, const run_buffers &rb);

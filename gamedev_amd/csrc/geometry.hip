@@ -1728,6 +1728,38 @@ __global__ __launch_bounds__(REV_BLOCK) void k_reverse(const int *nbr, int n, in
     }
 }
 
+// the lists of n > 0 owners' rows: slot j's owners are rev[beg[j] ... end[j])
+static void reverse_lists(const int *nbr, int n, unsigned *beg, unsigned *end, int *rev, sort_scratch &s, hipStream_t st)
+{
+    const int owners = n >= 256*REV_OWNERS ? REV_OWNERS : REV_OWNERS_SMALL, blocks = blocks_for(n, owners);
+    hip_check(hipMemsetAsync(end, 0, sizeof(unsigned)*size_t(n), st), "zero reverse counts");
+    k_reverse<false><<<blocks, REV_BLOCK, 0, st>>>(nbr, n, owners, end, nullptr);
+    hip_check(hipGetLastError(), "launch reverse count");
+    scan_exclusive_u32(end, beg, n, s, st);
+    hip_check(hipMemcpyAsync(end, beg, sizeof(unsigned)*size_t(n), hipMemcpyDeviceToDevice, st), "reverse cursors");
+    // after the fill each cursor is the end of its slot's list
+    k_reverse<true><<<blocks, REV_BLOCK, 0, st>>>(nbr, n, owners, end, rev);
+    hip_check(hipGetLastError(), "launch reverse fill");
+}
+
+// the lists of given rows (host arrays, nbr and rev n x N_K; test access)
+void check_reverse(const int *nbr, int n, unsigned *beg, unsigned *end, int *rev)
+{
+    dbuf<int> rows, lists;
+    dbuf<unsigned> from, to;
+    sort_scratch s;
+    const size_t entries = size_t(n)*N_K;
+    rows.alloc(entries);
+    lists.alloc(entries);
+    from.alloc(size_t(n));
+    to.alloc(size_t(n));
+    hip_check(hipMemcpy(rows.p, nbr, sizeof(int)*entries, hipMemcpyHostToDevice), "rows");
+    reverse_lists(rows.p, n, from.p, to.p, lists.p, s, nullptr);
+    hip_check(hipMemcpy(beg, from.p, sizeof(unsigned)*size_t(n), hipMemcpyDeviceToHost), "reverse lists");
+    hip_check(hipMemcpy(end, to.p, sizeof(unsigned)*size_t(n), hipMemcpyDeviceToHost), "reverse lists");
+    hip_check(hipMemcpy(rev, lists.p, sizeof(int)*entries, hipMemcpyDeviceToHost), "reverse lists");
+}
+
 void build_reverse(context &c)
 {
     const int n = c.n_active;
@@ -1735,23 +1767,10 @@ void build_reverse(context &c)
         throw status_error(GDX_COL_ERR_ARG, "a swarm with a majorant holds at most " + std::to_string(MAJORANT_MAX_OWNERS)
                                             + " active owners (32-bit reverse neighbour offsets)");
     const size_t na = size_t(std::max(1, n));
-    hipStream_t st = c.stream;
     c.rev_beg.alloc(na);
     c.rev_end.alloc(na);
     c.rev.alloc(na*N_K);
-    if (n > 0)
-    {
-        const int owners = n >= 256*REV_OWNERS ? REV_OWNERS : REV_OWNERS_SMALL, blocks = blocks_for(n, owners);
-        hip_check(hipMemsetAsync(c.rev_end.p, 0, sizeof(unsigned)*na, st), "zero reverse counts");
-        k_reverse<false><<<blocks, REV_BLOCK, 0, st>>>(c.nbr.p, n, owners, c.rev_end.p, nullptr);
-        hip_check(hipGetLastError(), "launch reverse count");
-        scan_exclusive_u32(c.rev_end.p, c.rev_beg.p, n, c.scratch, st);
-        hip_check(hipMemcpyAsync(c.rev_end.p, c.rev_beg.p, sizeof(unsigned)*na, hipMemcpyDeviceToDevice, st),
-                  "reverse cursors");
-        // after the fill each cursor is the end of its slot's list
-        k_reverse<true><<<blocks, REV_BLOCK, 0, st>>>(c.nbr.p, n, owners, c.rev_end.p, c.rev.p);
-        hip_check(hipGetLastError(), "launch reverse fill");
-    }
+    if (n > 0) reverse_lists(c.nbr.p, n, c.rev_beg.p, c.rev_end.p, c.rev.p, c.scratch, c.stream);
     c.rev_valid = true;
     invalidate_bounds(c);
 }

@@ -266,6 +266,10 @@ int gdx_col_check_arithmetic(long long n, const double *a, const double *b, doub
 int gdx_col_check_solo_rates(int owners, const double *owner5, const double *slots3, double *rates, double *speeds,
                              int *route);
 
+/* the reverse lists of given neighbour rows (nbr: n x N_K slots, -1 empty): slot j is in the rows of the owners
+ * rev[beg[j]] ... rev[end[j] - 1], in any order; rev holds n x N_K entries */
+int gdx_col_check_reverse(int n, const int *nbr, unsigned int *beg, unsigned int *end, int *rev);
+
 /* ---- host controller and scheduler, callable without a GPU (same code the operator runs) ---- */
 /* _build_col_binmap (inc/swarm/_col_bound.cuh:45-98): returns the merged-bin count */
 int gdx_col_host_binmap(const int *raw_count, int raw_bins, int *raw_to_merged, int *merged);

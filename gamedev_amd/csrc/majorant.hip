@@ -415,7 +415,7 @@ __global__ __launch_bounds__(STATS_BLOCK) void k_feature_fold(const double *part
 // where there is no successor). The steps are grouped by one stable sort; the walks end, since they ascend, after
 // one link on average and ln n or so at most. 262144 samples: 1.7 ms on the host and 1 MB copied -> 65 us.
 constexpr int SHUFFLE_BLOCK = 256;
-// the host shuffles larger sets: the sort takes 28 bytes a sample
+// the host shuffles larger sets: the draws, links and the sort's second copies take 32 bytes a sample
 constexpr long long SHUFFLE_MAX = 1ll << 26;
 
 // first: state before the epoch's first draw, which step n - 1 takes

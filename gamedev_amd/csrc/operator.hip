@@ -1756,55 +1756,6 @@ __device__ __forceinline__ double solo_pair_rate(const owner_terms &t, const sol
     return s.has ? r : 0.0;
 }
 
-// ---- test access to the forms that exist on the device only ----
-__global__ __launch_bounds__(BLOCK) void k_check_arithmetic(const double *a, const double *b, long long n, double *out)
-{
-    __shared__ log_entry logs[LOG_CELLS];
-    copy_log_table(logs, BLOCK);
-    __syncthreads();
-    const long long i = (long long)blockIdx.x*BLOCK + threadIdx.x;
-    if (i >= n) return;
-    const double x = a[i], y = b[i];
-    const double v[8] = {quot(x, y), quot_any(x, y), recip(y), root(x), ulog1p_finite(x, log_source{logs}),
-                         ulog(y, log_source{logs}), ulog1p(x), ulog(y)};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) out[k*n + i] = v[k];
-}
-
-// per owner, a wavefront each: solo_pair_rate beside eval_pair_rate with and without held partner factors; route: 1
-// where the lanes share regimes 4 and 5, 2 where they share regime 6, plus 4 with a sticking packet
-__global__ __launch_bounds__(WAVE) void k_check_solo_rates(const double *owner, const double *slots, int owners,
-                                                          double *rates, double *speeds, int *route)
-{
-    const int o = blockIdx.x, k = threadIdx.x % N_K;
-    const double *me = owner + 5ll*o, *slot = slots + 3ll*((long long)o*N_K + k);
-    gdx_env e{};
-    if constexpr (COAG_KERNEL == 3) e = make_env(me[0], me[1]);
-    const double lambda_0 = me[4];
-    const owner_terms t = make_owner(e, me[2], me[3], slots[3ll*o*N_K + 2]);
-    const partner q{slot[0], slot[1], slot[2], slot[1] >= 0.0};
-    const solo_partner s = make_solo_partner(t, q);
-    double vrel;
-    const double rate = solo_pair_rate(t, s, lambda_0, vrel);
-    const pair_term p = eval_pair_rate(t, q, lambda_0), h = eval_pair_rate<true>(t, q, lambda_0, s.pt);
-    int r = 0;
-    if constexpr (COAG_KERNEL == 3)
-    {
-        const double sl = fmax(t.si, s.pt.sj);
-        if (__ballot(sl < 5.0*t.ris) == 0ull) r = __ballot(sl < 1.0) == ~0ull ? 1 : (__ballot(sl < 1.0) == 0ull ? 2 : 0);
-    }
-    const double ratio = div_rn(q.size_j, t.size_i, t.inv_size), cube = ratio*ratio*ratio;
-    if (__ballot(cube > 0.0 && cube <= 1.0e-06)) r |= 4;
-    if (threadIdx.x == 0) route[o] = r;
-    if (threadIdx.x >= N_K) return;
-    const long long at = (long long)o*N_K + k, all = (long long)owners*N_K;
-    rates[at] = rate;
-    rates[all + at] = p.rate;
-    rates[2*all + at] = h.rate;
-    speeds[at] = vrel;
-    speeds[all + at] = p.vrel;
-}
-
 // event chains (col_chain_run.cu:127-382): a persistent grid over the queued owners. Each K-lane segment
 // of a wavefront runs one owner to its bath end, then takes the wavefront's next owner; the chain sums go
 // to the owner's queue position for the audit pass. The owners are dealt out without atomics: heavy
@@ -2608,23 +2559,6 @@ __global__ __launch_bounds__(BLOCK) void k_chain_audit(gdx_wave w, gdx_chain_log
     flush_audit(a, G.raw_audit);
 }
 
-// the chain sums that the audit reads and the events of a phase's chained owners, in particle order (test access)
-__global__ __launch_bounds__(BLOCK) void k_chain_sums(gdx_wave w, gdx_chain_log clog, double4 *sums, int *events)
-{
-    int gi, s0, s1;
-    if (!due_block(w, BLOCK, gi, s0, s1)) return;
-    const gdx_gref &G = w.table[w.ref[gi]];
-    const int h1 = w.beg[gi] + *G.hcount, l0 = w.beg[gi] + w.cnt[gi] - *G.qcount;
-    const int pos = s0 + int(threadIdx.x);
-    if (pos >= s1 || (pos >= h1 && pos < l0)) return;
-    double4 sum = G.qsum[pos];
-    if (clog.enabled && w.qprefix[w.n] <= clog.owners && pos < h1)
-        add_logged(clog, w.qprefix[gi] - w.beg[gi] + pos, sum);
-    const int p = G.slot_pidx[G.queue[pos]];
-    sums[p] = sum;
-    events[p] = G.qevents[pos];
-}
-
 __global__ __launch_bounds__(256) void k_cached_to_particles(const double4 *cached, const int *slot_pidx, int n_active,
                                                             double *out)
 {
@@ -2656,6 +2590,72 @@ __global__ __launch_bounds__(256) void k_pair_rates(gdx_gref G, int n_active, do
         r = eval_pair_rate(t, load_partner(G.nbr[e], G.res, G.hgs), G.lambda_0).rate;
     }
     out[(long long)G.slot_pidx[s]*N_K + bitrev_slot(pos)] = r;
+}
+
+// the chain sums that the audit reads and the events of a phase's chained owners, in particle order (test access)
+__global__ __launch_bounds__(BLOCK) void k_chain_sums(gdx_wave w, gdx_chain_log clog, double4 *sums, int *events)
+{
+    int gi, s0, s1;
+    if (!due_block(w, BLOCK, gi, s0, s1)) return;
+    const gdx_gref &G = w.table[w.ref[gi]];
+    const int h1 = w.beg[gi] + *G.hcount, l0 = w.beg[gi] + w.cnt[gi] - *G.qcount;
+    const int pos = s0 + int(threadIdx.x);
+    if (pos >= s1 || (pos >= h1 && pos < l0)) return;
+    double4 sum = G.qsum[pos];
+    if (clog.enabled && w.qprefix[w.n] <= clog.owners && pos < h1)
+        add_logged(clog, w.qprefix[gi] - w.beg[gi] + pos, sum);
+    const int p = G.slot_pidx[G.queue[pos]];
+    sums[p] = sum;
+    events[p] = G.qevents[pos];
+}
+
+// ---- test access to the forms that exist on the device only ----
+__global__ __launch_bounds__(BLOCK) void k_check_arithmetic(const double *a, const double *b, long long n, double *out)
+{
+    __shared__ log_entry logs[LOG_CELLS];
+    copy_log_table(logs, BLOCK);
+    __syncthreads();
+    const long long i = (long long)blockIdx.x*BLOCK + threadIdx.x;
+    if (i >= n) return;
+    const double x = a[i], y = b[i];
+    const double v[8] = {quot(x, y), quot_any(x, y), recip(y), root(x), ulog1p_finite(x, log_source{logs}),
+                         ulog(y, log_source{logs}), ulog1p(x), ulog(y)};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) out[k*n + i] = v[k];
+}
+
+// per owner, a wavefront each: solo_pair_rate beside eval_pair_rate with and without held partner factors; route: 1
+// where the lanes share regimes 4 and 5, 2 where they share regime 6, plus 4 with a sticking packet
+__global__ __launch_bounds__(WAVE) void k_check_solo_rates(const double *owner, const double *slots, int owners,
+                                                          double *rates, double *speeds, int *route)
+{
+    const int o = blockIdx.x, k = threadIdx.x % N_K;
+    const double *me = owner + 5ll*o, *slot = slots + 3ll*((long long)o*N_K + k);
+    gdx_env e{};
+    if constexpr (COAG_KERNEL == 3) e = make_env(me[0], me[1]);
+    const double lambda_0 = me[4];
+    const owner_terms t = make_owner(e, me[2], me[3], slots[3ll*o*N_K + 2]);
+    const partner q{slot[0], slot[1], slot[2], slot[1] >= 0.0};
+    const solo_partner s = make_solo_partner(t, q);
+    double vrel;
+    const double rate = solo_pair_rate(t, s, lambda_0, vrel);
+    const pair_term p = eval_pair_rate(t, q, lambda_0), h = eval_pair_rate<true>(t, q, lambda_0, s.pt);
+    int r = 0;
+    if constexpr (COAG_KERNEL == 3)
+    {
+        const double sl = fmax(t.si, s.pt.sj);
+        if (__ballot(sl < 5.0*t.ris) == 0ull) r = __ballot(sl < 1.0) == ~0ull ? 1 : (__ballot(sl < 1.0) == 0ull ? 2 : 0);
+    }
+    const double ratio = div_rn(q.size_j, t.size_i, t.inv_size), cube = ratio*ratio*ratio;
+    if (__ballot(cube > 0.0 && cube <= 1.0e-06)) r |= 4;
+    if (threadIdx.x == 0) route[o] = r;
+    if (threadIdx.x >= N_K) return;
+    const long long at = (long long)o*N_K + k, all = (long long)owners*N_K;
+    rates[at] = rate;
+    rates[all + at] = p.rate;
+    rates[2*all + at] = h.rate;
+    speeds[at] = vrel;
+    speeds[all + at] = p.vrel;
 }
 
 }  // namespace
